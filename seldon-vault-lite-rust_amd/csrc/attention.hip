@@ -166,7 +166,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attn_mfma_kernel(AttnArgs p) {
 
     if (vvalid) {
         const float inv = 1.0f / l_run;
-        float *orow = p.out + (int64_t)(tile.tok0 + qpos) * p.ldo + qhead * HD;
+        float *orow = p.out + (int64_t)(tile.tok0 + qpos) * p.ldo;
+        const int ocol = qhead * HD;
         bool ok = isfinite(inv);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -175,7 +176,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attn_mfma_kernel(AttnArgs p) {
             for (int t = 0; t < NT; ++t) {
                 const float y = o[t][r] * inv;
                 ok = ok && isfinite(y);
-                orow[i * NT + t] = y;
+                if (p.out_scale > 0.f) split_store1(orow, ocol + i * NT + t, y * p.out_scale);
+                else orow[ocol + i * NT + t] = y;
             }
         }
         if (!ok) raise_flag(p.flag, FLAG_NONFINITE);
@@ -593,7 +595,8 @@ __global__ __launch_bounds__(64 * WAVES, (attn_min_blocks<HD, WAVES, NS>())) voi
         // lane l holds, for its query vector, dims 64 c + 16 (l / 16) + 4 r
         // + t in register r of tile 4 c + t
         const float inv = 1.0f / l_run;
-        float *orow = p.out + (int64_t)(tile.tok0 + qpos) * p.ldo + qhead * HD + dpart * HDW + opart * HDO;
+        float *orow = p.out + (int64_t)(tile.tok0 + qpos) * p.ldo;
+        const int ocol = qhead * HD + dpart * HDW + opart * HDO;
         bool ok = isfinite(inv);
 #pragma unroll
         for (int c = 0; c < HDO / 64; ++c)
@@ -603,7 +606,9 @@ __global__ __launch_bounds__(64 * WAVES, (attn_min_blocks<HD, WAVES, NS>())) voi
 #pragma unroll
                 for (int t = 0; t < 4; ++t) d[t] = o[4 * c + t][r] * inv;
                 ok = ok && finite4(d);
-                *(f32x4 *)(orow + 64 * c + 16 * g + 4 * r) = d;
+                const int col = ocol + 64 * c + 16 * g + 4 * r;
+                if (p.out_scale > 0.f) split_store4(orow, col, d * p.out_scale);
+                else *(f32x4 *)(orow + col) = d;
             }
         if (!ok) raise_flag(p.flag, FLAG_NONFINITE);
     }
@@ -650,7 +655,7 @@ __global__ __launch_bounds__(64) void attn_simple_kernel(AttnArgs p) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float *out = p.out + t * p.ldo + (int64_t)h * p.hd;
+    float *out = p.out + t * p.ldo;
     for (int d = lane; d < p.hd; d += 64) {
         float acc = 0.f;
         for (int j = 0; j < width; ++j) {
@@ -659,7 +664,8 @@ __global__ __launch_bounds__(64) void attn_simple_kernel(AttnArgs p) {
             acc += pj * p.v[(tok0 + lo + j) * p.ldv + (int64_t)g * p.hd + d];
         }
         ok = ok && isfinite(acc);
-        out[d] = acc;
+        if (p.out_scale > 0.f) split_store1(out, h * p.hd + d, acc * p.out_scale);
+        else out[h * p.hd + d] = acc;
     }
     if (!ok) raise_flag(p.flag, FLAG_NONFINITE);
 }

@@ -924,7 +924,7 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
         {   // rows [0, H) are the gated values, [H, 2H) the gates
             std::vector<float> first(a.begin(), a.begin() + m->H * m->H),
                 second(a.begin() + m->H * m->H, a.end());
-            const std::vector<float> il = interleave_gate_up(first, second, m->H, m->H_pad, m->H);
+            const std::vector<float> il = interleave_gate_up(first, second, m->H, m->H_pad, m->H, 32);
             ST_TRY(upload_owned(m->allocations, il.data(), il.size(), &ly.w_start));
         }
         ST_TRY(read_bounds(by_name, p + "lconv1d.linear_start", ly.bstart));

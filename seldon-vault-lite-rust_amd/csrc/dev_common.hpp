@@ -10,6 +10,8 @@ namespace svl {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int WAVE = 64;
 
@@ -113,6 +115,61 @@ __device__ __forceinline__ float silu_ref(float v) {
 __device__ __forceinline__ float sigmoid_ref(float v) {
     const float e = expf(-fabsf(v));
     return (v >= 0.0f ? 1.0f : e) / (1.0f + e);
+}
+
+// Split rows: the operand format of the F16 matrix-core GEMMs. A row of K
+// floats (K % 32 == 0) keeps its 4 K bytes; every block of 32 values holds
+// their high halves (64 bytes) and then their low halves: x * scale = hi +
+// lo, hi = half(x * scale), lo = half(x * scale - hi), 22 bits and sign of
+// the scaled value. Within a block, 16-byte chunk c holds values 4c .. 4c + 3
+// and 16 + 4c .. 16 + 4c + 3 (every row permutes its k alike, so products of
+// rows are unchanged): the eight values a GEMM lane's accumulators hold.
+// Scales are powers of two that keep every |x * scale| at most 2^14 or so:
+// halves reach 65504, and the low half's last bit is 2^-24, 2^-38 of that.
+__device__ __forceinline__ void split4(const f32x4 v, f16x4 &hi, f16x4 &lo) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        hi[r] = (_Float16)v[r];
+        lo[r] = (_Float16)(v[r] - (float)hi[r]);
+    }
+}
+
+// Values col .. col + 3 (col % 4 == 0) of a split row, already scaled.
+__device__ __forceinline__ void split_store4(float *row, int col, const f32x4 v) {
+    f16x4 hi, lo;
+    split4(v, hi, lo);
+    char *p = (char *)row + (col >> 5) * 128 + ((col >> 2) & 3) * 16 + ((col >> 4) & 1) * 8;
+    *(f16x4 *)p = hi;
+    *(f16x4 *)(p + 64) = lo;
+}
+
+__device__ __forceinline__ void split_store1(float *row, int col, float v) {
+    const _Float16 hi = (_Float16)v;
+    _Float16 *p = (_Float16 *)((char *)row + (col >> 5) * 128 + ((col >> 2) & 3) * 16 +
+                               ((col >> 4) & 1) * 8) + (col & 3);
+    p[0] = hi;
+    p[32] = (_Float16)(v - (float)hi);
+}
+
+// Chunk c of the 32-value block at column cb: values cb + 4c .. + 3 (x) and
+// cb + 16 + 4c .. + 3 (y).
+__device__ __forceinline__ void split_store8(float *row, int cb, int c, const f32x4 x,
+                                             const f32x4 y) {
+    f16x4 xh, xl, yh, yl;
+    split4(x, xh, xl);
+    split4(y, yh, yl);
+    char *p = (char *)row + (cb >> 5) * 128 + c * 16;
+    *(f16x8 *)p = __builtin_shufflevector(xh, yh, 0, 1, 2, 3, 4, 5, 6, 7);
+    *(f16x8 *)(p + 64) = __builtin_shufflevector(xl, yl, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// The power of two that brings a largest magnitude into [2^13, 2^14), within
+// 2^-100 .. 2^100 (1 for zero and non-finite values).
+__device__ __forceinline__ float split_scale_of(float mx) {
+    if (!(mx > 0.f) || !isfinite(mx)) return 1.f;
+    int e;
+    (void)frexpf(mx, &e);  // mx = f 2^e, f in [0.5, 1)
+    return ldexpf(1.f, max(-100, min(100, 14 - e)));
 }
 
 __device__ __forceinline__ void raise_flag(int *flag, int bit) {

@@ -943,6 +943,7 @@ static hipError_t launch_simple(const GemmArgs &a, hipStream_t s) {
 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
+    if (a.wd) return launch_gemm_split(a, s);
     const bool vec_ok = (a.K % 4 == 0) && (a.lda % 4 == 0) && (a.ldw % 4 == 0) &&
                         ((uintptr_t)a.A % 16 == 0) && ((uintptr_t)a.W % 16 == 0);
     if (!vec_ok) return launch_gemm_simple(a, s);

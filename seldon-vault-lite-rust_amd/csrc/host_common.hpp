@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/svl_hip.h"
+#include "svl_internal.hpp"
 
 struct svl_ctx {
     int device;
@@ -183,19 +184,73 @@ inline svl_status upload_owned(std::vector<float *> &owned, const float *host, s
     return SVL_OK;
 }
 
-// Gate and up projections [I, H] interleaved in 32-row blocks
-// [g 0..31, u 0..31, g 32..63, ...], padded to I_pad rows each, for the
-// GeGLU epilogue of the gate/up GEMM.
+// The power of two that brings a bound on a split operand's magnitude into
+// [2^13, 2^14) (halves reach 65504), within 2^-100 .. 2^100.
+inline float split_scale(double bound) {
+    if (!(bound > 0) || !std::isfinite(bound)) return 1.f;
+    int e;
+    (void)std::frexp(bound, &e);
+    return std::ldexp(1.f, std::max(-100, std::min(100, 14 - e)));
+}
+
+// Largest magnitude of RMSNorm(x) * w over rows of w.size() values: each
+// normalised value is at most sqrt(n) (w empty: unscaled, n = width).
+inline double norm_bound(const std::vector<float> &w) {
+    double mx = 0;
+    for (float v : w) mx = std::max(mx, (double)std::fabs(v));
+    return std::sqrt((double)w.size()) * mx;
+}
+
+// Largest |RMSNorm(x) * w . row| over the rows [rows, K] of a weight
+// (Cauchy-Schwarz: sqrt(K) * |w o row|; w null: a K-vector of norm sqrt(K)),
+// written per row to `each` when given.
+inline double product_bound(const float *rows, int64_t n, int64_t K, const float *w,
+                            std::vector<double> *each = nullptr) {
+    double mx = 0;
+    if (each) each->resize((size_t)n);
+    for (int64_t r = 0; r < n; ++r) {
+        double part[8] = {0};  // independent sums: no serial chain of additions
+        for (int64_t k = 0; k < K; ++k) {
+            const double v = (double)rows[r * K + k] * (w ? (double)w[k] : 1.0);
+            part[k & 7] += v * v;
+        }
+        double s = 0;
+        for (double q : part) s += q;
+        s = std::sqrt(s * (double)K);
+        if (each) (*each)[(size_t)r] = s;
+        mx = std::max(mx, s);
+    }
+    return mx;
+}
+
+// A weight [rows, K] (K % 32 == 0) as split rows with the per-output descale
+// of its GEMM: factor / (row scale * a_scale), a_scale the A operand's scale. The
+// rows are converted in place on the null stream; the caller waits for it
+// before other streams read them.
+inline svl_status upload_split(std::vector<float *> &owned, const float *host, int64_t rows,
+                               int64_t K, float a_scale, float **w, float **wd,
+                               float factor = 1.f) {
+    ST_TRY(upload_owned(owned, host, (size_t)(rows * K), w));
+    float *d = nullptr;
+    HIP_TRY(hipMalloc((void **)&d, (size_t)std::max<int64_t>(rows, 1) * sizeof(float)));
+    owned.push_back(d);
+    HIP_TRY(launch_split_rows(*w, K, rows, (int)K, (int)K, factor / a_scale, *w, d, nullptr));
+    *wd = d;
+    return SVL_OK;
+}
+
+// Gate and up projections [I, H] interleaved in blocks of `block` rows
+// [g 0 .. block - 1, u 0 .. block - 1, g block .., ...], padded to I_pad rows
+// each, for the GeGLU epilogue of the gate/up GEMM (32-row blocks for the
+// FP32 GEMM, 16-row blocks for the split one).
 inline std::vector<float> interleave_gate_up(const std::vector<float> &gate,
                                              const std::vector<float> &up, int64_t I,
-                                             int64_t I_pad, int64_t H) {
+                                             int64_t I_pad, int64_t H, int64_t block) {
     std::vector<float> gu((size_t)(2 * I_pad * H), 0.f);
     for (int64_t j = 0; j < I; ++j) {
-        const int64_t blk = j / 32, off = j % 32;
-        std::copy(gate.begin() + j * H, gate.begin() + (j + 1) * H,
-                  gu.begin() + (64 * blk + off) * H);
-        std::copy(up.begin() + j * H, up.begin() + (j + 1) * H,
-                  gu.begin() + (64 * blk + 32 + off) * H);
+        const int64_t at = 2 * block * (j / block) + j % block;
+        std::copy(gate.begin() + j * H, gate.begin() + (j + 1) * H, gu.begin() + at * H);
+        std::copy(up.begin() + j * H, up.begin() + (j + 1) * H, gu.begin() + (at + block) * H);
     }
     return gu;
 }

@@ -44,6 +44,34 @@ constexpr int ROW_CHUNKS = 8;  // register-resident rows up to 8 * 256 floats
 // load order that holds fewer registers per wave.
 constexpr int64_t LOAD_FIRST_MAX_ROWS = 4096;
 
+// Values 4i .. 4i + 3 of an output row: floats, or split values times
+// `scale` when it is positive (a uniform branch).
+__device__ __forceinline__ void store_row4(float *row, int i, const f32x4 y, float scale) {
+    if (scale > 0.f) split_store4(row, 4 * i, y * scale);
+    else ((f32x4 *)row)[i] = y;
+}
+
+// Split copy of a wave's row (v[c] = values 4 (lane + 64 c) .. + 3), scaled by
+// the power of two of its largest magnitude.
+template <int NC>
+__device__ __forceinline__ void split_hidden(const f32x4 (&v)[NC], int nv, int lane,
+                                             const SplitRows &hs, int64_t row, int width) {
+    float mx = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+        if (lane + 64 * c < nv)
+            mx = fmaxf(fmaxf(fmaxf(mx, fabsf(v[c].x)), fmaxf(fabsf(v[c].y), fabsf(v[c].z))),
+                       fabsf(v[c].w));
+    const float sc = split_scale_of(wave_max(mx));
+    float *srow = hs.rows + row * width;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int i = lane + 64 * c;
+        if (i < nv) split_store4(srow, 4 * i, v[c] * sc);
+    }
+    if (lane == 0) hs.descale[row] = 1.f / sc;
+}
+
 // ---- RMSNorm rows (kernels.rs:727-857) ------------------------------------
 
 // Register-resident variant: width % 4 == 0 and width <= 2048.
@@ -147,7 +175,7 @@ template <int NC, bool LOAD_FIRST>
 __global__ __launch_bounds__(256) void resnorm_kernel(
     const float *__restrict__ x, const float *__restrict__ w1, const float *res, float *h_out,
     const float *__restrict__ w2, float *__restrict__ n_out,
-    float scale, int64_t rows, int width, float eps, int *flag) {
+    float scale, int64_t rows, int width, float eps, int *flag, float n_scale, SplitRows hs) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
@@ -200,10 +228,11 @@ __global__ __launch_bounds__(256) void resnorm_kernel(
             ss2 += hv.x * hv.x + hv.y * hv.y + hv.z * hv.z + hv.w * hv.w;
         }
     }
+    if (hs.rows) split_hidden<NC>(v, nv, lane, hs, row, width);
     if (w2) {
         ss2 = wave_sum(ss2);
         const float inv2 = rms_inverse(ss2, width, eps);
-        f32x4 *nrow = (f32x4 *)(n_out + row * width);
+        float *nrow = n_out + row * width;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             const int i = lane + 64 * c;
@@ -211,7 +240,7 @@ __global__ __launch_bounds__(256) void resnorm_kernel(
                 if constexpr (!LOAD_FIRST) w2v[c] = ((const f32x4 *)w2)[i];
                 const f32x4 y = v[c] * inv2 * w2v[c];
                 ok = ok && finite4(y);
-                nrow[i] = y;
+                store_row4(nrow, i, y, n_scale);
             }
         }
     }
@@ -220,16 +249,17 @@ __global__ __launch_bounds__(256) void resnorm_kernel(
 
 hipError_t launch_resnorm(const float *x, const float *w1, const float *res, float *h_out,
                           const float *w2, float *n_out, float scale, int64_t rows, int width,
-                          float eps, int *flag, hipStream_t s) {
+                          float eps, int *flag, hipStream_t s, float n_scale, SplitRows hs) {
     if (rows <= 0) return hipSuccess;
     if (width <= 0 || width % 4 != 0 || width > 256 * ROW_CHUNKS) return hipErrorInvalidValue;
+    if ((n_scale > 0.f || hs.rows) && width % 32 != 0) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((rows + 3) / 4));
     if (rows < LOAD_FIRST_MAX_ROWS) {
         SVL_DISPATCH_NC_B((width + 255) / 256, resnorm_kernel, true, grid, s, x, w1, res, h_out,
-                          w2, n_out, scale, rows, width, eps, flag);
+                          w2, n_out, scale, rows, width, eps, flag, n_scale, hs);
     } else {
         SVL_DISPATCH_NC_B((width + 255) / 256, resnorm_kernel, false, grid, s, x, w1, res, h_out,
-                          w2, n_out, scale, rows, width, eps, flag);
+                          w2, n_out, scale, rows, width, eps, flag, n_scale, hs);
     }
     return hipGetLastError();
 }
@@ -240,7 +270,7 @@ __global__ __launch_bounds__(256) void gather_kernel(
     const uint32_t *__restrict__ ids, const float *__restrict__ table, int64_t vocab,
     const int32_t *__restrict__ featmap, const float *__restrict__ feats, float scale,
     const float *__restrict__ w_in, float *__restrict__ h, float *__restrict__ n, int64_t tokens,
-    int width, float eps, int *flag) {
+    int width, float eps, int *flag, float n_scale, SplitRows hs) {
     const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (t >= tokens) return;
@@ -283,16 +313,17 @@ __global__ __launch_bounds__(256) void gather_kernel(
             ss += e.x * e.x + e.y * e.y + e.z * e.z + e.w * e.w;
         }
     }
+    if (hs.rows) split_hidden<NC>(v, nv, lane, hs, t, width);
     ss = wave_sum(ss);
     const float inv = rms_inverse(ss, width, eps);
-    f32x4 *nrow = (f32x4 *)(n + t * width);
+    float *nrow = n + t * width;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int i = lane + 64 * c;
         if (i < nv) {
             const f32x4 y = v[c] * inv * wv[c];
             ok = ok && finite4(y);
-            nrow[i] = y;
+            store_row4(nrow, i, y, n_scale);
         }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
@@ -301,11 +332,13 @@ __global__ __launch_bounds__(256) void gather_kernel(
 hipError_t launch_gather(const uint32_t *ids, const float *table, int64_t vocab,
                          const int32_t *featmap, const float *feats, float scale,
                          const float *w_in, float *h, float *n, int64_t tokens, int width,
-                         float eps, int *flag, hipStream_t s) {
+                         float eps, int *flag, hipStream_t s, float n_scale, SplitRows hs) {
     if (tokens <= 0) return hipSuccess;
     if (width <= 0 || width % 4 != 0 || width > 256 * ROW_CHUNKS) return hipErrorInvalidValue;
+    if ((n_scale > 0.f || hs.rows) && width % 32 != 0) return hipErrorInvalidValue;
     SVL_DISPATCH_NC((width + 255) / 256, gather_kernel, dim3((unsigned)((tokens + 3) / 4)), s, ids,
-                    table, vocab, featmap, feats, scale, w_in, h, n, tokens, width, eps, flag);
+                    table, vocab, featmap, feats, scale, w_in, h, n, tokens, width, eps, flag,
+                    n_scale, hs);
     return hipGetLastError();
 }
 

@@ -72,6 +72,12 @@ struct DevLayer {
           *ln_post_ple = nullptr, *q_norm = nullptr, *k_norm = nullptr;
     float scalar = 1.f;
     int hd = 0, nkv = 0, full = 0;
+    // split models: descale of each projection's outputs, and the scales of
+    // its split operands (norm outputs, attention output, GeGLU and PLE
+    // activations)
+    float *d_qkv = nullptr, *d_o = nullptr, *d_gu = nullptr, *d_down = nullptr, *d_pg = nullptr,
+          *d_pp = nullptr;
+    float s_in = 0.f, s_ff = 0.f, s_attn = 0.f, s_act = 1.f, s_pg = 1.f;
 };
 
 struct TimedLaunch {
@@ -95,6 +101,11 @@ struct svl_text_model {
     float eps = 0.f, full_theta = 0.f, slide_theta = 0.f;
     float embedding_scale = 1.f, ple_scale = 1.f;
     int64_t I_pad = 0;
+    // Every projection runs on split operands (gemm_split.hip): the widths are
+    // multiples of 32. Other models take the FP32 GEMMs.
+    bool split = false;
+    float *d_out_proj = nullptr, *d_ple_model = nullptr;
+    float s_final = 0.f;
     std::vector<DevLayer> layers;
     std::vector<float *> allocations;
     float *embed = nullptr, *out_proj = nullptr, *final_norm = nullptr, *ple_model = nullptr,
@@ -114,7 +125,10 @@ struct svl_text_model {
     std::mutex mu;
 
     // workspace
-    DevBuf<float> h, n, tmp, qkv, attn, act, ple, pg, proj, feats, pooled, normalized, trunc;
+    // (split models: attn also holds the split copy of the hidden rows for the
+    // PLE projections, whose lifetime ends before the next attention output;
+    // rs their scales)
+    DevBuf<float> h, n, tmp, qkv, attn, act, ple, pg, proj, feats, pooled, normalized, trunc, rs;
     DevBuf<int32_t> pos, rowlen, featmap;
     DevBuf<uint32_t> ids;
     // A pass's metadata in one device block, filled by one copy from pinned
@@ -147,7 +161,7 @@ struct svl_text_model {
         }
         h.release(); n.release(); tmp.release(); qkv.release(); attn.release(); act.release();
         ple.release(); pg.release(); proj.release(); feats.release(); pooled.release();
-        normalized.release(); trunc.release(); pos.release(); rowlen.release();
+        normalized.release(); trunc.release(); rs.release(); pos.release(); rowlen.release();
         featmap.release(); ids.release(); meta.release();
         if (ev_meta) {
             (void)hipEventSynchronize(ev_meta);
@@ -470,6 +484,7 @@ svl_status ensure_workspace(svl_text_model *m, const Batch &b, int64_t feat_floa
     HIP_TRY(m->tmp.ensure(T * m->H));
     HIP_TRY(m->qkv.ensure(T * m->max_qkv));
     HIP_TRY(m->attn.ensure(T * m->max_q));
+    if (m->split) HIP_TRY(m->rs.ensure(T));
     HIP_TRY(m->act.ensure(T * m->I));
     HIP_TRY(m->ple.ensure(T * m->L * m->P));
     HIP_TRY(m->pg.ensure(T * m->P));
@@ -507,6 +522,9 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     int32_t *pos = m->pos.p + t0, *rowlen = m->rowlen.p + t0;
     const int64_t *offs = m->offsets.p + grp.off_slot;
     const int64_t T_all = b.hidden_stride > 0 ? b.hidden_stride : b.T;
+    // split models: the split copy of h that the PLE projections read
+    const SplitRows hs = m->split ? SplitRows{attn, m->rs.p + t0} : SplitRows();
+    const float *h_in = m->split ? attn : h, *h_rs = hs.descale;
     // CUs each launch can expect while the batch's groups run side by side
     const int cus = b.groups.size() > 1 ? (int)(256 / b.groups.size()) : 0;
 
@@ -515,7 +533,8 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         Timer tm(m, s, KC_GATHER, Td * H * 4 * 3);
         HIP_TRY(launch_gather(d_ids + t0, m->embed, m->V, d_featmap ? d_featmap + t0 : nullptr,
                               d_feats, m->embedding_scale,
-                              m->layers[0].ln_in, h, n, T, (int)H, m->eps, flag, s));
+                              m->layers[0].ln_in, h, n, T, (int)H, m->eps, flag, s,
+                              m->layers[0].s_in, hs));
     }
     if (h_hidden)
         HIP_TRY(hipMemcpyAsync(h_hidden + t0 * H, h, (size_t)(T * H) * 4, hipMemcpyDeviceToHost,
@@ -523,9 +542,12 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
 
     // Projection-only per-layer embeddings (text.rs:285-306).
     {
-        GemmArgs g{h, H, m->ple_model, H, ple, L * P, (int)T, (int)(L * P), (int)H, EPI_SCALE,
-                   m->ple_scale, nullptr, 0, 0};
+        // (the split descale carries ple_scale)
+        GemmArgs g{h_in, H, m->ple_model, H, ple, L * P, (int)T, (int)(L * P), (int)H,
+                   m->split ? EPI_STORE : EPI_SCALE, m->ple_scale, nullptr, 0, 0};
         g.cus = cus;
+        g.wd = m->d_ple_model;
+        g.rs = h_rs;
         Timer tm(m, s, KC_GEMM_PLE_MODEL, 2.0 * Td * H * L * P);
         HIP_TRY(launch_gemm(g, s));
     }
@@ -540,6 +562,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{n, H, ly.w_qkv, H, qkv, ldqkv, (int)T, (int)ldqkv, (int)H, EPI_STORE, 1.f,
                        nullptr, 0, 0};
+            g.wd = ly.d_qkv;
             g.cus = cus;
             Timer tm(m, s, KC_GEMM_QKV, 2.0 * Td * H * ldqkv);
             HIP_TRY(launch_gemm(g, s));
@@ -571,12 +594,14 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             a.flag = flag;
             a.max_len = std::min<int64_t>(T, MAX_TEXT_TOKENS);  // validate_row caps every row
             a.shortest = grp.shortest;
+            a.out_scale = ly.s_attn;
             Timer tm(m, s, KC_ATTENTION, grp.attn_flops[ly.full]);
             HIP_TRY(launch_attention(a, s));
         }
         {
             GemmArgs g{attn, qd, ly.w_o, qd, tmp, H, (int)T, (int)H, (int)qd, EPI_STORE, 1.f,
                        nullptr, 0, 0};
+            g.wd = ly.d_o;
             g.cus = cus;
             Timer tm(m, s, KC_GEMM_O, 2.0 * Td * qd * H);
             HIP_TRY(launch_gemm(g, s));
@@ -584,11 +609,13 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             Timer tm(m, s, KC_RESNORM, Td * H * 4 * 4);
             HIP_TRY(launch_resnorm(tmp, ly.ln_post_attn, h, h, ly.ln_pre_ff, n, 1.0f, T, (int)H,
-                                   m->eps, flag, s));
+                                   m->eps, flag, s, ly.s_ff));
         }
         {
             GemmArgs g{n, H, ly.w_gu, H, act, m->I, (int)T, (int)(2 * m->I_pad), (int)H, EPI_GEGLU,
                        1.f, nullptr, 0, (int)m->I};
+            g.wd = ly.d_gu;
+            g.out_scale = ly.s_act;
             g.cus = cus;
             Timer tm(m, s, KC_GEMM_GATE_UP, 2.0 * Td * H * 2 * m->I);
             HIP_TRY(launch_gemm(g, s));
@@ -596,6 +623,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{act, m->I, ly.w_down, m->I, tmp, H, (int)T, (int)H, (int)m->I, EPI_STORE,
                        1.f, nullptr, 0, 0};
+            g.wd = ly.d_down;
             g.cus = cus;
             Timer tm(m, s, KC_GEMM_DOWN, 2.0 * Td * m->I * H);
             HIP_TRY(launch_gemm(g, s));
@@ -603,11 +631,14 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             Timer tm(m, s, KC_RESNORM, Td * H * 4 * 3);
             HIP_TRY(launch_resnorm(tmp, ly.ln_post_ff, h, h, nullptr, nullptr, 1.0f, T, (int)H,
-                                   m->eps, flag, s));
+                                   m->eps, flag, s, 0.f, hs));
         }
         {
-            GemmArgs g{h, H, ly.w_pg, H, pg, P, (int)T, (int)P, (int)H, EPI_GELU_MUL, 1.f,
+            GemmArgs g{h_in, H, ly.w_pg, H, pg, P, (int)T, (int)P, (int)H, EPI_GELU_MUL, 1.f,
                        ple + l * P, L * P, 0};
+            g.wd = ly.d_pg;
+            g.rs = h_rs;
+            g.out_scale = ly.s_pg;
             g.cus = cus;
             Timer tm(m, s, KC_GEMM_PLE_GATE, 2.0 * Td * H * P);
             HIP_TRY(launch_gemm(g, s));
@@ -615,15 +646,18 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{pg, P, ly.w_pp, P, tmp, H, (int)T, (int)H, (int)P, EPI_STORE, 1.f, nullptr,
                        0, 0};
+            g.wd = ly.d_pp;
+            g.rs = h_rs;
             g.cus = cus;
             Timer tm(m, s, KC_GEMM_PLE_PROJ, 2.0 * Td * P * H);
             HIP_TRY(launch_gemm(g, s));
         }
         {
             const float *next = l + 1 < L ? m->layers[(size_t)l + 1].ln_in : m->final_norm;
+            const float s_next = l + 1 < L ? m->layers[(size_t)l + 1].s_in : m->s_final;
             Timer tm(m, s, KC_RESNORM, Td * H * 4 * 4);
             HIP_TRY(launch_resnorm(tmp, ly.ln_post_ple, h, h, next, n, ly.scalar, T, (int)H,
-                                   m->eps, flag, s));
+                                   m->eps, flag, s, s_next));
         }
         if (h_hidden)
             HIP_TRY(hipMemcpyAsync(h_hidden + (size_t)((l + 1) * T_all * H + t0 * H), h,
@@ -634,6 +668,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     {
         GemmArgs g{n, H, m->out_proj, H, proj, E, (int)T, (int)E, (int)H, EPI_STORE, 1.f, nullptr,
                    0, 0};
+        g.wd = m->d_out_proj;
         g.cus = cus;
         Timer tm(m, s, KC_GEMM_OUT, 2.0 * Td * H * E);
         HIP_TRY(launch_gemm(g, s));
@@ -973,17 +1008,31 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
     auto get = [&](const std::string &name, std::vector<float> &buf) -> svl_status {
         return decode_named(by_name, name, buf);
     };
-    std::vector<float> a, b2, c2;
+    m->split = m->H % 32 == 0 && m->I % 32 == 0 && m->P % 32 == 0;
+    for (int64_t l = 0; l < m->L; ++l)
+        m->split = m->split && (m->NH * cfg->head_dim[l]) % 32 == 0;
+    // A projection weight [rows, K], for an A operand scaled by a_scale.
+    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, float **dst,
+                   float **descale, float factor = 1.f) -> svl_status {
+        if (!m->split) return upload(m, w.data(), w.size(), dst);
+        return upload_split(m->allocations, w.data(), (int64_t)w.size() / K, K, a_scale, dst,
+                            descale, factor);
+    };
+    std::vector<float> a, b2, c2, nw;
     ST_TRY(get("language_model.embed_tokens.weight", a));
     ST_TRY(upload(m, a.data(), a.size(), &m->embed));
-    ST_TRY(get("language_model.embedding_projection.weight", a));
-    ST_TRY(upload(m, a.data(), a.size(), &m->out_proj));
     ST_TRY(get("language_model.norm.weight", a));
     ST_TRY(upload(m, a.data(), a.size(), &m->final_norm));
+    if (m->split) m->s_final = split_scale(norm_bound(a));
+    ST_TRY(get("language_model.embedding_projection.weight", a));
+    ST_TRY(put(a, m->H, m->s_final, &m->out_proj, &m->d_out_proj));
+    // the hidden rows carry scales of their own (SplitRows); the descale also
+    // applies the projection's 1 / sqrt(H)
     ST_TRY(get("language_model.ple.per_layer_model_projection.weight", a));
-    ST_TRY(upload(m, a.data(), a.size(), &m->ple_model));
+    ST_TRY(put(a, m->H, 1.f, &m->ple_model, &m->d_ple_model, m->ple_scale));
     ST_TRY(get("language_model.ple.per_layer_projection_norm.weight", a));
     ST_TRY(upload(m, a.data(), a.size(), &m->ple_norm));
+    const double ple_bound = norm_bound(a);
 
     m->layers.resize((size_t)m->L);
     for (int64_t l = 0; l < m->L; ++l) {
@@ -996,25 +1045,46 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
         const int64_t H = m->H, qd = m->NH * ly.hd, kd = (int64_t)ly.nkv * ly.hd;
         // fused QKV weight: rows [q; k; v]
         std::vector<float> qkv((size_t)((qd + 2 * kd) * H));
+        ST_TRY(get(p + "input_layernorm.weight", nw));
+        if (m->split) ly.s_in = split_scale(norm_bound(nw));
         ST_TRY(get(p + "self_attn.q_proj.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin());
         ST_TRY(get(p + "self_attn.k_proj.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + qd * H);
         ST_TRY(get(p + "self_attn.v_proj.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + (qd + kd) * H);
-        ST_TRY(upload(m, qkv.data(), qkv.size(), &ly.w_qkv));
+        ST_TRY(put(qkv, H, ly.s_in, &ly.w_qkv, &ly.d_qkv));
+        // attention outputs are convex sums of RMS-normalised value rows
+        if (m->split) ly.s_attn = split_scale(std::sqrt((double)ly.hd));
         ST_TRY(get(p + "self_attn.o_proj.weight", a));
-        ST_TRY(upload(m, a.data(), a.size(), &ly.w_o));
+        ST_TRY(put(a, qd, ly.s_attn, &ly.w_o, &ly.d_o));
         ST_TRY(get(p + "mlp.gate_proj.weight", b2));
         ST_TRY(get(p + "mlp.up_proj.weight", c2));
-        const std::vector<float> gu = interleave_gate_up(b2, c2, m->I, m->I_pad, m->H);
-        ST_TRY(upload(m, gu.data(), gu.size(), &ly.w_gu));
+        if (m->split) {
+            ST_TRY(get(p + "pre_feedforward_layernorm.weight", nw));
+            ly.s_ff = split_scale(norm_bound(nw));
+            // |gelu(g) u| <= |g| |u|
+            std::vector<double> bg, bu;
+            product_bound(b2.data(), m->I, H, nw.data(), &bg);
+            product_bound(c2.data(), m->I, H, nw.data(), &bu);
+            double act = 0;
+            for (size_t j = 0; j < bg.size(); ++j) act = std::max(act, bg[j] * bu[j]);
+            ly.s_act = split_scale(act);
+        }
+        const std::vector<float> gu =
+            interleave_gate_up(b2, c2, m->I, m->I_pad, m->H, m->split ? 16 : 32);
+        ST_TRY(put(gu, H, ly.s_ff, &ly.w_gu, &ly.d_gu));
         ST_TRY(get(p + "mlp.down_proj.weight", a));
-        ST_TRY(upload(m, a.data(), a.size(), &ly.w_down));
+        ST_TRY(put(a, m->I, ly.s_act, &ly.w_down, &ly.d_down));
         ST_TRY(get(p + "ple_block.per_layer_input_gate.weight", a));
-        ST_TRY(upload(m, a.data(), a.size(), &ly.w_pg));
+        ST_TRY(put(a, H, 1.f, &ly.w_pg, &ly.d_pg));
+        // A hidden row whose scale is 1 / rs has values below 2^14 rs, so its
+        // gates are at most 2^14 rs sqrt(H) |W row|; s_pg / rs brings gate x
+        // per-layer input below 2^14.
+        if (m->split)
+            ly.s_pg = split_scale(16384.0 * product_bound(a.data(), m->P, H, nullptr) * ple_bound);
         ST_TRY(get(p + "ple_block.per_layer_projection.weight", a));
-        ST_TRY(upload(m, a.data(), a.size(), &ly.w_pp));
+        ST_TRY(put(a, m->P, ly.s_pg, &ly.w_pp, &ly.d_pp));
         struct {
             const char *name;
             float **dst;
@@ -1048,6 +1118,10 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
     for (const DevLayer &ly : m->layers) {
         m->max_qkv = std::max<int64_t>(m->max_qkv, m->NH * ly.hd + 2 * (int64_t)ly.nkv * ly.hd);
         m->max_q = std::max<int64_t>(m->max_q, m->NH * ly.hd);
+    }
+    if (m->split) {
+        m->max_q = std::max(m->max_q, m->H);
+        HIP_TRY(hipStreamSynchronize(nullptr));  // the weights' conversion
     }
     HIP_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming));

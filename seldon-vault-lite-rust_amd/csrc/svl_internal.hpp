@@ -66,6 +66,10 @@ struct GemmArgs {
     const uint8_t *conv_mask = nullptr;
     int conv_c0 = 0, conv_f0 = 0, conv_f1 = 0;
     int64_t conv_a_floats = 0;  // floats of the layer-0 output (A's window)
+    // split operands (launch_gemm_split)
+    const float *wd = nullptr;  // [N] descale of each output column
+    const float *rs = nullptr;  // [M] descale of each A row (null: 1)
+    float out_scale = 1.f;      // scale of a split output
 };
 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t s);
@@ -77,21 +81,46 @@ hipError_t launch_gemm_conv(const GemmArgs &a, hipStream_t s);
 // (K % 4 != 0); same epilogues.
 hipError_t launch_gemm_simple(const GemmArgs &a, hipStream_t s);
 
+// The same products on the F16 matrix cores (gemm_split.hip), taken when
+// a.wd is set: A and W hold split rows (dev_common.hpp: 4 bytes per element,
+// K % 32 == 0), and every epilogue value is first descaled by wd[n] (and
+// rs[m] where rows carry scales of their own): C = epilogue((A . W^T) *
+// rs[m] * wd[n]). Paired epilogues take W rows interleaved in 16-row blocks.
+// The epilogues whose output only another GEMM reads (GEGLU, GELU_MUL,
+// CLIP_SILU) store split rows scaled by out_scale (out_scale / rs[m] with row
+// scales; ldc % 32 == 0, the output width a multiple of 32).
+hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s);
+constexpr int SPLIT_RASTER_M = 8;  // M blocks per rasterization group
+// x [rows, K] (leading dimension ldx) to split rows of K_pad >= K, each
+// scaled by its own power of two; descale[row] = also / scale.
+hipError_t launch_split_rows(const float *x, int64_t ldx, int64_t rows, int K, int K_pad,
+                             float also, float *out, float *descale, hipStream_t s);
+
 // out = rms_norm_rows(x, w) (w == nullptr: unscaled).
 hipError_t launch_rms_rows(const float *x, const float *w, float *out, int64_t rows, int width,
                            float eps, int *flag, hipStream_t s);
 
-// h_out = (res + rms(x, w1)) * scale ; if w2: n_out = rms(h_out, w2).
+// A row kernel's split copy of its hidden rows: each row scaled by its own
+// power of two (rows == nullptr: none).
+struct SplitRows {
+    float *rows = nullptr;     // [rows, width] split rows
+    float *descale = nullptr;  // [rows]
+};
+
+// h_out = (res + rms(x, w1)) * scale ; if w2: n_out = rms(h_out, w2), stored
+// as split rows times n_scale when n_scale > 0. `hs`: split copy of h_out.
 hipError_t launch_resnorm(const float *x, const float *w1, const float *res, float *h_out,
                           const float *w2, float *n_out, float scale, int64_t rows, int width,
-                          float eps, int *flag, hipStream_t s);
+                          float eps, int *flag, hipStream_t s, float n_scale = 0.f,
+                          SplitRows hs = SplitRows());
 
 // h[t] = table[ids[t]] * scale, or feats[featmap[t]] when featmap[t] >= 0;
-// n[t] = rms(h[t], w_in).
+// n[t] = rms(h[t], w_in); n_scale and hs as in launch_resnorm.
 hipError_t launch_gather(const uint32_t *ids, const float *table, int64_t vocab,
                          const int32_t *featmap, const float *feats, float scale,
                          const float *w_in, float *h, float *n, int64_t tokens, int width,
-                         float eps, int *flag, hipStream_t s);
+                         float eps, int *flag, hipStream_t s, float n_scale = 0.f,
+                         SplitRows hs = SplitRows());
 
 // In place on qkv[T, ld]: per-head q RMSNorm(q_norm) + RoPE, k RMSNorm(k_norm)
 // + RoPE, v unscaled RMSNorm. cos/sin tables are [positions, hd/2].
@@ -130,6 +159,7 @@ struct AttnArgs {
     int *flag;
     int64_t max_len = 0;    // bound on the row length (0: unknown, bounded by tokens)
     int64_t shortest = 0;   // shortest row of the launch (0: unknown)
+    float out_scale = 0.f;  // > 0: out holds split rows scaled by it (ldo % 32 == 0)
 };
 // Query vectors per work item of the MFMA kernel (0 if hd has no MFMA kernel).
 int attn_block_vectors(int hd);

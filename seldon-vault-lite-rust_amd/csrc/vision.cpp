@@ -768,7 +768,7 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         ST_TRY(up(p + "self_attn.o_proj.linear.weight", &ly.w_o));
         ST_TRY(decode_named(by_name, p + "mlp.gate_proj.linear.weight", b2));
         ST_TRY(decode_named(by_name, p + "mlp.up_proj.linear.weight", c2));
-        const std::vector<float> gu = interleave_gate_up(b2, c2, v->I, v->I_pad, v->H);
+        const std::vector<float> gu = interleave_gate_up(b2, c2, v->I, v->I_pad, v->H, 32);
         ST_TRY(upload_owned(v->allocations, gu.data(), gu.size(), &ly.w_gu));
         ST_TRY(up(p + "mlp.down_proj.linear.weight", &ly.w_down));
         ST_TRY(up(p + "input_layernorm.weight", &ly.ln_in));
