@@ -1,14 +1,18 @@
 // FP32-accurate GEMM on the F16 matrix cores: C = epilogue(A[M,K] . W[N,K]^T)
 // with both operands held as pairs of halves (split rows, dev_common.hpp).
 //
-// Every product of two operands x = xh + xl, y = yh + yl is taken as
-// xl.yh + xh.yl + xh.yh: three F16 MFMAs into one FP32 accumulator. xh and
+// Every product of two operands x = xh + xl, y = yh + yl is taken as xh.yh in
+// one FP32 accumulator and xl.yh + xh.yl in a second: three F16 MFMAs. xh and
 // yh carry the leading 11 bits of the scaled values and xl, yl the next 11,
 // so the dropped xl.yl is below 2^-22 of the product, and an MFMA of 32 k
 // rounds its accumulator 4 times (once per 8 products, probed) where the FP32
-// MFMA chain rounds 32 times. Against 64-bit sums of normal inputs the three
-// products are off by 1.0e-7 / 3.0e-7 / 7.1e-7 (K = 64 / 768 / 4096, relative
-// 2-norm), the FP32 MFMA chain by 1.4e-7 / 5.0e-7 / 1.14e-6.
+// MFMA chain rounds 32 times. Against 64-bit sums of normal inputs the result
+// is off by 0.95e-7 / 1.9e-7 / 4.2e-7 (K = 64 / 768 / 4096, relative 2-norm)
+// with a mean of -3e-9, the FP32 MFMA chain by 1.4e-7 / 5.0e-7 / 1.14e-6 with
+// 3e-9. The mixed products have an accumulator of their own because the MFMA
+// drops the bits of small addends downwards: in one accumulator the sums were
+// off by 3.0e-7 with a mean of -1.6e-8, which averaging rows does not remove
+// (2304-key attention: the image embeddings were twice as far from 64 bits).
 //
 // What bounds it: the F16 matrix pipes deliver 1230 TFLOP/s to a register-only
 // loop of 16x16x32 MFMAs, i.e. 410 TFLOP/s of FP32 products, against 145 for
@@ -263,11 +267,12 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
         }
     }
 
-    f32x4 acc[TM][TN];
+    // high products, and the two mixed ones
+    f32x4 acc[TM][TN], acl[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TN; ++j) acc[i][j] = acl[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // 16-row blocks start at multiples of 16, so a row's swizzle depends on
     // the lane's row only
@@ -314,9 +319,11 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            t == 1 ? bl[j] : bh[j], t == 0 ? al[i] : ah[i], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < TN; ++j) {
+                        f32x4 &to = t == 1 ? acc[i][j] : acl[i][j];
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            t == 2 ? bl[j] : bh[j], t == 0 ? al[i] : ah[i], to, 0, 0, 0);
+                    }
                 if (refill) {
 #pragma unroll
                     for (int q = 0; q < NDMA; ++q)
@@ -342,7 +349,7 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
     // column limit of C; vector stores need aligned rows
     const int limit = split_paired<EPI>() ? p.n_out : N;
     const bool vec = (p.ldc & 3) == 0 && ((uintptr_t)p.C & 15) == 0;
-    auto value = [&](int i, int j) { return acc[i][j] * rs[i] * wd[j]; };
+    auto value = [&](int i, int j) { return (acc[i][j] + acl[i][j]) * rs[i] * wd[j]; };
     constexpr int NBLK = NARROW ? 1 : WTN / 32;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -498,6 +505,14 @@ hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s) {
         case EPI_CLIP_GLU: return launch_split_auto<EPI_CLIP_GLU>(a, s);
     }
     return hipErrorInvalidValue;
+}
+
+// The implicit-im2col convolution (gemm_conv_ok holds): 32-k slices that each
+// lie within one tap; the waves stacked along M for at most 32 channels.
+hipError_t launch_gemm_conv_split(const GemmArgs &a, hipStream_t s) {
+    if (a.K % 32 || (uintptr_t)a.wd % 16) return hipErrorInvalidValue;
+    if (a.N <= 32) return launch_split_tile<128, 32, 1, EPI_STORE, 4, 2, 4, 1, true>(a, s);
+    return launch_split_tile<64, 64, 1, EPI_STORE, 4, 2, 2, 2, true>(a, s);
 }
 
 // ---- split rows -----------------------------------------------------------------

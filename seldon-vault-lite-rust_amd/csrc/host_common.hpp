@@ -209,13 +209,24 @@ inline double product_bound(const float *rows, int64_t n, int64_t K, const float
     double mx = 0;
     if (each) each->resize((size_t)n);
     for (int64_t r = 0; r < n; ++r) {
-        double part[8] = {0};  // independent sums: no serial chain of additions
-        for (int64_t k = 0; k < K; ++k) {
-            const double v = (double)rows[r * K + k] * (w ? (double)w[k] : 1.0);
-            part[k & 7] += v * v;
-        }
+        const float *row = rows + r * K;
+        // independent float sums (vector code); the margin covers their rounding
+        float part[16] = {0};
+        int64_t k = 0;
+        for (; k + 16 <= K; k += 16)
+            for (int j = 0; j < 16; ++j) {
+                const float v = w ? row[k + j] * w[k + j] : row[k + j];
+                part[j] += v * v;
+            }
         double s = 0;
-        for (double q : part) s += q;
+        for (float q : part) s += q;
+        s *= 1.001;
+        for (; k < K; ++k) s += std::pow((double)row[k] * (w ? (double)w[k] : 1.0), 2);
+        // squares outside the float range
+        if (!std::isfinite(s) || s < 1e-30) {
+            s = 0;
+            for (k = 0; k < K; ++k) s += std::pow((double)row[k] * (w ? (double)w[k] : 1.0), 2);
+        }
         s = std::sqrt(s * (double)K);
         if (each) (*each)[(size_t)r] = s;
         mx = std::max(mx, s);
@@ -223,20 +234,44 @@ inline double product_bound(const float *rows, int64_t n, int64_t K, const float
     return mx;
 }
 
+// Largest |gelu(g) u| of the gate and up projections [I, K] of RMSNorm(x) * w:
+// at most |g| |u|.
+inline double geglu_bound(const std::vector<float> &gate, const std::vector<float> &up, int64_t I,
+                          int64_t K, const std::vector<float> &w) {
+    std::vector<double> bg, bu;
+    (void)product_bound(gate.data(), I, K, w.data(), &bg);
+    (void)product_bound(up.data(), I, K, w.data(), &bu);
+    double mx = 0;
+    for (size_t j = 0; j < bg.size(); ++j) mx = std::max(mx, bg[j] * bu[j]);
+    return mx;
+}
+
 // A weight [rows, K] (K % 32 == 0) as split rows with the per-output descale
 // of its GEMM: factor / (row scale * a_scale), a_scale the A operand's scale. The
 // rows are converted in place on the null stream; the caller waits for it
 // before other streams read them.
+// Parts [rows, K] of one weight may read A operands of their own scales.
+inline svl_status upload_split_parts(std::vector<float *> &owned, const float *host, int parts,
+                                     int64_t rows, int64_t K, const float *a_scale, float **w,
+                                     float **wd, float factor = 1.f) {
+    const size_t count = (size_t)(parts * rows * K);
+    float *d = nullptr;
+    HIP_TRY(hipMalloc((void **)&d, (count + (size_t)std::max<int64_t>(parts * rows, 1)) * sizeof(float)));
+    owned.push_back(d);
+    HIP_TRY(hipMemcpy(d, host, count * sizeof(float), hipMemcpyHostToDevice));
+    *w = d;
+    d += count;  // the descales follow the weight (K % 32 == 0 keeps them aligned)
+    for (int j = 0; j < parts; ++j)
+        HIP_TRY(launch_split_rows(*w + j * rows * K, K, rows, (int)K, (int)K, factor / a_scale[j],
+                                  *w + j * rows * K, d + j * rows, nullptr));
+    *wd = d;
+    return SVL_OK;
+}
+
 inline svl_status upload_split(std::vector<float *> &owned, const float *host, int64_t rows,
                                int64_t K, float a_scale, float **w, float **wd,
                                float factor = 1.f) {
-    ST_TRY(upload_owned(owned, host, (size_t)(rows * K), w));
-    float *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, (size_t)std::max<int64_t>(rows, 1) * sizeof(float)));
-    owned.push_back(d);
-    HIP_TRY(launch_split_rows(*w, K, rows, (int)K, (int)K, factor / a_scale, *w, d, nullptr));
-    *wd = d;
-    return SVL_OK;
+    return upload_split_parts(owned, host, 1, rows, K, &a_scale, w, wd, factor);
 }
 
 // Gate and up projections [I, H] interleaved in blocks of `block` rows

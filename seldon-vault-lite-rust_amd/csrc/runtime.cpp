@@ -525,8 +525,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     // split models: the split copy of h that the PLE projections read
     const SplitRows hs = m->split ? SplitRows{attn, m->rs.p + t0} : SplitRows();
     const float *h_in = m->split ? attn : h, *h_rs = hs.descale;
-    // CUs each launch can expect while the batch's groups run side by side
-    const int cus = b.groups.size() > 1 ? (int)(256 / b.groups.size()) : 0;
 
     HIP_TRY(launch_positions(offs, grp.nrows, pos, rowlen, s));
     {
@@ -545,7 +543,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         // (the split descale carries ple_scale)
         GemmArgs g{h_in, H, m->ple_model, H, ple, L * P, (int)T, (int)(L * P), (int)H,
                    m->split ? EPI_STORE : EPI_SCALE, m->ple_scale, nullptr, 0, 0};
-        g.cus = cus;
         g.wd = m->d_ple_model;
         g.rs = h_rs;
         Timer tm(m, s, KC_GEMM_PLE_MODEL, 2.0 * Td * H * L * P);
@@ -563,7 +560,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             GemmArgs g{n, H, ly.w_qkv, H, qkv, ldqkv, (int)T, (int)ldqkv, (int)H, EPI_STORE, 1.f,
                        nullptr, 0, 0};
             g.wd = ly.d_qkv;
-            g.cus = cus;
             Timer tm(m, s, KC_GEMM_QKV, 2.0 * Td * H * ldqkv);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -602,7 +598,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             GemmArgs g{attn, qd, ly.w_o, qd, tmp, H, (int)T, (int)H, (int)qd, EPI_STORE, 1.f,
                        nullptr, 0, 0};
             g.wd = ly.d_o;
-            g.cus = cus;
             Timer tm(m, s, KC_GEMM_O, 2.0 * Td * qd * H);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -616,7 +611,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
                        1.f, nullptr, 0, (int)m->I};
             g.wd = ly.d_gu;
             g.out_scale = ly.s_act;
-            g.cus = cus;
             Timer tm(m, s, KC_GEMM_GATE_UP, 2.0 * Td * H * 2 * m->I);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -624,7 +618,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             GemmArgs g{act, m->I, ly.w_down, m->I, tmp, H, (int)T, (int)H, (int)m->I, EPI_STORE,
                        1.f, nullptr, 0, 0};
             g.wd = ly.d_down;
-            g.cus = cus;
             Timer tm(m, s, KC_GEMM_DOWN, 2.0 * Td * m->I * H);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -639,7 +632,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             g.wd = ly.d_pg;
             g.rs = h_rs;
             g.out_scale = ly.s_pg;
-            g.cus = cus;
             Timer tm(m, s, KC_GEMM_PLE_GATE, 2.0 * Td * H * P);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -648,7 +640,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
                        0, 0};
             g.wd = ly.d_pp;
             g.rs = h_rs;
-            g.cus = cus;
             Timer tm(m, s, KC_GEMM_PLE_PROJ, 2.0 * Td * P * H);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -669,7 +660,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         GemmArgs g{n, H, m->out_proj, H, proj, E, (int)T, (int)E, (int)H, EPI_STORE, 1.f, nullptr,
                    0, 0};
         g.wd = m->d_out_proj;
-        g.cus = cus;
         Timer tm(m, s, KC_GEMM_OUT, 2.0 * Td * H * E);
         HIP_TRY(launch_gemm(g, s));
     }
@@ -1063,13 +1053,7 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
         if (m->split) {
             ST_TRY(get(p + "pre_feedforward_layernorm.weight", nw));
             ly.s_ff = split_scale(norm_bound(nw));
-            // |gelu(g) u| <= |g| |u|
-            std::vector<double> bg, bu;
-            product_bound(b2.data(), m->I, H, nw.data(), &bg);
-            product_bound(c2.data(), m->I, H, nw.data(), &bu);
-            double act = 0;
-            for (size_t j = 0; j < bg.size(); ++j) act = std::max(act, bg[j] * bu[j]);
-            ly.s_act = split_scale(act);
+            ly.s_act = split_scale(geglu_bound(b2, c2, m->I, H, nw));
         }
         const std::vector<float> gu =
             interleave_gate_up(b2, c2, m->I, m->I_pad, m->H, m->split ? 16 : 32);

@@ -47,7 +47,6 @@ struct GemmArgs {
     const float *aux;
     int64_t ldaux;
     int n_out;  // EPI_GEGLU / EPI_CLIP_GLU: number of real output columns
-    int cus = 0;               // > 0: the launch shares the GPU with other streams
     int clip_cols = 0;         // output columns per clip segment (0: one segment)
     float clip[4][4] = {};     // per segment: input min, input max, output min, output max
     int64_t a_seg = 0;         // floats from one clip segment's A operand to the next's
@@ -90,6 +89,8 @@ hipError_t launch_gemm_simple(const GemmArgs &a, hipStream_t s);
 // CLIP_SILU) store split rows scaled by out_scale (out_scale / rs[m] with row
 // scales; ldc % 32 == 0, the output width a multiple of 32).
 hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s);
+// launch_gemm_conv on split operands.
+hipError_t launch_gemm_conv_split(const GemmArgs &a, hipStream_t s);
 constexpr int SPLIT_RASTER_M = 8;  // M blocks per rasterization group
 // x [rows, K] (leading dimension ldx) to split rows of K_pad >= K, each
 // scaled by its own power of two; descale[row] = also / scale.
@@ -218,21 +219,25 @@ hipError_t launch_finite_check(const float *x, int64_t n, int *flag, hipStream_t
 // ---- vision tower row kernels ------------------------------------------------
 // y = 2 * (x - 0.5), n % 4 == 0.
 hipError_t launch_patch_scale(const float *x, float *y, int64_t n, hipStream_t s);
+// In place on x [rows, 768], with a split copy of the rescaled rows.
+hipError_t launch_patch_scale_split(float *x, int64_t rows, SplitRows out, hipStream_t s);
 // h[t] += table[0][x_t] + table[1][y_t] with pos [T, 2] (x, y) and table
-// [2, pos_size, width]; n[t] = rms(h[t], w). width % 4 == 0, <= 2048.
+// [2, pos_size, width]; n[t] = rms(h[t], w), split rows times n_scale when it
+// is positive. width % 4 == 0, <= 2048.
 hipError_t launch_patch_pos(float *h, const int32_t *pos, const float *table, int64_t pos_size,
                             const float *w, float *n, int64_t rows, int width, float eps,
-                            int *flag, hipStream_t s);
+                            int *flag, hipStream_t s, float n_scale = 0.f);
 // In place on qkv[T, ld]: per-head q RMSNorm(qn) + axial RoPE, k RMSNorm(kn)
 // + axial RoPE, v unscaled RMSNorm. cos/sin tables are [coordinate, hd/4].
 hipError_t launch_qkv_post_axial(float *qkv, int64_t ld, int64_t tokens, int nh, int nkv, int hd,
                                  const float *qn, const float *kn, const float *cos_t,
                                  const float *sin_t, const int32_t *pos, float eps, int *flag,
                                  hipStream_t s);
-// out[s] = unscaled_rms((sum of h over bin s in patch order / divisor) * scale).
+// out[s] = unscaled_rms((sum of h over bin s in patch order / divisor) * scale),
+// split rows times out_scale when it is positive.
 hipError_t launch_pool_bins(const float *h, const int32_t *bin_start, const int32_t *bin_patch,
                             int64_t soft_tokens, int width, float divisor, float scale, float eps,
-                            float *out, int *flag, hipStream_t s);
+                            float *out, int *flag, hipStream_t s, float out_scale = 0.f);
 
 // ---- audio tower kernels -----------------------------------------------------
 
@@ -250,18 +255,24 @@ static_assert(sizeof(SscpRow) == 3 * sizeof(int32_t), "GemmArgs::conv_rows reads
 // masked frames skipped, LayerNorm + ReLU). C0 <= 512.
 hipError_t launch_sscp_conv0(const float *mel, const uint8_t *mask, const SscpRow *rows,
                              int64_t n_rows, const float *w, const float *ln, int C0, float eps,
-                             float *out, int *flag, hipStream_t s);
+                             float *out, int *flag, hipStream_t s, float out_scale = 0.f);
 // In place: x[p] = relu(layernorm(x[p], ln)) over C channels, n positions.
+// Both store split values times out_scale when it is positive (C0 = 128,
+// C = 32 or 64).
 hipError_t launch_sscp_ln_relu(float *x, const float *ln, int C, int64_t n, float eps, int *flag,
-                               hipStream_t s);
+                               hipStream_t s, float out_scale = 0.f);
 // Clamped stores of a row kernel's last output (the A operand of a clipped
 // linear): copy c goes to out + c * stride clamped to [lo[c], hi[c]]. The
-// default is one unclamped copy.
+// default is one unclamped copy. A copy with a positive scale is stored as
+// split rows; `split` receives a further, unclamped split copy.
 struct OutClamp {
     int copies = 1;
     int64_t stride = 0;
     float lo[3] = {-__builtin_huge_valf(), -__builtin_huge_valf(), -__builtin_huge_valf()};
     float hi[3] = {__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
+    float scale[3] = {0.f, 0.f, 0.f};
+    float *split = nullptr;
+    float split_scale = 0.f;
 };
 // t = w1 ? rms(clamp(x, +-c1), w1) : x; h = res ? res + t * rw : t (-> h_out);
 // if w2: n_out = rms(clamp(h, +-c2), w2). `oc` applies to the last output
@@ -287,6 +298,7 @@ struct AudioAttnArgs {
     int *flag;
     // the output projection's input bounds, applied as the output is stored
     float out_lo = -__builtin_huge_valf(), out_hi = __builtin_huge_valf();
+    float out_scale = 0.f;  // > 0: out holds split rows scaled by it
 };
 hipError_t launch_audio_attention(const AudioAttnArgs &a, hipStream_t s);
 // Causal depthwise conv (dw tap-major, [K, width]) within each clip, clamp, RMSNorm(w), SiLU,
@@ -294,10 +306,12 @@ hipError_t launch_audio_attention(const AudioAttnArgs &a, hipStream_t s);
 hipError_t launch_lconv(const float *gated, const float *dw, int K, const int32_t *pos, float clip,
                         const float *w, float *out, int64_t rows, int width, float eps, int *flag,
                         hipStream_t s, float out_lo = -__builtin_huge_valf(),
-                        float out_hi = __builtin_huge_valf());
-// out[j] = unscaled_rms(x[idx[j]]).
+                        float out_hi = __builtin_huge_valf(), float out_scale = 0.f);
+// out[j] = unscaled_rms(x[idx[j]]). Both store split rows times out_scale when
+// it is positive (width % 32 == 0).
 hipError_t launch_compact_rms(const float *x, const int32_t *idx, float *out, int64_t rows,
-                              int width, float eps, int *flag, hipStream_t s);
+                              int width, float eps, int *flag, hipStream_t s,
+                              float out_scale = 0.f);
 
 // ---- log-mel front end ---------------------------------------------------------
 // One clip of packed 16 kHz samples: samples [sample_base, sample_base +

@@ -47,6 +47,9 @@ struct VisLayer {
     float *w_qkv = nullptr, *w_o = nullptr, *w_gu = nullptr, *w_down = nullptr;
     float *ln_in = nullptr, *ln_post_attn = nullptr, *ln_pre_ff = nullptr, *ln_post_ff = nullptr,
           *q_norm = nullptr, *k_norm = nullptr;
+    // split towers: descale of each projection's outputs, scales of its operands
+    float *d_qkv = nullptr, *d_o = nullptr, *d_gu = nullptr, *d_down = nullptr;
+    float s_in = 0.f, s_ff = 0.f, s_act = 1.f;
 };
 
 }  // namespace
@@ -59,12 +62,18 @@ struct svl_vision_model {
     std::vector<float> inv_freq;  // axial_inv_freq, hd / 4 entries
     std::vector<float *> allocations;
     float *w_in = nullptr, *pos_table = nullptr, *w_proj = nullptr;
+    // Every projection runs on split operands (gemm_split.hip): the widths are
+    // multiples of 32. Other towers take the FP32 GEMMs.
+    bool split = false;
+    float *d_in = nullptr, *d_proj = nullptr;
+    float s_attn = 0.f, s_pool = 0.f;
     std::vector<VisLayer> layers;
     // axial RoPE angle tables [n_coord, hd/4] for coordinates 0..n_coord-1
     DevBuf<float> cos_t, sin_t;
     int64_t n_coord = 0;
     // workspace
-    DevBuf<float> pix, h, n, tmp, qkv, attn, act, pooled, soft;
+    // (split towers: qkv also holds the split patches, rs their scales)
+    DevBuf<float> pix, h, n, tmp, qkv, attn, act, pooled, soft, rs;
     DevBuf<int32_t> apos, rowlen;
     // A call's metadata in one device block, filled by one copy from pinned
     // host memory: the error flag (cleared), the patch coordinates, the
@@ -99,7 +108,7 @@ struct svl_vision_model {
         for (float *p : allocations) (void)hipFree(p);
         cos_t.release(); sin_t.release();
         pix.release(); h.release(); n.release(); tmp.release(); qkv.release(); attn.release();
-        act.release(); pooled.release(); soft.release();
+        act.release(); pooled.release(); soft.release(); rs.release();
         apos.release(); rowlen.release(); meta.release();
         if (ev_meta) {
             (void)hipEventSynchronize(ev_meta);
@@ -380,7 +389,8 @@ svl_status ensure_vis_workspace(svl_vision_model *v, const VisBatch &b) {
     HIP_TRY(v->h.ensure(T * v->H));
     HIP_TRY(v->n.ensure(T * v->H));
     HIP_TRY(v->tmp.ensure(T * v->H));
-    HIP_TRY(v->qkv.ensure(T * (v->qd + 2 * v->kd)));
+    HIP_TRY(v->qkv.ensure(T * std::max(v->qd + 2 * v->kd, v->split ? PATCH_VALUES : int64_t(0))));
+    if (v->split) HIP_TRY(v->rs.ensure(T));
     HIP_TRY(v->attn.ensure(T * v->qd));
     HIP_TRY(v->act.ensure(T * v->I));
     HIP_TRY(v->pooled.ensure(S * v->H));
@@ -444,7 +454,6 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
     if (R <= 0) return SVL_OK;
     int *flag = v->flag.p;
     const int64_t ldqkv = v->qd + 2 * v->kd;
-    const int cus = b.groups.size() > 1 ? (int)(256 / b.groups.size()) : 0;
     float *h = v->h.p + g.t0 * H, *n = v->n.p + g.t0 * H, *tmp = v->tmp.p + g.t0 * H,
           *qkv = v->qkv.p + g.t0 * ldqkv, *attn = v->attn.p + g.t0 * v->qd, *act = v->act.p + g.t0 * v->I;
     for (int64_t l = 0; l < v->L; ++l) {
@@ -452,7 +461,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         {
             GemmArgs ga{n, H, ly.w_qkv, H, qkv, ldqkv, (int)R, (int)ldqkv, (int)H, EPI_STORE, 1.f,
                         nullptr, 0, 0};
-            ga.cus = cus;
+            ga.wd = ly.d_qkv;
             HIP_TRY(launch_gemm(ga, s));
         }
         HIP_TRY(launch_qkv_post_axial(qkv, ldqkv, R, (int)v->NH, (int)v->NKV, (int)v->hd,
@@ -477,31 +486,33 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
             a.rowlen = v->rowlen.p;
             a.tokens = T;
             a.flag = flag;
+            a.out_scale = v->s_attn;
             HIP_TRY(launch_attention(a, s));
         }
         {
             GemmArgs ga{attn, v->qd, ly.w_o, v->qd, tmp, H, (int)R, (int)H, (int)v->qd, EPI_STORE,
                         1.f, nullptr, 0, 0};
-            ga.cus = cus;
+            ga.wd = ly.d_o;
             HIP_TRY(launch_gemm(ga, s));
         }
         HIP_TRY(launch_resnorm(tmp, ly.ln_post_attn, h, h, ly.ln_pre_ff, n, 1.0f, R, (int)H, v->eps,
-                               flag, s));
+                               flag, s, ly.s_ff));
         {
             GemmArgs ga{n, H, ly.w_gu, H, act, v->I, (int)R, (int)(2 * v->I_pad), (int)H, EPI_GEGLU,
                         1.f, nullptr, 0, (int)v->I};
-            ga.cus = cus;
+            ga.wd = ly.d_gu;
+            ga.out_scale = ly.s_act;
             HIP_TRY(launch_gemm(ga, s));
         }
         {
             GemmArgs ga{act, v->I, ly.w_down, v->I, tmp, H, (int)R, (int)H, (int)v->I, EPI_STORE,
                         1.f, nullptr, 0, 0};
-            ga.cus = cus;
+            ga.wd = ly.d_down;
             HIP_TRY(launch_gemm(ga, s));
         }
         const float *next = l + 1 < v->L ? v->layers[(size_t)l + 1].ln_in : nullptr;
         HIP_TRY(launch_resnorm(tmp, ly.ln_post_ff, h, h, next, next ? n : nullptr, 1.0f, R, (int)H,
-                               v->eps, flag, s));
+                               v->eps, flag, s, next ? v->layers[(size_t)l + 1].s_in : 0.f));
         if (h_hidden)
             HIP_TRY(hipMemcpyAsync(h_hidden + (size_t)((l + 1) * Ts * H), v->h.p,
                                    (size_t)(T * H) * 4, hipMemcpyDeviceToHost, s));
@@ -518,15 +529,18 @@ svl_status enqueue_vision(svl_vision_model *v, const VisBatch &b, float *d_pix, 
     if (T == 0) return SVL_OK;
     int *flag = v->flag.p;
     HIP_TRY(launch_positions(v->offsets.p, b.B, v->apos.p, v->rowlen.p, s));
-    HIP_TRY(launch_patch_scale(d_pix, d_pix, T * PATCH_VALUES, s));
+    if (v->split) HIP_TRY(launch_patch_scale_split(d_pix, T, SplitRows{v->qkv.p, v->rs.p}, s));
+    else HIP_TRY(launch_patch_scale(d_pix, d_pix, T * PATCH_VALUES, s));
     {
-        GemmArgs g{d_pix, PATCH_VALUES, v->w_in, PATCH_VALUES, v->h.p, H, (int)T, (int)H,
-                   (int)PATCH_VALUES, EPI_STORE, 1.f, nullptr, 0, 0};
+        GemmArgs g{v->split ? v->qkv.p : d_pix, PATCH_VALUES, v->w_in, PATCH_VALUES, v->h.p, H,
+                   (int)T, (int)H, (int)PATCH_VALUES, EPI_STORE, 1.f, nullptr, 0, 0};
+        g.wd = v->d_in;
+        g.rs = v->split ? v->rs.p : nullptr;
         HIP_TRY(launch_gemm(g, s));
     }
     // position add fused with layer 0's input norm (the model has >= 1 layer)
     HIP_TRY(launch_patch_pos(v->h.p, v->coord.p, v->pos_table, v->pos_size, v->layers[0].ln_in,
-                             v->n.p, T, (int)H, v->eps, flag, s));
+                             v->n.p, T, (int)H, v->eps, flag, s, v->layers[0].s_in));
     if (h_hidden)
         HIP_TRY(hipMemcpyAsync(h_hidden, v->h.p, (size_t)(T * H) * 4, hipMemcpyDeviceToHost, s));
 
@@ -545,10 +559,11 @@ svl_status enqueue_vision(svl_vision_model *v, const VisBatch &b, float *d_pix, 
     // pool_patches + rms_norm_rows_unscaled + embedding projection
     // (vision.rs:937-951).
     HIP_TRY(launch_pool_bins(v->h.p, v->bin_start.p, v->bin_patch.p, S, (int)H, (float)(POOL * POOL),
-                             std::sqrt((float)H), v->eps, v->pooled.p, flag, s));
+                             std::sqrt((float)H), v->eps, v->pooled.p, flag, s, v->s_pool));
     {
         GemmArgs g{v->pooled.p, H, v->w_proj, H, v->soft.p, v->text_hidden, (int)S,
                    (int)v->text_hidden, (int)H, EPI_STORE, 1.f, nullptr, 0, 0};
+        g.wd = v->d_proj;
         HIP_TRY(launch_gemm(g, s));
     }
     HIP_TRY(launch_finite_check(v->soft.p, S * v->text_hidden, flag, s));
@@ -744,33 +759,57 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         v->inv_freq.push_back(value);
     }
 
+    v->split = v->H % 32 == 0 && v->I % 32 == 0 && v->qd % 32 == 0;
+    std::vector<float> a, b2, c2, nw;
     auto up = [&](const std::string &name, float **dst) -> svl_status {
-        std::vector<float> a;
         ST_TRY(decode_named(by_name, name, a));
         return upload_owned(v->allocations, a.data(), a.size(), dst);
     };
-    ST_TRY(up("vision_tower.patch_embedder.input_proj.weight", &v->w_in));
+    // A projection weight [rows, K], for an A operand scaled by a_scale.
+    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, float **dst,
+                   float **descale) -> svl_status {
+        if (!v->split) return upload_owned(v->allocations, w.data(), w.size(), dst);
+        return upload_split(v->allocations, w.data(), (int64_t)w.size() / K, K, a_scale, dst,
+                            descale);
+    };
+    if (v->split) {
+        // convex sums of RMS-normalised value rows; unscaled norms of the bins
+        v->s_attn = split_scale(std::sqrt((double)v->hd));
+        v->s_pool = split_scale(std::sqrt((double)v->H));
+    }
+    ST_TRY(decode_named(by_name, "vision_tower.patch_embedder.input_proj.weight", a));
+    ST_TRY(put(a, PATCH_VALUES, 1.f, &v->w_in, &v->d_in));  // patches carry row scales
     ST_TRY(up("vision_tower.patch_embedder.position_embedding_table", &v->pos_table));
-    ST_TRY(up("embed_vision.embedding_projection.weight", &v->w_proj));
+    ST_TRY(decode_named(by_name, "embed_vision.embedding_projection.weight", a));
+    ST_TRY(put(a, v->H, v->s_pool, &v->w_proj, &v->d_proj));
     v->layers.resize((size_t)v->L);
-    std::vector<float> a, b2, c2;
     for (int64_t l = 0; l < v->L; ++l) {
         VisLayer &ly = v->layers[(size_t)l];
         const std::string p = "vision_tower.encoder.layers." + std::to_string(l) + ".";
         std::vector<float> qkv((size_t)((v->qd + 2 * v->kd) * v->H));
+        ST_TRY(decode_named(by_name, p + "input_layernorm.weight", nw));
+        if (v->split) ly.s_in = split_scale(norm_bound(nw));
         ST_TRY(decode_named(by_name, p + "self_attn.q_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin());
         ST_TRY(decode_named(by_name, p + "self_attn.k_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + v->qd * v->H);
         ST_TRY(decode_named(by_name, p + "self_attn.v_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + (v->qd + v->kd) * v->H);
-        ST_TRY(upload_owned(v->allocations, qkv.data(), qkv.size(), &ly.w_qkv));
-        ST_TRY(up(p + "self_attn.o_proj.linear.weight", &ly.w_o));
+        ST_TRY(put(qkv, v->H, ly.s_in, &ly.w_qkv, &ly.d_qkv));
+        ST_TRY(decode_named(by_name, p + "self_attn.o_proj.linear.weight", a));
+        ST_TRY(put(a, v->qd, v->s_attn, &ly.w_o, &ly.d_o));
         ST_TRY(decode_named(by_name, p + "mlp.gate_proj.linear.weight", b2));
         ST_TRY(decode_named(by_name, p + "mlp.up_proj.linear.weight", c2));
-        const std::vector<float> gu = interleave_gate_up(b2, c2, v->I, v->I_pad, v->H, 32);
-        ST_TRY(upload_owned(v->allocations, gu.data(), gu.size(), &ly.w_gu));
-        ST_TRY(up(p + "mlp.down_proj.linear.weight", &ly.w_down));
+        if (v->split) {
+            ST_TRY(decode_named(by_name, p + "pre_feedforward_layernorm.weight", nw));
+            ly.s_ff = split_scale(norm_bound(nw));
+            ly.s_act = split_scale(geglu_bound(b2, c2, v->I, v->H, nw));
+        }
+        const std::vector<float> gu =
+            interleave_gate_up(b2, c2, v->I, v->I_pad, v->H, v->split ? 16 : 32);
+        ST_TRY(put(gu, v->H, ly.s_ff, &ly.w_gu, &ly.d_gu));
+        ST_TRY(decode_named(by_name, p + "mlp.down_proj.linear.weight", a));
+        ST_TRY(put(a, v->I, ly.s_act, &ly.w_down, &ly.d_down));
         ST_TRY(up(p + "input_layernorm.weight", &ly.ln_in));
         ST_TRY(up(p + "post_attention_layernorm.weight", &ly.ln_post_attn));
         ST_TRY(up(p + "pre_feedforward_layernorm.weight", &ly.ln_pre_ff));
@@ -778,6 +817,7 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         ST_TRY(up(p + "self_attn.q_norm.weight", &ly.q_norm));
         ST_TRY(up(p + "self_attn.k_norm.weight", &ly.k_norm));
     }
+    if (v->split) HIP_TRY(hipStreamSynchronize(nullptr));  // the weights' conversion
     HIP_TRY(hipStreamCreateWithFlags(&v->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&v->extra, hipStreamNonBlocking));
     HIP_TRY(hipEventCreateWithFlags(&v->ev_fork, hipEventDisableTiming));

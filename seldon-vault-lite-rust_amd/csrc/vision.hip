@@ -40,6 +40,34 @@ hipError_t launch_patch_scale(const float *x, float *y, int64_t n, hipStream_t s
     return hipGetLastError();
 }
 
+// The same, one wave per patch of 768 values (three float4 per lane), with a
+// split copy of the rescaled patch for the patch projection.
+__global__ __launch_bounds__(256) void patch_scale_split_kernel(float *__restrict__ x, int64_t rows,
+                                                                SplitRows out) {
+    constexpr int NC = 3, WIDTH = 768;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    f32x4 *xr = (f32x4 *)(x + row * WIDTH);
+    f32x4 v[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = xr[lane + 64 * c];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[c][r] = 2.0f * (v[c][r] - 0.5f);
+        xr[lane + 64 * c] = v[c];
+    }
+    split_hidden<NC>(v, WIDTH / 4, lane, out, row, WIDTH);
+}
+
+hipError_t launch_patch_scale_split(float *x, int64_t rows, SplitRows out, hipStream_t s) {
+    if (rows <= 0) return hipSuccess;
+    hipLaunchKernelGGL(patch_scale_split_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s,
+                       x, rows, out);
+    return hipGetLastError();
+}
+
 // ---- position add + first input norm ----------------------------------------
 // h[t] += table[0][x_t] + table[1][y_t]   (the two table rows summed first,
 // as vision.rs:806-808 does), then n[t] = rms(h[t], w). One wave per patch.
@@ -50,7 +78,8 @@ __global__ __launch_bounds__(256) void patch_pos_kernel(float *__restrict__ h,
                                                         int64_t pos_size,
                                                         const float *__restrict__ w,
                                                         float *__restrict__ n, int64_t rows,
-                                                        int width, float eps, int *flag) {
+                                                        int width, float eps, int *flag,
+                                                        float n_scale) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
@@ -75,14 +104,14 @@ __global__ __launch_bounds__(256) void patch_pos_kernel(float *__restrict__ h,
     ss = wave_sum(ss);
     const float inv = rms_inverse(ss, width, eps);
     ok = ok && isfinite(ss);
-    f32x4 *nr = (f32x4 *)(n + row * width);
+    float *nr = n + row * width;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int i = lane + 64 * c;
         if (i < nv) {
             const f32x4 y = v[c] * inv * ((const f32x4 *)w)[i];
             ok = ok && finite4(y);
-            nr[i] = y;
+            store_row4(nr, i, y, n_scale);
         }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
@@ -90,16 +119,16 @@ __global__ __launch_bounds__(256) void patch_pos_kernel(float *__restrict__ h,
 
 hipError_t launch_patch_pos(float *h, const int32_t *pos, const float *table, int64_t pos_size,
                             const float *w, float *n, int64_t rows, int width, float eps,
-                            int *flag, hipStream_t s) {
+                            int *flag, hipStream_t s, float n_scale) {
     if (rows <= 0) return hipSuccess;
-    if (width % 4 || width > 2048) return hipErrorInvalidValue;
+    if (width % 4 || width > 2048 || (n_scale > 0.f && width % 32)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((rows + 3) / 4));
     switch ((width + 255) / 256) {
-        case 1: hipLaunchKernelGGL(patch_pos_kernel<1>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag); break;
-        case 2: hipLaunchKernelGGL(patch_pos_kernel<2>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag); break;
-        case 3: hipLaunchKernelGGL(patch_pos_kernel<3>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag); break;
-        case 4: hipLaunchKernelGGL(patch_pos_kernel<4>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag); break;
-        default: hipLaunchKernelGGL(patch_pos_kernel<8>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag); break;
+        case 1: hipLaunchKernelGGL(patch_pos_kernel<1>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag, n_scale); break;
+        case 2: hipLaunchKernelGGL(patch_pos_kernel<2>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag, n_scale); break;
+        case 3: hipLaunchKernelGGL(patch_pos_kernel<3>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag, n_scale); break;
+        case 4: hipLaunchKernelGGL(patch_pos_kernel<4>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag, n_scale); break;
+        default: hipLaunchKernelGGL(patch_pos_kernel<8>, grid, dim3(256), 0, s, h, pos, table, pos_size, w, n, rows, width, eps, flag, n_scale); break;
     }
     return hipGetLastError();
 }
@@ -250,7 +279,7 @@ __global__ __launch_bounds__(256) void pool_bins_kernel(const float *__restrict_
                                                         const int32_t *__restrict__ bin_patch,
                                                         int width, float divisor, float scale,
                                                         float eps, float *__restrict__ out,
-                                                        int *flag) {
+                                                        int *flag, float out_scale) {
     __shared__ float red[4];
     const int s = blockIdx.x, tid = threadIdx.x;
     const int k0 = bin_start[s], k1 = bin_start[s + 1];
@@ -281,7 +310,8 @@ __global__ __launch_bounds__(256) void pool_bins_kernel(const float *__restrict_
         if (col < width) {
             const float y = v[c] * inv;
             ok = ok && isfinite(y);
-            out[(int64_t)s * width + col] = y;
+            if (out_scale > 0.f) split_store1(out + (int64_t)s * width, col, y * out_scale);
+            else out[(int64_t)s * width + col] = y;
         }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
@@ -289,11 +319,11 @@ __global__ __launch_bounds__(256) void pool_bins_kernel(const float *__restrict_
 
 hipError_t launch_pool_bins(const float *h, const int32_t *bin_start, const int32_t *bin_patch,
                             int64_t soft_tokens, int width, float divisor, float scale, float eps,
-                            float *out, int *flag, hipStream_t s) {
+                            float *out, int *flag, hipStream_t s, float out_scale) {
     if (soft_tokens <= 0) return hipSuccess;
     if (width > 2048) return hipErrorInvalidValue;
     hipLaunchKernelGGL(pool_bins_kernel, dim3((unsigned)soft_tokens), dim3(256), 0, s, h,
-                       bin_start, bin_patch, width, divisor, scale, eps, out, flag);
+                       bin_start, bin_patch, width, divisor, scale, eps, out, flag, out_scale);
     return hipGetLastError();
 }
 
