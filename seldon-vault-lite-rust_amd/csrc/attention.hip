@@ -730,9 +730,11 @@ static hipError_t launch_attn16(const AttnArgs &a, hipStream_t s) {
 static std::atomic<int> g_attention_path{ATTN_PATH_AUTO};
 
 void set_attention_path(int path) { g_attention_path.store(path, std::memory_order_relaxed); }
+int get_attention_path() { return g_attention_path.load(std::memory_order_relaxed); }
 
 hipError_t launch_attention(const AttnArgs &a, hipStream_t s) {
     if (a.tokens <= 0) return hipSuccess;
+    if (a.split_qkv) return launch_attention_split(a, s);
     const dim3 block(64 * ATTN_WAVES);
     const int path = g_attention_path.load(std::memory_order_relaxed);
     if (path == ATTN_PATH_GENERIC) {

@@ -351,7 +351,8 @@ constexpr int QKV_MAX_HD = 1024;
 __global__ __launch_bounds__(256) void qkv_post_kernel(
     float *__restrict__ qkv, int64_t ld, int64_t tokens, int nh, int nkv, int hd,
     const float *__restrict__ qn, const float *__restrict__ kn, const float *__restrict__ cos_t,
-    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag) {
+    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag,
+    QkvSplit sc) {
     __shared__ float stage[4][QKV_MAX_HD];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int per_tok = nh + 2 * nkv;
@@ -368,14 +369,15 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(
     ss = wave_sum(ss);
     const float inv = rms_inverse(ss, hd, eps);
     bool ok = isfinite(ss);
+    float *st = stage[wave];
     if (kind == 2) {
         for (int i = lane; i < hd; i += 64) {
             const float y = row[i] * inv;
             ok = ok && isfinite(y);
-            row[i] = y;
+            if (sc.q > 0.f) st[i] = y * sc.v;
+            else row[i] = y;
         }
     } else {
-        float *st = stage[wave];
         for (int i = lane; i < hd; i += 64) st[i] = row[i] * inv * w[i];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -388,9 +390,22 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(
             const float a = first * c - second * sn;
             const float b = first * sn + second * c;
             ok = ok && isfinite(a) && isfinite(b);
-            row[j] = a;
-            row[j + half] = b;
+            if (sc.q > 0.f) {
+                // each lane reads its pair before it writes it
+                st[j] = kind == 0 ? a * sc.q_mul * sc.q : a * sc.k;
+                st[j + half] = kind == 0 ? b * sc.q_mul * sc.q : b * sc.k;
+            } else {
+                row[j] = a;
+                row[j + half] = b;
+            }
         }
+    }
+    if (sc.q > 0.f) {
+        // the whole row has been read: its split values replace it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int i = lane; i < hd; i += 64) split_store1(row, i, st[i]);
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
 }
@@ -404,7 +419,8 @@ template <int PAIRS, bool LOAD_FIRST>
 __global__ __launch_bounds__(256) void qkv_post256_kernel(
     float *__restrict__ qkv, int64_t ld, int64_t tokens, int nh, int nkv,
     const float *__restrict__ qn, const float *__restrict__ kn, const float *__restrict__ cos_t,
-    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag) {
+    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag,
+    QkvSplit sc) {
     const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (t >= tokens) return;
@@ -471,11 +487,12 @@ __global__ __launch_bounds__(256) void qkv_post256_kernel(
         if (k >= per_tok) continue;
         ok = ok && isfinite(ss[i]);
         const float inv = rms_inverse(ss[i], 256, eps);
+        float *head = qkv + t * ld + 256 * k;
         if (k >= nh + nkv) {  // value head: unscaled norm, no rotation
             const f32x4 y0 = x[i][0] * inv, y1 = x[i][1] * inv;
             ok = ok && finite4(y0) && finite4(y1);
-            row[128 * i] = y0;
-            row[128 * i + 32] = y1;
+            store_row4(head, l32, y0, sc.v);
+            store_row4(head, l32 + 32, y1, sc.v);
             continue;
         }
         const f32x4 first = x[i][0] * inv * (k < nh ? wq0 : wk0);
@@ -483,8 +500,13 @@ __global__ __launch_bounds__(256) void qkv_post256_kernel(
         const f32x4 a = first * c - second * sn;
         const f32x4 b = first * sn + second * c;
         ok = ok && finite4(a) && finite4(b);
-        row[128 * i] = a;
-        row[128 * i + 32] = b;
+        if (k < nh && sc.q > 0.f) {
+            split_store4(head, 4 * l32, a * sc.q_mul * sc.q);
+            split_store4(head, 128 + 4 * l32, b * sc.q_mul * sc.q);
+        } else {
+            store_row4(head, l32, a, sc.k);
+            store_row4(head, l32 + 32, b, sc.k);
+        }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
 }
@@ -496,7 +518,8 @@ template <int ROWS, bool LOAD_FIRST>
 __global__ __launch_bounds__(256) void qkv_post512_kernel(
     float *__restrict__ qkv, int64_t ld, int64_t tokens, int nh, int nkv,
     const float *__restrict__ qn, const float *__restrict__ kn, const float *__restrict__ cos_t,
-    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag) {
+    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag,
+    QkvSplit sc) {
     const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (t >= tokens) return;
@@ -558,11 +581,12 @@ __global__ __launch_bounds__(256) void qkv_post512_kernel(
         if (k >= per_tok) continue;
         ok = ok && isfinite(ss[k]);
         const float inv = rms_inverse(ss[k], 512, eps);
+        float *head = qkv + t * ld + 512 * k;
         if (k >= nh + nkv) {  // value head: unscaled norm, no rotation
             const f32x4 y0 = x[k][0] * inv, y1 = x[k][1] * inv;
             ok = ok && finite4(y0) && finite4(y1);
-            row[128 * k] = y0;
-            row[128 * k + 64] = y1;
+            store_row4(head, lane, y0, sc.v);
+            store_row4(head, lane + 64, y1, sc.v);
             continue;
         }
         const f32x4 first = x[k][0] * inv * (k < nh ? wq0 : wk0);
@@ -570,8 +594,13 @@ __global__ __launch_bounds__(256) void qkv_post512_kernel(
         const f32x4 a = first * c - second * sn;
         const f32x4 b = first * sn + second * c;
         ok = ok && finite4(a) && finite4(b);
-        row[128 * k] = a;
-        row[128 * k + 64] = b;
+        if (k < nh && sc.q > 0.f) {
+            split_store4(head, 4 * lane, a * sc.q_mul * sc.q);
+            split_store4(head, 256 + 4 * lane, b * sc.q_mul * sc.q);
+        } else {
+            store_row4(head, lane, a, sc.k);
+            store_row4(head, lane + 64, b, sc.k);
+        }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
 }
@@ -579,7 +608,7 @@ __global__ __launch_bounds__(256) void qkv_post512_kernel(
 hipError_t launch_qkv_post(float *qkv, int64_t ld, int64_t tokens, int nh, int nkv, int hd,
                            const float *qn, const float *kn, const float *cos_t,
                            const float *sin_t, const int32_t *pos, float eps, int *flag,
-                           hipStream_t s) {
+                           hipStream_t s, QkvSplit sc) {
     const int64_t head_rows = tokens * (nh + 2 * nkv);
     if (head_rows <= 0) return hipSuccess;
     if (hd > QKV_MAX_HD || hd % 2) return hipErrorInvalidValue;
@@ -590,17 +619,17 @@ hipError_t launch_qkv_post(float *qkv, int64_t ld, int64_t tokens, int nh, int n
         if (nh + 2 * nkv <= 6) {
             if (first)
                 hipLaunchKernelGGL((qkv_post256_kernel<3, true>), grid, dim3(256), 0, s, qkv, ld,
-                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag);
+                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
             else
                 hipLaunchKernelGGL((qkv_post256_kernel<3, false>), grid, dim3(256), 0, s, qkv, ld,
-                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag);
+                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
         } else {
             if (first)
                 hipLaunchKernelGGL((qkv_post256_kernel<4, true>), grid, dim3(256), 0, s, qkv, ld,
-                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag);
+                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
             else
                 hipLaunchKernelGGL((qkv_post256_kernel<4, false>), grid, dim3(256), 0, s, qkv, ld,
-                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag);
+                                   tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
         }
         return hipGetLastError();
     }
@@ -608,14 +637,14 @@ hipError_t launch_qkv_post(float *qkv, int64_t ld, int64_t tokens, int nh, int n
         const dim3 grid((unsigned)((tokens + 3) / 4));
         if (tokens < LOAD_FIRST_MAX_ROWS)
             hipLaunchKernelGGL((qkv_post512_kernel<6, true>), grid, dim3(256), 0, s, qkv, ld,
-                               tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag);
+                               tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
         else
             hipLaunchKernelGGL((qkv_post512_kernel<6, false>), grid, dim3(256), 0, s, qkv, ld,
-                               tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag);
+                               tokens, nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(qkv_post_kernel, dim3((unsigned)((head_rows + 3) / 4)), dim3(256), 0, s,
-                       qkv, ld, tokens, nh, nkv, hd, qn, kn, cos_t, sin_t, pos, eps, flag);
+                       qkv, ld, tokens, nh, nkv, hd, qn, kn, cos_t, sin_t, pos, eps, flag, sc);
     return hipGetLastError();
 }
 

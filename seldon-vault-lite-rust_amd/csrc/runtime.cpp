@@ -78,6 +78,7 @@ struct DevLayer {
     float *d_qkv = nullptr, *d_o = nullptr, *d_gu = nullptr, *d_down = nullptr, *d_pg = nullptr,
           *d_pp = nullptr;
     float s_in = 0.f, s_ff = 0.f, s_attn = 0.f, s_act = 1.f, s_pg = 1.f;
+    QkvSplit s_heads;  // of the normalised and rotated Q, K and V rows
 };
 
 struct TimedLaunch {
@@ -563,10 +564,14 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             Timer tm(m, s, KC_GEMM_QKV, 2.0 * Td * H * ldqkv);
             HIP_TRY(launch_gemm(g, s));
         }
+        // attention on split head rows (validate_row caps every row)
+        const int64_t max_len = std::min<int64_t>(T, MAX_TEXT_TOKENS);
+        const bool split_heads = m->split && attention_takes_split(ly.hd, ldqkv, max_len);
         {
             Timer tm(m, s, KC_QKV_POST, Td * ldqkv * 8);
             HIP_TRY(launch_qkv_post(qkv, ldqkv, T, (int)m->NH, ly.nkv, ly.hd, ly.q_norm, ly.k_norm,
-                                    m->cos_t[ly.full], m->sin_t[ly.full], pos, m->eps, flag, s));
+                                    m->cos_t[ly.full], m->sin_t[ly.full], pos, m->eps, flag, s,
+                                    split_heads ? ly.s_heads : QkvSplit()));
         }
         {
             const auto range = grp.tile_ranges.at(std::make_pair(ly.nkv, ly.hd));
@@ -588,7 +593,12 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             a.rowlen = rowlen;
             a.tokens = T;
             a.flag = flag;
-            a.max_len = std::min<int64_t>(T, MAX_TEXT_TOKENS);  // validate_row caps every row
+            a.max_len = max_len;
+            a.split_qkv = split_heads;
+            if (split_heads) {
+                a.qk_descale = 1.0f / (ly.s_heads.q * ly.s_heads.k);
+                a.v_descale = 1.0f / ly.s_heads.v;
+            }
             a.shortest = grp.shortest;
             a.out_scale = ly.s_attn;
             Timer tm(m, s, KC_ATTENTION, grp.attn_flops[ly.full]);
@@ -1046,6 +1056,16 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
         ST_TRY(put(qkv, H, ly.s_in, &ly.w_qkv, &ly.d_qkv));
         // attention outputs are convex sums of RMS-normalised value rows
         if (m->split) ly.s_attn = split_scale(std::sqrt((double)ly.hd));
+        if (m->split) {
+            // a rotated row's values are at most the row's norm; scale 1.0
+            // (text.rs:421) times log2(e) for scores in log2 units
+            ST_TRY(get(p + "self_attn.q_norm.weight", nw));
+            ly.s_heads.q_mul = 1.4426950408889634f;
+            ly.s_heads.q = split_scale(norm_bound(nw) * ly.s_heads.q_mul);
+            ST_TRY(get(p + "self_attn.k_norm.weight", nw));
+            ly.s_heads.k = split_scale(norm_bound(nw));
+            ly.s_heads.v = ly.s_attn;
+        }
         ST_TRY(get(p + "self_attn.o_proj.weight", a));
         ST_TRY(put(a, qd, ly.s_attn, &ly.w_o, &ly.d_o));
         ST_TRY(get(p + "mlp.gate_proj.weight", b2));

@@ -4,6 +4,7 @@
 #include "gemm_split.hip"
 #include "rows.hip"
 #include "attention.hip"
+#include "attention_split.hip"
 #include "vision.hip"
 #include "audio.hip"
 #include "mel.hip"

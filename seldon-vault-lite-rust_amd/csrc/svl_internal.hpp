@@ -123,12 +123,19 @@ hipError_t launch_gather(const uint32_t *ids, const float *table, int64_t vocab,
                          float eps, int *flag, hipStream_t s, float n_scale = 0.f,
                          SplitRows hs = SplitRows());
 
+// Split head rows out of a Q/K/V norm kernel: queries times q_mul and then q,
+// keys times k, values times v (q == 0: FP32 rows, q_mul unused).
+struct QkvSplit {
+    float q = 0.f, k = 0.f, v = 0.f;
+    float q_mul = 1.f;
+};
+
 // In place on qkv[T, ld]: per-head q RMSNorm(q_norm) + RoPE, k RMSNorm(k_norm)
 // + RoPE, v unscaled RMSNorm. cos/sin tables are [positions, hd/2].
 hipError_t launch_qkv_post(float *qkv, int64_t ld, int64_t tokens, int nh, int nkv, int hd,
                            const float *qn, const float *kn, const float *cos_t,
                            const float *sin_t, const int32_t *pos, float eps, int *flag,
-                           hipStream_t s);
+                           hipStream_t s, QkvSplit sc = QkvSplit());
 
 // RoPE only (kernel seam): values [T, heads, hd], position = pos0 + t.
 hipError_t launch_rope(float *x, int64_t tokens, int heads, int hd, const float *cos_t,
@@ -161,16 +168,29 @@ struct AttnArgs {
     int64_t max_len = 0;    // bound on the row length (0: unknown, bounded by tokens)
     int64_t shortest = 0;   // shortest row of the launch (0: unknown)
     float out_scale = 0.f;  // > 0: out holds split rows scaled by it (ldo % 32 == 0)
+    // split operands (launch_attention_split): score = (q . k) * qk_descale in
+    // log2 units, value = v * v_descale
+    bool split_qkv = false;
+    float qk_descale = 1.f, v_descale = 1.f;
 };
+// Log2 of the scale of the probabilities' split (they stay below 2^(8 + 6)).
+constexpr float ATTN_P_LOG2 = 6.0f;
+// True when the models' attention over rows of at most max_len tokens (token
+// stride ld) runs on split operands: head_dim 64, 256 or 512, windows below 2
+// GiB, no other kernel forced by set_attention_path.
+bool attention_takes_split(int hd, int64_t ld, int64_t max_len);
 // Query vectors per work item of the MFMA kernel (0 if hd has no MFMA kernel).
 int attn_block_vectors(int hd);
 hipError_t launch_attention(const AttnArgs &a, hipStream_t s);
+// Q, K and V as split head rows (queries times scale * log2(e)); out_scale > 0.
+hipError_t launch_attention_split(const AttnArgs &a, hipStream_t s);
 // Attention kernel choice for every later launch in the process (a test
 // hook): by shape (the DMA kernel whenever a row's operand window fits 2 GiB),
 // the fallback that longer windows take (the register-staged MFMA kernel at
 // head_dim 64 / 128 / 256, the generic kernel at 512), or the generic kernel.
 constexpr int ATTN_PATH_AUTO = 0, ATTN_PATH_FALLBACK = 1, ATTN_PATH_GENERIC = 2;
 void set_attention_path(int path);
+int get_attention_path();
 
 // Scratch of the allocation-free attention entry point (noalloc.hip), one
 // copy per GPU: work items, then per-token positions and row lengths, then
@@ -232,7 +252,7 @@ hipError_t launch_patch_pos(float *h, const int32_t *pos, const float *table, in
 hipError_t launch_qkv_post_axial(float *qkv, int64_t ld, int64_t tokens, int nh, int nkv, int hd,
                                  const float *qn, const float *kn, const float *cos_t,
                                  const float *sin_t, const int32_t *pos, float eps, int *flag,
-                                 hipStream_t s);
+                                 hipStream_t s, QkvSplit sc = QkvSplit());
 // out[s] = unscaled_rms((sum of h over bin s in patch order / divisor) * scale),
 // split rows times out_scale when it is positive.
 hipError_t launch_pool_bins(const float *h, const int32_t *bin_start, const int32_t *bin_patch,

@@ -50,6 +50,7 @@ struct VisLayer {
     // split towers: descale of each projection's outputs, scales of its operands
     float *d_qkv = nullptr, *d_o = nullptr, *d_gu = nullptr, *d_down = nullptr;
     float s_in = 0.f, s_ff = 0.f, s_act = 1.f;
+    QkvSplit s_heads;  // of the normalised and rotated Q, K and V rows
 };
 
 }  // namespace
@@ -454,6 +455,11 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
     if (R <= 0) return SVL_OK;
     int *flag = v->flag.p;
     const int64_t ldqkv = v->qd + 2 * v->kd;
+    // attention on split head rows; its windows span one image
+    int64_t longest = 0;
+    for (size_t i = 0; i + 1 < b.offsets.size(); ++i)
+        longest = std::max(longest, b.offsets[i + 1] - b.offsets[i]);
+    const bool split_heads = v->split && v->hd <= 256 && attention_takes_split((int)v->hd, ldqkv, longest);
     float *h = v->h.p + g.t0 * H, *n = v->n.p + g.t0 * H, *tmp = v->tmp.p + g.t0 * H,
           *qkv = v->qkv.p + g.t0 * ldqkv, *attn = v->attn.p + g.t0 * v->qd, *act = v->act.p + g.t0 * v->I;
     for (int64_t l = 0; l < v->L; ++l) {
@@ -466,7 +472,8 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         }
         HIP_TRY(launch_qkv_post_axial(qkv, ldqkv, R, (int)v->NH, (int)v->NKV, (int)v->hd,
                                       ly.q_norm, ly.k_norm, v->cos_t.p, v->sin_t.p,
-                                      v->coord.p + 2 * g.t0, v->eps, flag, s));
+                                      v->coord.p + 2 * g.t0, v->eps, flag, s,
+                                      split_heads ? ly.s_heads : QkvSplit()));
         {
             AttnArgs a{};
             a.q = v->qkv.p;
@@ -487,6 +494,11 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
             a.tokens = T;
             a.flag = flag;
             a.out_scale = v->s_attn;
+            a.split_qkv = split_heads;
+            if (split_heads) {
+                a.qk_descale = 1.0f / (ly.s_heads.q * ly.s_heads.k);
+                a.v_descale = 1.0f / ly.s_heads.v;
+            }
             HIP_TRY(launch_attention(a, s));
         }
         {
@@ -796,6 +808,16 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         ST_TRY(decode_named(by_name, p + "self_attn.v_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + (v->qd + v->kd) * v->H);
         ST_TRY(put(qkv, v->H, ly.s_in, &ly.w_qkv, &ly.d_qkv));
+        if (v->split) {
+            // a rotated row's values are at most the row's norm; scale 1.0
+            // (vision.rs:881) times log2(e) for scores in log2 units
+            ST_TRY(decode_named(by_name, p + "self_attn.q_norm.weight", nw));
+            ly.s_heads.q_mul = 1.4426950408889634f;
+            ly.s_heads.q = split_scale(norm_bound(nw) * ly.s_heads.q_mul);
+            ST_TRY(decode_named(by_name, p + "self_attn.k_norm.weight", nw));
+            ly.s_heads.k = split_scale(norm_bound(nw));
+            ly.s_heads.v = v->s_attn;
+        }
         ST_TRY(decode_named(by_name, p + "self_attn.o_proj.linear.weight", a));
         ST_TRY(put(a, v->qd, v->s_attn, &ly.w_o, &ly.d_o));
         ST_TRY(decode_named(by_name, p + "mlp.gate_proj.linear.weight", b2));

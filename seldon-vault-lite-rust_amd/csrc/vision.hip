@@ -193,7 +193,8 @@ template <int EPL>
 __global__ __launch_bounds__(256) void qkv_post_axial_rows_kernel(
     float *__restrict__ qkv, int64_t ld, int64_t tokens, int nh, int nkv,
     const float *__restrict__ qn, const float *__restrict__ kn, const float *__restrict__ cos_t,
-    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag) {
+    const float *__restrict__ sin_t, const int32_t *__restrict__ pos, float eps, int *flag,
+    QkvSplit sc) {
     constexpr int RL = 16, HD = RL * EPL, HALF = HD / 2, QUARTER = HD / 4;
     static_assert(QUARTER % RL == 0, "rotation pairs share a lane");
     const int slots = nh + 2 * nkv;
@@ -231,15 +232,22 @@ __global__ __launch_bounds__(256) void qkv_post_axial_rows_kernel(
             const float y0 = f * c - g * sn;
             const float y1 = g * c + f * sn;
             ok = ok && isfinite(y0) && isfinite(y1);
-            row[e0] = y0;
-            row[e1] = y1;
+            if (sc.q > 0.f) {
+                const bool q = slot < nh;
+                split_store1(row, e0, q ? y0 * sc.q_mul * sc.q : y0 * sc.k);
+                split_store1(row, e1, q ? y1 * sc.q_mul * sc.q : y1 * sc.k);
+            } else {
+                row[e0] = y0;
+                row[e1] = y1;
+            }
         }
     } else {
 #pragma unroll
         for (int m = 0; m < EPL; ++m) {
             const float y = v[m] * inv;
             ok = ok && isfinite(y);
-            row[sub + RL * m] = y;
+            if (sc.q > 0.f) split_store1(row, sub + RL * m, y * sc.v);
+            else row[sub + RL * m] = y;
         }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
@@ -248,14 +256,14 @@ __global__ __launch_bounds__(256) void qkv_post_axial_rows_kernel(
 hipError_t launch_qkv_post_axial(float *qkv, int64_t ld, int64_t tokens, int nh, int nkv, int hd,
                                  const float *qn, const float *kn, const float *cos_t,
                                  const float *sin_t, const int32_t *pos, float eps, int *flag,
-                                 hipStream_t s) {
+                                 hipStream_t s, QkvSplit sc) {
     if (tokens <= 0) return hipSuccess;
-    if (hd % 4) return hipErrorInvalidValue;
+    if (hd % 4 || (sc.q > 0.f && hd != 64 && hd != 128 && hd != 256)) return hipErrorInvalidValue;
     const int64_t rows = tokens * (nh + 2 * nkv);
     const dim3 grid16((unsigned)((rows + 15) / 16));
 #define QPA_LAUNCH(EPL)                                                                       \
     hipLaunchKernelGGL(qkv_post_axial_rows_kernel<EPL>, grid16, dim3(256), 0, s, qkv, ld, tokens, \
-                       nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag)
+                       nh, nkv, qn, kn, cos_t, sin_t, pos, eps, flag, sc)
     switch (hd) {
         case 64: QPA_LAUNCH(4); break;
         case 128: QPA_LAUNCH(8); break;

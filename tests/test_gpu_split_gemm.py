@@ -60,3 +60,23 @@ def test_split_scales_follow_the_weights(gain):
     ref = O.OracleTextModel(cfg, w).forward(row)["normalized"]
     assert np.abs(model.forward(row).normalized() - ref).max() <= 1e-4
     model.close()
+
+
+# head_dim 256, 512 (shape B's global layers) and 64, one and two layers deep: the rows alone take
+# the short-grid variants (several waves per 16 queries), the whole batch the large-grid ones
+@pytest.mark.parametrize("heads,kv,hd", [(3, 1, 256), (4, 2, 256), (4, 1, 512), (4, 4, 64)])
+def test_split_attention_matches_the_oracle_and_itself(heads, kv, hd):
+    cfg = small_config(256, 128, 64, heads, kv, hd, 128)
+    cfg.update(sliding_window=40)
+    w = svl_synth.weights(cfg, seed=7)
+    model = svl_amd.TextModel(svl_amd.TextConfig.from_json_value(cfg), w)
+    oracle = O.OracleTextModel(cfg, w)
+    # below one key tile, at its edges, past the window, and one long row
+    lengths = [1, 31, 32, 33, 64, 65, 129, 300] + [257] * 28
+    rows = svl_synth.token_rows(97, lengths, seed=8)
+    outs = model.forward_batch(rows)
+    for i in range(8):
+        alone = model.forward(rows[i])
+        assert np.array_equal(alone.projected(), outs[i].projected())
+        assert np.abs(alone.normalized() - oracle.forward(rows[i])["normalized"]).max() <= 1e-4
+    model.close()
