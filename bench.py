@@ -10,7 +10,7 @@ Token ids are resident in HBM before the timed region; every step runs the
 whole encoder and writes the normalised embeddings to HBM.
 
 Prints one JSON line: embeddings/s (value, timed on the production path:
-three row groups on three streams), the roofline of the dominant kernel (the
+one row group on one stream), the roofline of the dominant kernel (the
 gate/up GEMM; its launches timed with HIP events on the stream they run on,
 in a second pass of the same steps on one stream so that each kernel's
 duration is its own), the CPU oracle timed on this host's cores on a bounded
@@ -62,7 +62,7 @@ def parse():
                     help="timed batches of the headline batch at the manifest shape (0 skips it)")
     ap.add_argument("--host-steps", type=int, default=10,
                     help="timed batches of the host-ids to host-vectors path (0 skips it)")
-    ap.add_argument("--row-groups", type=int, default=3,
+    ap.add_argument("--row-groups", type=int, default=1,
                     help="row groups (streams) the batch is split into")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run a plain 1 GiB device-to-device copy (3 times), the reference "
@@ -526,8 +526,8 @@ def main():
         step()
     torch.cuda.synchronize()
 
-    # Timed region: K steps of the production path (row groups on their own
-    # streams, three by default), bracketed by device synchronisation.
+    # Timed region: K steps of the production path (one row group unless
+    # --row-groups asks for more), bracketed by device synchronisation.
     step_ms = []
     torch.cuda.synchronize()
     t0 = time.perf_counter()

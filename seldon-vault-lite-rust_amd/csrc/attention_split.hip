@@ -22,7 +22,11 @@
 //    last bit is 2^-24 of the half range, 2^-30 of the largest probability.
 //  * O^T += V^T . P^T: V rows stay row-major in LDS and are read transposed
 //    (ds_read_b64_tr_b16: a 16-lane group reads four keys x 16 dims, lane i
-//    receiving dim i of each key), four reads per 16-dim tile and 32 keys. The
+//    receiving dim i of each key), four reads per 16-dim tile and 32 keys. A
+//    tile's 16 dims are both halves of two chunks, and the V rows' chunks are
+//    swizzled so that the four keys of a group lie in different quarters of
+//    the banks: no conflicts (with the first halves of four chunks and the K
+//    rows' swizzle, conflicts took 36 % of the kernel's cycles). The
 //    mixed products run in an accumulator of their own from zero each tile and
 //    are added by the vector unit (the MFMA drops small addends' bits
 //    downwards, which a sum over thousands of positive weights would keep).
@@ -39,9 +43,12 @@ namespace svl {
 
 typedef __fp16 fp16x4_raw __attribute__((vector_size(8)));
 
+// Chunk swizzle of key r's V row.
+__device__ __forceinline__ int v_swizzle(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+
 // Four keys x 16 dims read transposed: `p` is this lane's 8-byte piece (key
-// (lane % 16) / 4 of the group's four, dims 4 (lane % 4) .. + 3); the result
-// holds dim lane % 16 of the four keys.
+// (lane % 16) / 4 of the group's four, piece lane % 4 of its 16 dims); the
+// result holds element lane % 16 of the four keys' pieces.
 __device__ __forceinline__ f16x4 read_transposed(const char *p) {
     const fp16x4_raw v = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
         (__attribute__((address_space(3))) fp16x4_raw *)p);
@@ -120,8 +127,8 @@ __global__ __launch_bounds__(64 * WAVES, MINB) void attn_split_kernel(AttnArgs p
     const int n_tiles = (k_hi - k_first) / KT + 1;
 
     // Buffer windows over this row's keys of this KV head; keys past the row
-    // end fall outside them and read as zero. Both operands' 16-byte chunks
-    // are XOR-swizzled by key % 16 on the way into LDS.
+    // end fall outside them and read as zero. The rows' 16-byte chunks are
+    // XOR-swizzled by key % 16 (V: v_swizzle of it) on the way into LDS.
     const int ldk = (int)p.ldk, ldv = (int)p.ldv;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(p.k + (int64_t)tile.tok0 * p.ldk + tile.kvh * HD), (short)0,
@@ -135,7 +142,7 @@ __global__ __launch_bounds__(64 * WAVES, MINB) void attn_split_kernel(AttnArgs p
         const int e = (wave * NDMA + q) * 256 + 4 * lane;
         const int r = e / HD, slot = (e % HD) / 4;
         koff[q] = (r * ldk + 4 * (slot ^ (r & 15))) * 4;
-        voff[q] = (r * ldv + 4 * (slot ^ (r & 15))) * 4;
+        voff[q] = (r * ldv + 4 * (slot ^ v_swizzle(r & 15))) * 4;
     }
     auto issue_k = [&](int k0) {
 #pragma unroll
@@ -155,7 +162,25 @@ __global__ __launch_bounds__(64 * WAVES, MINB) void attn_split_kernel(AttnArgs p
     issue_k(k_first);
     wait_vmcnt<0>();
     __syncthreads();
-    const int c0 = dpart * (HDW / 4);  // first 16-byte chunk of the wave's dims
+    // Fragment addresses: the swizzles move a chunk within its group of 16, so
+    // block b reads at the address of its parity plus a constant (an address
+    // per block would take 48 registers and spill).
+    const char *ks[2][2], *vs[2][2][2];  // [block parity][tile of the block][high, low]
+    {
+        const int c0 = dpart * (HDW / 4);  // first 16-byte chunk of the wave's dims
+        const int kr = 4 * g + (l16 >> 2), j = l16 & 3, vz = v_swizzle(kr);
+#pragma unroll
+        for (int pb = 0; pb < 2; ++pb)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl) {
+                ks[pb][hl] = (const char *)(Ks + l16 * HD) +
+                             16 * (c0 + ((8 * pb + 4 * hl + g) ^ l16));
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    vs[pb][e][hl] = (const char *)(Vs + kr * HD) + (j & 1) * 8 +
+                                    16 * (c0 + ((8 * pb + 4 * hl + 2 * e + (j >> 1)) ^ vz));
+            }
+    }
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     for (int it = 0; it < n_tiles; ++it) {
         const int k0 = k_first + it * KT;
@@ -164,19 +189,18 @@ __global__ __launch_bounds__(64 * WAVES, MINB) void attn_split_kernel(AttnArgs p
         // S^T for keys 16 kb + 4 g + r (register r of block kb), query l16
         f32x4 s[NKB];
         {
-            const float *kr = Ks + l16 * HD;
             f32x4 part[NP][NKB];
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
                 f32x4 hh[NKB], mx[NKB];
 #pragma unroll
                 for (int b = 2 * q; b < 2 * q + 2; ++b) {
-                    const int ch = c0 + 8 * b + g;
+                    const int at = 128 * (b & ~1);
                     f16x8 kh[NKB], kl[NKB];
 #pragma unroll
                     for (int kb = 0; kb < NKB; ++kb) {
-                        kh[kb] = *(const f16x8 *)(kr + kb * 16 * HD + 4 * (ch ^ l16));
-                        kl[kb] = *(const f16x8 *)(kr + kb * 16 * HD + 4 * ((ch + 4) ^ l16));
+                        kh[kb] = *(const f16x8 *)(ks[b & 1][0] + at + kb * 64 * HD);
+                        kl[kb] = *(const f16x8 *)(ks[b & 1][1] + at + kb * 64 * HD);
                     }
 #pragma unroll
                     for (int kb = 0; kb < NKB; ++kb)
@@ -266,20 +290,23 @@ __global__ __launch_bounds__(64 * WAVES, MINB) void attn_split_kernel(AttnArgs p
         }
         l_run += fold_xor16_32_sum(psum);
 
-        // O^T += V^T P^T: tile t is dims 16 t .. + 15 of the wave's block
+        // O^T += V^T P^T: tile t = 2 b + e takes chunks 2e and 2e + 1 of 32-dim
+        // block b, whose row 4 q .. 4 q + 3 (register r of lane group q) is
+        // dims 32 b + 8 e + 4 (q / 2) + 16 (q % 2) + r
         {
-            const int kr = 4 * g + (l16 >> 2), j = l16 & 3;  // this lane's key and piece
-            const char *vr = (const char *)(Vs + kr * HD);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const int ch = c0 + 8 * (t >> 1) + j, half = (t & 1) * 8;
-                const int oh = 16 * (ch ^ kr) + half, ol = 16 * ((ch + 4) ^ kr) + half;
+                const int b = t >> 1;
+                const char *ph0 = vs[b & 1][t & 1][0] + 128 * (b & ~1);
+                const char *pl0 = vs[b & 1][t & 1][1] + 128 * (b & ~1);
                 f32x4 mx = zero;
 #pragma unroll
                 for (int u = 0; u < KT / 32; ++u) {
-                    const char *b0 = vr + (32 * u) * HD * 4, *b1 = b0 + 16 * HD * 4;
-                    const f16x8 vh = __builtin_shufflevector(read_transposed(b0 + oh), read_transposed(b1 + oh), 0, 1, 2, 3, 4, 5, 6, 7);
-                    const f16x8 vl = __builtin_shufflevector(read_transposed(b0 + ol), read_transposed(b1 + ol), 0, 1, 2, 3, 4, 5, 6, 7);
+                    const int k0b = 128 * u * HD, k1b = k0b + 64 * HD;  // keys 32 u and 32 u + 16
+                    const f16x8 vh = __builtin_shufflevector(
+                        read_transposed(ph0 + k0b), read_transposed(ph0 + k1b), 0, 1, 2, 3, 4, 5, 6, 7);
+                    const f16x8 vl = __builtin_shufflevector(
+                        read_transposed(pl0 + k0b), read_transposed(pl0 + k1b), 0, 1, 2, 3, 4, 5, 6, 7);
                     mx = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[u], mx, 0, 0, 0);
                     o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[u], o[t], 0, 0, 0);
                     mx = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[u], mx, 0, 0, 0);
@@ -297,10 +324,10 @@ __global__ __launch_bounds__(64 * WAVES, MINB) void attn_split_kernel(AttnArgs p
         const int ocol = qhead * HD + dpart * HDW;
         bool ok = isfinite(inv);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const f32x4 x = o[2 * b] * inv, y = o[2 * b + 1] * inv;
-            ok = ok && finite4(x) && finite4(y);
-            split_store8(orow, ocol + 32 * b, g, x, y);
+        for (int t = 0; t < NT; ++t) {
+            const f32x4 y = o[t] * inv;
+            ok = ok && finite4(y);
+            split_store4(orow, ocol + 32 * (t >> 1) + 8 * (t & 1) + 4 * (g >> 1) + 16 * (g & 1), y);
         }
         if (!ok) raise_flag(p.flag, FLAG_NONFINITE);
     }

@@ -410,12 +410,12 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
 #endif
 }
 
-// The grouped tile order (RASTER) is taken by outputs of 1024 columns or
+// The grouped tile order (RASTER) is taken by outputs of 1280 columns or
 // more: 18688 x 2304 x 768 187.1 -> 185.4 us, 6230 x 2304 x 768 72.5 -> 69.7
 // us, and one-row launches, whose weights come from HBM, fetch each W panel on
 // one XCD (512 x 2304 x 768 16.6 -> 13.6 us). Narrower outputs keep N fastest
-// (6230 x 768 x 768 28.5 against 29.7 us).
-constexpr int SPLIT_RASTER_MIN_N = 1024;
+// (6230 x 768 x 768 26.5 against 27.2 us, 3000 x 1024 x 4096 75.7 against 79.4).
+constexpr int SPLIT_RASTER_MIN_N = 1280;
 
 template <int BM, int BN, int KB, int EPI, int MINB, int NS, int WMW, int WNW, bool CONV = false>
 static hipError_t launch_split_tile(const GemmArgs &a, hipStream_t s) {
@@ -444,9 +444,10 @@ static hipError_t launch_split_tile(const GemmArgs &a, hipStream_t s) {
 //  * Larger grids: the least work on the busiest CU, ceil(tiles / 256) times
 //    the tile's area over its measured rate: 128x128 (two per CU; a count of
 //    one runs alone on its CU and an odd count leaves half of it idle) 1,
-//    128x64 0.9, 64x64 0.75, ties to the larger. 18688 x 2304 x 768: 185 us
-//    on 128x128; 6230 x 768 x 1152: 40.0 on 128x64; 3000 x 1024 x 1024:
-//    23.1 on 64x64, 24.8 on 128x64.
+//    64x128 with the four waves side by side (three per CU) 0.87, 64x64 (four
+//    per CU) 0.72, ties to the larger. 18688 x 2304 x 768: 186 us on 128x128,
+//    197 on 64x128; 6230 x 768 x 768: 26.5 on 64x128, 28.4 on 128x64, 29.4 on
+//    128x128; 3000 x 1024 x 1024: 22.2 on 64x64, 25.0 on 64x128.
 // 256x128, 128x256 and 256x256 tiles (one workgroup per CU) were within 3 % or
 // slower on every shape swept.
 template <int EPI>
@@ -481,10 +482,10 @@ static hipError_t launch_split_auto(const GemmArgs &a, hipStream_t s) {
     auto per_cu = [&](int bm, int bn) { return (double)((tiles(bm, bn) + 255) / 256); };
     const double n128 = per_cu(128, 128);
     const double c128 = (n128 < 2 ? 1.25 : (int)n128 % 2 ? n128 + 0.5 : n128) * (128.0 * 128.0);
-    const double c12864 = per_cu(128, 64) * (128.0 * 64.0) / 0.9;
-    const double c64 = per_cu(64, 64) * (64.0 * 64.0) / 0.75;
-    if (c64 < c128 && c64 < c12864) return launch_split_tile<64, 64, 1, EPI, 4, 2, 2, 2>(a, s);
-    if (c12864 < c128) return launch_split_tile<128, 64, 1, EPI, 2, 2, 2, 2>(a, s);
+    const double c64128 = per_cu(64, 128) * (64.0 * 128.0) / 0.87;
+    const double c64 = per_cu(64, 64) * (64.0 * 64.0) / 0.72;
+    if (c64 < c128 && c64 < c64128) return launch_split_tile<64, 64, 1, EPI, 4, 2, 2, 2>(a, s);
+    if (c64128 < c128) return launch_split_tile<64, 128, 1, EPI, 3, 2, 1, 4>(a, s);
     return launch_split_tile<128, 128, 1, EPI, 2, 2, 2, 2>(a, s);
 }
 

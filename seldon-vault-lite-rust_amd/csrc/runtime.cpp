@@ -121,7 +121,7 @@ struct svl_text_model {
     static constexpr int MAX_GROUPS = 4;
     hipStream_t extra[MAX_GROUPS - 1] = {};  // streams of row groups 1..3
     hipEvent_t ev_fork = nullptr, ev_join[MAX_GROUPS - 1] = {};
-    int row_groups = 3;                      // row groups per large batch
+    int row_groups = 1;                      // row groups per large batch
     int64_t pass_tokens = 0;                 // tokens per pass (0: from PASS_BYTES)
     std::mutex mu;
 
@@ -356,12 +356,16 @@ void collect_timing(svl_text_model *m) {
 // ---------------------------------------------------------------------------
 // Per-call geometry.
 //
-// A large batch is cut into a few groups of consecutive rows with about the
-// same number of tokens. Each group runs the whole encoder on its own stream
-// (all at the default priority), on its own token range of every workspace
-// buffer, so the streams' kernels fill each other's partial last rounds of
-// workgroups and the bandwidth-bound norm kernels of one group overlap the
-// MFMA-bound GEMMs of another. Every row's arithmetic is unchanged.
+// A large batch may be cut into a few groups of consecutive rows with about
+// the same number of tokens. Each group runs the whole encoder on its own
+// stream (all at the default priority), on its own token range of every
+// workspace buffer, so the streams' kernels fill each other's partial last
+// rounds of workgroups. Every row's arithmetic is unchanged. One group is the
+// default: with the projections and attention on split operands a launch over
+// the whole batch fills the GPU better than three smaller ones beside each
+// other (64 rows, 18432 tokens: 19.5 ms as one group, 21.1 as two, 20.7 as
+// three; 30 rows, 8640 tokens: 10.3, 10.3, 10.9; 40 rows, 14640 tokens: 16.8,
+// 16.0, 18.5), where three groups were 11 % faster on FP32 MFMAs.
 
 constexpr int64_t SPLIT_MIN_TOKENS = 4096;
 
@@ -446,7 +450,7 @@ void build_groups(const svl_text_model *m, Batch &b, int max_groups) {
     // attention gives each XCD a contiguous range of its work items
     // (launch_attention). Concurrent row groups interleave their workgroups
     // over the XCDs and lose that placement, which is worth more than their
-    // overlap: 8 x 2048 tokens take 43.2 ms as one group, 44.3 ms as three.
+    // overlap.
     bool windowed = false;
     for (const DevLayer &ly : m->layers) windowed = windowed || !ly.full;
     if (windowed && m->window >= 0 && b.B > 0) {
