@@ -298,15 +298,18 @@ double clamp_bound(double bound, float lo, float hi) {
 }
 
 // Largest magnitude of a clipped linear's outputs over inputs clamp(x, in)
-// with x = RMSNorm(.) * norm of width K (Cauchy-Schwarz).
-double clipped_bound(const std::vector<float> &w, int64_t K, const std::vector<float> &norm,
-                     const Bounds &b) {
-    const int64_t rows = (int64_t)w.size() / K;
-    const double most = std::max(std::fabs((double)b.v[0]), std::fabs((double)b.v[1]));
-    double out = product_bound(w.data(), rows, K, nullptr) * most;
-    if (b.v[0] <= 0.f && b.v[1] >= 0.f)
-        out = std::min(out, product_bound(w.data(), rows, K, norm.data()));
-    return clamp_bound(out, b.v[2], b.v[3]);
+// with x = RMSNorm(.) * norm of width K, for its uploaded FP32 weight.
+svl_status clipped_bound(const float *w, int64_t rows, int64_t K, const float *norm,
+                         const Bounds &b, float *scratch, double *out) {
+    std::vector<float> each;
+    ST_TRY(product_bounds(w, rows, K, nullptr, scratch, each));
+    double bound = largest(each) * std::max(std::fabs((double)b.v[0]), std::fabs((double)b.v[1]));
+    if (b.v[0] <= 0.f && b.v[1] >= 0.f) {  // the clamp only shrinks
+        ST_TRY(product_bounds(w, rows, K, norm, scratch, each));
+        bound = std::min(bound, largest(each));
+    }
+    *out = clamp_bound(bound, b.v[2], b.v[3]);
+    return SVL_OK;
 }
 
 // The FFN up projection's SiLU output is the down projection's A operand.
@@ -959,11 +962,18 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             ST_TRY(read_bounds(by_name, q + "ffw_layer_2", ly.ff_b2[f]));
             ST_TRY(norm_scale(q + "pre_layer_norm.weight", &ly.ff_b1[f], &ly.s_up[f]));
             ST_TRY(decode_named(by_name, q + "ffw_layer_1.linear.weight", a));
-            ST_TRY(put(a, m->H, ly.s_up[f], &ly.ff_w1[f], &ly.d_w1[f]));
-            // |silu(x)| <= |x|, then the down projection's input clamp
-            if (m->split)
-                ly.s_down[f] = split_scale(clamp_bound(clipped_bound(a, m->H, nw, ly.ff_b1[f]),
-                                                       ly.ff_b2[f].v[0], ly.ff_b2[f].v[1]));
+            if (m->split) {
+                // |silu(x)| <= |x|, then the down projection's input clamp
+                double up_bound;
+                ST_TRY(upload_rows(m->allocations, a.data(), m->I, m->H, &ly.ff_w1[f], &ly.d_w1[f]));
+                ST_TRY(clipped_bound(ly.ff_w1[f], m->I, m->H, ly.ff_pre[f], ly.ff_b1[f],
+                                     ly.d_w1[f], &up_bound));
+                ly.s_down[f] =
+                    split_scale(clamp_bound(up_bound, ly.ff_b2[f].v[0], ly.ff_b2[f].v[1]));
+                ST_TRY(split_weight(ly.ff_w1[f], m->I, m->H, ly.s_up[f], ly.d_w1[f]));
+            } else {
+                ST_TRY(upload_owned(m->allocations, a.data(), a.size(), &ly.ff_w1[f]));
+            }
             ST_TRY(decode_named(by_name, q + "ffw_layer_2.linear.weight", a));
             ST_TRY(put(a, m->I, ly.s_down[f], &ly.ff_w2[f], &ly.d_w2[f]));
         }
@@ -976,14 +986,18 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             ST_TRY(read_bounds(by_name, p + "self_attn." + projs[j], *bs[j]));
             ST_TRY(norm_scale(p + "norm_pre_attn.weight", bs[j], &ly.s_qkv[j]));
         }
-        // `a` holds the value projection: attention outputs are convex sums of
-        // its outputs (or zero)
-        const double v_bound = m->split ? clipped_bound(a, m->H, nw, ly.bv) : 0;
-        if (m->split)
-            ST_TRY(upload_split_parts(m->allocations, qkv.data(), 3, m->H, m->H, ly.s_qkv,
-                                      &ly.w_qkv, &ly.d_qkv));
-        else
+        ST_TRY(up(p + "norm_pre_attn.weight", &ly.norm_pre_attn));
+        double v_bound = 0;  // attention outputs are convex sums of value rows (or zero)
+        if (m->split) {
+            const int64_t H = m->H;
+            ST_TRY(upload_rows(m->allocations, qkv.data(), 3 * H, H, &ly.w_qkv, &ly.d_qkv));
+            ST_TRY(clipped_bound(ly.w_qkv + 2 * H * H, H, H, ly.norm_pre_attn, ly.bv, ly.d_qkv,
+                                 &v_bound));
+            for (int j = 0; j < 3; ++j)
+                ST_TRY(split_weight(ly.w_qkv + j * H * H, H, H, ly.s_qkv[j], ly.d_qkv + j * H));
+        } else {
             ST_TRY(upload_owned(m->allocations, qkv.data(), qkv.size(), &ly.w_qkv));
+        }
         ST_TRY(read_bounds(by_name, p + "self_attn.post", ly.bpost));
         if (m->split) ly.s_post = split_scale(clamp_bound(v_bound, ly.bpost.v[0], ly.bpost.v[1]));
         ST_TRY(decode_named(by_name, p + "self_attn.post.linear.weight", a));
@@ -1039,7 +1053,6 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             ST_TRY(upload_owned(m->allocations, dwt.data(), dwt.size(), &ly.dw));
         }
         ST_TRY(up(p + "lconv1d.conv_norm.weight", &ly.lc_norm));
-        ST_TRY(up(p + "norm_pre_attn.weight", &ly.norm_pre_attn));
         ST_TRY(up(p + "norm_post_attn.weight", &ly.norm_post_attn));
         ST_TRY(up(p + "norm_out.weight", &ly.norm_out));
     }

@@ -127,11 +127,8 @@ __device__ __forceinline__ float sigmoid_ref(float v) {
 // Scales are powers of two that keep every |x * scale| at most 2^14 or so:
 // halves reach 65504, and the low half's last bit is 2^-24, 2^-38 of that.
 __device__ __forceinline__ void split4(const f32x4 v, f16x4 &hi, f16x4 &lo) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        hi[r] = (_Float16)v[r];
-        lo[r] = (_Float16)(v[r] - (float)hi[r]);
-    }
+    hi = __builtin_convertvector(v, f16x4);
+    lo = __builtin_convertvector(v - __builtin_convertvector(hi, f32x4), f16x4);
 }
 
 // Values col .. col + 3 (col % 4 == 0) of a split row, already scaled.

@@ -543,6 +543,32 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float *x, int64_t
     if (lane == 0) descale[row] = also / sc;
 }
 
+// One wave per row; the squares are summed in double (no overflow or underflow
+// of the floats' range).
+__global__ __launch_bounds__(256) void row_bounds_kernel(const float *__restrict__ x, int64_t rows,
+                                                         int K, const float *__restrict__ w,
+                                                         float *__restrict__ out) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    double s = 0.0;
+    for (int k = lane; k < K; k += 64) {
+        const double v = (double)x[row * K + k] * (w ? (double)w[k] : 1.0);
+        s += v * v;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0) out[row] = (float)(sqrt(s * (double)K) * 1.0005);
+}
+
+hipError_t launch_row_bounds(const float *x, int64_t rows, int K, const float *w, float *out,
+                             hipStream_t s) {
+    if (rows <= 0) return hipSuccess;
+    hipLaunchKernelGGL(row_bounds_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x,
+                       rows, K, w, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_split_rows(const float *x, int64_t ldx, int64_t rows, int K, int K_pad,
                              float also, float *out, float *descale, hipStream_t s) {
     if (rows <= 0) return hipSuccess;

@@ -201,77 +201,65 @@ inline double norm_bound(const std::vector<float> &w) {
     return std::sqrt((double)w.size()) * mx;
 }
 
-// Largest |RMSNorm(x) * w . row| over the rows [rows, K] of a weight
-// (Cauchy-Schwarz: sqrt(K) * |w o row|; w null: a K-vector of norm sqrt(K)),
-// written per row to `each` when given.
-inline double product_bound(const float *rows, int64_t n, int64_t K, const float *w,
-                            std::vector<double> *each = nullptr) {
-    double mx = 0;
-    if (each) each->resize((size_t)n);
-    for (int64_t r = 0; r < n; ++r) {
-        const float *row = rows + r * K;
-        // independent float sums (vector code); the margin covers their rounding
-        float part[16] = {0};
-        int64_t k = 0;
-        for (; k + 16 <= K; k += 16)
-            for (int j = 0; j < 16; ++j) {
-                const float v = w ? row[k + j] * w[k + j] : row[k + j];
-                part[j] += v * v;
-            }
-        double s = 0;
-        for (float q : part) s += q;
-        s *= 1.001;
-        for (; k < K; ++k) s += std::pow((double)row[k] * (w ? (double)w[k] : 1.0), 2);
-        // squares outside the float range
-        if (!std::isfinite(s) || s < 1e-30) {
-            s = 0;
-            for (k = 0; k < K; ++k) s += std::pow((double)row[k] * (w ? (double)w[k] : 1.0), 2);
-        }
-        s = std::sqrt(s * (double)K);
-        if (each) (*each)[(size_t)r] = s;
-        mx = std::max(mx, s);
-    }
-    return mx;
-}
-
-// Largest |gelu(g) u| of the gate and up projections [I, K] of RMSNorm(x) * w:
-// at most |g| |u|.
-inline double geglu_bound(const std::vector<float> &gate, const std::vector<float> &up, int64_t I,
-                          int64_t K, const std::vector<float> &w) {
-    std::vector<double> bg, bu;
-    (void)product_bound(gate.data(), I, K, w.data(), &bg);
-    (void)product_bound(up.data(), I, K, w.data(), &bu);
-    double mx = 0;
-    for (size_t j = 0; j < bg.size(); ++j) mx = std::max(mx, bg[j] * bu[j]);
-    return mx;
-}
-
-// A weight [rows, K] (K % 32 == 0) as split rows with the per-output descale
-// of its GEMM: factor / (row scale * a_scale), a_scale the A operand's scale. The
-// rows are converted in place on the null stream; the caller waits for it
-// before other streams read them.
-// Parts [rows, K] of one weight may read A operands of their own scales.
-inline svl_status upload_split_parts(std::vector<float *> &owned, const float *host, int parts,
-                                     int64_t rows, int64_t K, const float *a_scale, float **w,
-                                     float **wd, float factor = 1.f) {
-    const size_t count = (size_t)(parts * rows * K);
+// A weight [rows, K] (K % 32 == 0) in device memory, still FP32, with room for
+// the descale of each row behind it (K % 32 == 0 keeps it aligned).
+inline svl_status upload_rows(std::vector<float *> &owned, const float *host, int64_t rows,
+                              int64_t K, float **w, float **wd) {
+    const size_t count = (size_t)(rows * K);
     float *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, (count + (size_t)std::max<int64_t>(parts * rows, 1)) * sizeof(float)));
+    HIP_TRY(hipMalloc((void **)&d, (count + (size_t)std::max<int64_t>(rows, 1)) * sizeof(float)));
     owned.push_back(d);
     HIP_TRY(hipMemcpy(d, host, count * sizeof(float), hipMemcpyHostToDevice));
     *w = d;
-    d += count;  // the descales follow the weight (K % 32 == 0 keeps them aligned)
-    for (int j = 0; j < parts; ++j)
-        HIP_TRY(launch_split_rows(*w + j * rows * K, K, rows, (int)K, (int)K, factor / a_scale[j],
-                                  *w + j * rows * K, d + j * rows, nullptr));
-    *wd = d;
+    *wd = d + count;
+    return SVL_OK;
+}
+
+// Its rows become split rows in place, with the per-output descale of its
+// GEMM: factor / (row scale * a_scale), a_scale the A operand's scale. On the
+// null stream; the caller waits for it before other streams read them.
+inline svl_status split_weight(float *w, int64_t rows, int64_t K, float a_scale, float *wd,
+                               float factor = 1.f) {
+    HIP_TRY(launch_split_rows(w, K, rows, (int)K, (int)K, factor / a_scale, w, wd, nullptr));
     return SVL_OK;
 }
 
 inline svl_status upload_split(std::vector<float *> &owned, const float *host, int64_t rows,
                                int64_t K, float a_scale, float **w, float **wd,
                                float factor = 1.f) {
-    return upload_split_parts(owned, host, 1, rows, K, &a_scale, w, wd, factor);
+    ST_TRY(upload_rows(owned, host, rows, K, w, wd));
+    return split_weight(*w, rows, K, a_scale, *wd, factor);
+}
+
+// Largest |RMSNorm(x) * norm . row| of each row of an uploaded FP32 weight
+// (Cauchy-Schwarz: sqrt(K) * |norm o row|; norm null: K-vectors of norm
+// sqrt(K)). `scratch`: rows floats on the device (the weight's descales).
+inline svl_status product_bounds(const float *w, int64_t rows, int64_t K, const float *norm,
+                                 float *scratch, std::vector<float> &each) {
+    each.resize((size_t)rows);
+    HIP_TRY(launch_row_bounds(w, rows, (int)K, norm, scratch, nullptr));
+    HIP_TRY(hipMemcpy(each.data(), scratch, (size_t)rows * sizeof(float), hipMemcpyDeviceToHost));
+    return SVL_OK;
+}
+
+inline double largest(const std::vector<float> &v) {
+    double mx = 0;
+    for (float x : v) mx = std::max(mx, (double)x);
+    return mx;
+}
+
+// Largest |gelu(g) u| (at most |g| |u|) of a fused gate/up weight [2 I, K]
+// (16-row blocks) over RMSNorm(x) * norm.
+inline svl_status geglu_bound(const float *w, int64_t I, int64_t K, const float *norm,
+                              float *scratch, double *bound) {
+    std::vector<float> b;
+    ST_TRY(product_bounds(w, 2 * I, K, norm, scratch, b));
+    *bound = 0;
+    for (int64_t j = 0; j < I; ++j) {
+        const size_t at = (size_t)(32 * (j / 16) + j % 16);
+        *bound = std::max(*bound, (double)b[at] * (double)b[at + 16]);
+    }
+    return SVL_OK;
 }
 
 // Gate and up projections [I, H] interleaved in blocks of `block` rows

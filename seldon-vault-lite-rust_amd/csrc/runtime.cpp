@@ -1047,6 +1047,20 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
         ly.full = cfg->layer_type[l];
         m->type_hd[ly.full] = ly.hd;
         const int64_t H = m->H, qd = m->NH * ly.hd, kd = (int64_t)ly.nkv * ly.hd;
+        struct {
+            const char *name;
+            float **dst;
+        } norms[] = {{"input_layernorm.weight", &ly.ln_in},
+                     {"post_attention_layernorm.weight", &ly.ln_post_attn},
+                     {"pre_feedforward_layernorm.weight", &ly.ln_pre_ff},
+                     {"post_feedforward_layernorm.weight", &ly.ln_post_ff},
+                     {"ple_block.post_per_layer_input_norm.weight", &ly.ln_post_ple},
+                     {"self_attn.q_norm.weight", &ly.q_norm},
+                     {"self_attn.k_norm.weight", &ly.k_norm}};
+        for (auto &nm : norms) {
+            ST_TRY(get(p + nm.name, a));
+            ST_TRY(upload(m, a.data(), a.size(), nm.dst));
+        }
         // fused QKV weight: rows [q; k; v]
         std::vector<float> qkv((size_t)((qd + 2 * kd) * H));
         ST_TRY(get(p + "input_layernorm.weight", nw));
@@ -1074,39 +1088,36 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
         ST_TRY(put(a, qd, ly.s_attn, &ly.w_o, &ly.d_o));
         ST_TRY(get(p + "mlp.gate_proj.weight", b2));
         ST_TRY(get(p + "mlp.up_proj.weight", c2));
+        const std::vector<float> gu =
+            interleave_gate_up(b2, c2, m->I, m->I_pad, m->H, m->split ? 16 : 32);
         if (m->split) {
             ST_TRY(get(p + "pre_feedforward_layernorm.weight", nw));
             ly.s_ff = split_scale(norm_bound(nw));
-            ly.s_act = split_scale(geglu_bound(b2, c2, m->I, H, nw));
+            ST_TRY(upload_rows(m->allocations, gu.data(), 2 * m->I, H, &ly.w_gu, &ly.d_gu));
+            double act;
+            ST_TRY(geglu_bound(ly.w_gu, m->I, H, ly.ln_pre_ff, ly.d_gu, &act));
+            ly.s_act = split_scale(act);
+            ST_TRY(split_weight(ly.w_gu, 2 * m->I, H, ly.s_ff, ly.d_gu));
+        } else {
+            ST_TRY(upload(m, gu.data(), gu.size(), &ly.w_gu));
         }
-        const std::vector<float> gu =
-            interleave_gate_up(b2, c2, m->I, m->I_pad, m->H, m->split ? 16 : 32);
-        ST_TRY(put(gu, H, ly.s_ff, &ly.w_gu, &ly.d_gu));
         ST_TRY(get(p + "mlp.down_proj.weight", a));
         ST_TRY(put(a, m->I, ly.s_act, &ly.w_down, &ly.d_down));
         ST_TRY(get(p + "ple_block.per_layer_input_gate.weight", a));
-        ST_TRY(put(a, H, 1.f, &ly.w_pg, &ly.d_pg));
         // A hidden row whose scale is 1 / rs has values below 2^14 rs, so its
         // gates are at most 2^14 rs sqrt(H) |W row|; s_pg / rs brings gate x
         // per-layer input below 2^14.
-        if (m->split)
-            ly.s_pg = split_scale(16384.0 * product_bound(a.data(), m->P, H, nullptr) * ple_bound);
+        if (m->split) {
+            std::vector<float> b;
+            ST_TRY(upload_rows(m->allocations, a.data(), m->P, H, &ly.w_pg, &ly.d_pg));
+            ST_TRY(product_bounds(ly.w_pg, m->P, H, nullptr, ly.d_pg, b));
+            ly.s_pg = split_scale(16384.0 * largest(b) * ple_bound);
+            ST_TRY(split_weight(ly.w_pg, m->P, H, 1.f, ly.d_pg));
+        } else {
+            ST_TRY(upload(m, a.data(), a.size(), &ly.w_pg));
+        }
         ST_TRY(get(p + "ple_block.per_layer_projection.weight", a));
         ST_TRY(put(a, m->P, ly.s_pg, &ly.w_pp, &ly.d_pp));
-        struct {
-            const char *name;
-            float **dst;
-        } norms[] = {{"input_layernorm.weight", &ly.ln_in},
-                     {"post_attention_layernorm.weight", &ly.ln_post_attn},
-                     {"pre_feedforward_layernorm.weight", &ly.ln_pre_ff},
-                     {"post_feedforward_layernorm.weight", &ly.ln_post_ff},
-                     {"ple_block.post_per_layer_input_norm.weight", &ly.ln_post_ple},
-                     {"self_attn.q_norm.weight", &ly.q_norm},
-                     {"self_attn.k_norm.weight", &ly.k_norm}};
-        for (auto &nm : norms) {
-            ST_TRY(get(p + nm.name, a));
-            ST_TRY(upload(m, a.data(), a.size(), nm.dst));
-        }
         ST_TRY(get(p + "layer_scalar", a));
         ly.scalar = a[0];
     }

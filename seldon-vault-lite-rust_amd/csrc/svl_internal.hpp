@@ -96,6 +96,10 @@ constexpr int SPLIT_RASTER_M = 8;  // M blocks per rasterization group
 // scaled by its own power of two; descale[row] = also / scale.
 hipError_t launch_split_rows(const float *x, int64_t ldx, int64_t rows, int K, int K_pad,
                              float also, float *out, float *descale, hipStream_t s);
+// out[r] >= sqrt(K * sum_k (x[r, k] * w[k])^2) (w == nullptr: ones), at most
+// 0.1 % above it.
+hipError_t launch_row_bounds(const float *x, int64_t rows, int K, const float *w, float *out,
+                             hipStream_t s);
 
 // out = rms_norm_rows(x, w) (w == nullptr: unscaled).
 hipError_t launch_rms_rows(const float *x, const float *w, float *out, int64_t rows, int width,

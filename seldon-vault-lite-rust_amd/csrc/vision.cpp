@@ -822,19 +822,23 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         ST_TRY(put(a, v->qd, v->s_attn, &ly.w_o, &ly.d_o));
         ST_TRY(decode_named(by_name, p + "mlp.gate_proj.linear.weight", b2));
         ST_TRY(decode_named(by_name, p + "mlp.up_proj.linear.weight", c2));
-        if (v->split) {
-            ST_TRY(decode_named(by_name, p + "pre_feedforward_layernorm.weight", nw));
-            ly.s_ff = split_scale(norm_bound(nw));
-            ly.s_act = split_scale(geglu_bound(b2, c2, v->I, v->H, nw));
-        }
         const std::vector<float> gu =
             interleave_gate_up(b2, c2, v->I, v->I_pad, v->H, v->split ? 16 : 32);
-        ST_TRY(put(gu, v->H, ly.s_ff, &ly.w_gu, &ly.d_gu));
+        ST_TRY(up(p + "pre_feedforward_layernorm.weight", &ly.ln_pre_ff));
+        if (v->split) {
+            ly.s_ff = split_scale(norm_bound(a));  // `up` left the norm weights in a
+            ST_TRY(upload_rows(v->allocations, gu.data(), 2 * v->I, v->H, &ly.w_gu, &ly.d_gu));
+            double act;
+            ST_TRY(geglu_bound(ly.w_gu, v->I, v->H, ly.ln_pre_ff, ly.d_gu, &act));
+            ly.s_act = split_scale(act);
+            ST_TRY(split_weight(ly.w_gu, 2 * v->I, v->H, ly.s_ff, ly.d_gu));
+        } else {
+            ST_TRY(upload_owned(v->allocations, gu.data(), gu.size(), &ly.w_gu));
+        }
         ST_TRY(decode_named(by_name, p + "mlp.down_proj.linear.weight", a));
         ST_TRY(put(a, v->I, ly.s_act, &ly.w_down, &ly.d_down));
         ST_TRY(up(p + "input_layernorm.weight", &ly.ln_in));
         ST_TRY(up(p + "post_attention_layernorm.weight", &ly.ln_post_attn));
-        ST_TRY(up(p + "pre_feedforward_layernorm.weight", &ly.ln_pre_ff));
         ST_TRY(up(p + "post_feedforward_layernorm.weight", &ly.ln_post_ff));
         ST_TRY(up(p + "self_attn.q_norm.weight", &ly.q_norm));
         ST_TRY(up(p + "self_attn.k_norm.weight", &ly.k_norm));
