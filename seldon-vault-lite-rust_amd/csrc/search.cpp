@@ -30,6 +30,44 @@ using namespace svl;
 
 constexpr int64_t MAX_EMBEDDING_DIMENSION = 8192;  // storage/model.rs:35
 
+// Pinned host memory of an index that the kernels of one call read and write
+// in place of copies: per query a flag word, a candidate count and the page
+// length, and the page where it is small.
+constexpr size_t HOST_PAGE_BYTES = (size_t)1 << 20;  // larger pages are copied instead
+struct HostPage {
+    unsigned char *p = nullptr;
+    size_t bytes = 0;
+    int *flags = nullptr;
+    unsigned int *found = nullptr;
+    int64_t *take = nullptr, *index = nullptr;  // index, score: null for large pages
+    double *score = nullptr;
+
+    hipError_t ensure(int64_t nq, int64_t limit) {
+        const bool page = limit <= (int64_t)(HOST_PAGE_BYTES / 16) / nq;
+        const size_t need = (size_t)nq * 16 + (page ? (size_t)(nq * limit) * 16 : 0);
+        if (need > bytes) {
+            release();
+            const hipError_t e = hipHostMalloc((void **)&p, need, hipHostMallocDefault);
+            if (e != hipSuccess) {
+                p = nullptr;
+                return e;
+            }
+            bytes = need;
+        }
+        take = reinterpret_cast<int64_t *>(p);
+        flags = reinterpret_cast<int *>(take + nq);
+        found = reinterpret_cast<unsigned int *>(flags + nq);
+        index = page ? reinterpret_cast<int64_t *>(found + nq) : nullptr;
+        score = page ? reinterpret_cast<double *>(index + nq * limit) : nullptr;
+        return hipSuccess;
+    }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+};
+
 }  // namespace
 
 struct svl_vector_index {
@@ -45,12 +83,12 @@ struct svl_vector_index {
     // per-call workspace
     DevBuf<float> Q;
     DevBuf<double> qnorm, Qd;
-    DevBuf<int> qflags;
+    HostPage page;  // flags, counts and page entries that kernels write for the host
     DevBuf<uint8_t> mask;
     DevBuf<uint64_t> keys, keys_alt;
     DevBuf<uint32_t> idx, idx_alt, qkey;
     DevBuf<unsigned char> tmp;
-    DevBuf<uint64_t> samples, cand_key, cand_key_alt;
+    DevBuf<uint64_t> thresh, cand_key, cand_key_alt;
     DevBuf<uint32_t> cand_idx, cand_idx_alt;
     DevBuf<unsigned int> cnt, seg_begin, seg_end, blk_count;
     DevBuf<int64_t> take, out_index;
@@ -60,9 +98,9 @@ struct svl_vector_index {
     ~svl_vector_index() {
         if (device >= 0) (void)hipSetDevice(device);
         V.release(); cnorm.release(); perm.release(); Q.release(); qnorm.release();
-        qflags.release(); Qd.release(); mask.release(); keys.release(); keys_alt.release(); idx.release();
+        page.release(); Qd.release(); mask.release(); keys.release(); keys_alt.release(); idx.release();
         idx_alt.release(); qkey.release(); tmp.release(); take.release(); out_index.release();
-        samples.release(); cand_key.release(); cand_key_alt.release();
+        thresh.release(); cand_key.release(); cand_key_alt.release();
         cand_idx.release(); cand_idx_alt.release(); cnt.release(); seg_begin.release();
         seg_end.release(); blk_count.release();
         out_score.release();
@@ -97,53 +135,120 @@ svl_status check_query(const float *q, int64_t len, int64_t index_dim, bool has_
     return SVL_OK;
 }
 
-// Pages much smaller than the index (offset + limit <= n / 16): exact top-K
-// by threshold. S = 4096 evenly spaced keys per query are sorted; the sample
-// at a rank with margin above the expected (offset + limit) / n quantile is a
-// threshold, and every admitted key at or below it is a candidate (gathered
-// in position order without atomics). When each
-// query has at least min(offset + limit, admitted) candidates (and no more
-// than the buffer holds), its page lies among them, and sorting only the
-// candidates by (key, position) gives the ranking's exact entries; otherwise
-// `selected` stays false and the full sort runs.
-svl_status select_top(svl_vector_index *ix, int32_t nq, int64_t offset, int64_t limit,
-                      const std::vector<int64_t> &take, const std::vector<int64_t> &pass,
-                      int64_t *out_index, double *out_score, hipStream_t s, bool &selected) {
-    selected = false;
-    const int64_t n = ix->n, K = offset + limit;
-    constexpr int S = SAMPLE_COUNT;
-    if (n < 16 * S || K > n / 16) return SVL_OK;
-    const int64_t stride = n / S;
-    const double f = (double)K * S / (double)n;
-    const int rank = (int)std::min<double>(S - 1, std::ceil(1.5 * f + 4.0 * std::sqrt(f) + 8.0));
-    const int64_t cap = std::min<int64_t>(n, 2 * (int64_t)(rank + 1) * stride + 4096);
-    if ((int64_t)nq * cap > (int64_t)UINT32_MAX) return SVL_OK;
-    HIP_TRY(ix->samples.ensure((size_t)nq * S));
-    HIP_TRY(ix->cand_key.ensure((size_t)(nq * cap)));
-    HIP_TRY(ix->cand_key_alt.ensure((size_t)(nq * cap)));
-    HIP_TRY(ix->cand_idx.ensure((size_t)(nq * cap)));
-    HIP_TRY(ix->cand_idx_alt.ensure((size_t)(nq * cap)));
-    HIP_TRY(ix->cnt.ensure((size_t)nq));
-    HIP_TRY(ix->blk_count.ensure((size_t)nq * (size_t)candidate_blocks(n)));
-    if (nq <= SELECT_SAMPLE_MAX_QUERIES)
-        HIP_TRY(select_sample(ix->keys.p, nq, n, rank, ix->samples.p, s));
-    else
-        HIP_TRY(sort_samples(ix->keys.p, nq, n, ix->samples.p, s));
-    HIP_TRY(launch_compact_keys(ix->keys.p, nq, n, ix->samples.p, S, rank, cap, ix->blk_count.p,
-                                ix->cnt.p, ix->cand_key.p, ix->cand_idx.p, s));
-    std::vector<unsigned int> cnt((size_t)nq);
-    HIP_TRY(hipMemcpyAsync(cnt.data(), ix->cnt.p, (size_t)nq * sizeof(unsigned int),
+// The page from device memory, after the kernels that write it.
+svl_status copy_page(svl_vector_index *ix, int32_t nq, int64_t limit, int64_t *out_index,
+                     double *out_score, hipStream_t s) {
+    HIP_TRY(hipMemcpyAsync(out_index, ix->out_index.p, (size_t)(nq * limit) * 8,
+                           hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(out_score, ix->out_score.p, (size_t)(nq * limit) * 8,
                            hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    int64_t most = 0;
-    for (int32_t q = 0; q < nq; ++q) {
-        const int64_t need = std::min(K, pass[(size_t)q]);
-        if ((int64_t)cnt[(size_t)q] < need || (int64_t)cnt[(size_t)q] > cap) return SVL_OK;
-        most = std::max<int64_t>(most, cnt[(size_t)q]);
+    return SVL_OK;
+}
+
+// vector.rs:24-53 for queries in HBM: what launch_prepare_queries found, read
+// after a synchronisation. `flags` null: checked on the host before.
+svl_status check_flags(const int *flags, int32_t nq, int64_t query_dim, int64_t index_dim,
+                       bool has_dim) {
+    for (int32_t q = 0; flags && q < nq; ++q) {
+        if (flags[q] & 1)
+            return fail(SVL_USAGE, "query %d: query embedding contains a non-finite value", q);
+        if (flags[q] & 2)
+            return fail(SVL_USAGE,
+                        "query %d: query embedding norm is zero or non-finite; cosine similarity is undefined", q);
+        if (has_dim && query_dim != index_dim)
+            return fail(SVL_USAGE, "query %d: query embedding dimension %lld does not match the index dimension %lld",
+                        q, (long long)query_dim, (long long)index_dim);
     }
+    return SVL_OK;
+}
+
+// Pages much smaller than the index (offset + limit <= n / 16): exact top-K
+// by threshold. The sample (of 4096 evenly spaced keys per query) at a rank
+// with margin above the expected (offset + limit) / n quantile is a threshold,
+// and every admitted key at or below it is a candidate. When each query has at
+// least min(offset + limit, admitted) candidates (and no more than the buffer
+// holds), its page lies among them, and sorting only the candidates by (key,
+// position) gives the ranking's exact entries; otherwise `selected` stays
+// false and the full sort runs.
+//
+// Where twice the expected candidates fit one block's sort (pages within the
+// first 300 hits of 1M chunks, 1000 of 200k), candidates are collected in any order, sorted
+// and their page written, all enqueued at once: the host waits once and finds
+// flags, counts and entries in its own memory. One query against 200003 x 768
+// chunks takes 178 us this way (294 us with two waits in between, four copies
+// and candidates counted, scanned and written in order), 64 queries 508
+// (667). Longer lists are gathered in position order for a stable sort.
+struct Selection {
+    bool small = false, runs = false;
+    int rank = 0;
+    int64_t cap = 0;
+};
+
+Selection plan_selection(int64_t n, int64_t K, int32_t nq) {
+    Selection p;
+    constexpr int S = SAMPLE_COUNT;
+    if (n < 16 * S || K > n / 16) return p;
+    const int64_t stride = n / S;
+    const double f = (double)K * S / (double)n;
+    p.rank = (int)std::min<double>(S - 1, std::ceil(1.5 * f + 4.0 * std::sqrt(f) + 8.0));
+    const int64_t twice = 2 * (int64_t)(p.rank + 1) * stride;
+    p.small = twice <= CAND_LDS;
+    p.cap = p.small ? CAND_LDS : std::min<int64_t>(n, twice + 4096);
+    p.runs = (int64_t)nq * p.cap <= (int64_t)UINT32_MAX;
+    return p;
+}
+
+bool lists_hold_pages(const unsigned int *found, const std::vector<int64_t> &pass, int64_t K,
+                      int64_t cap, int64_t &most) {
+    most = 0;
+    for (size_t q = 0; q < pass.size(); ++q) {
+        if ((int64_t)found[q] < std::min(K, pass[q]) || (int64_t)found[q] > cap) return false;
+        most = std::max<int64_t>(most, found[q]);
+    }
+    return true;
+}
+
+svl_status ensure_candidates(svl_vector_index *ix, int32_t nq, int64_t cap) {
+    HIP_TRY(ix->thresh.ensure((size_t)nq));
+    HIP_TRY(ix->cnt.ensure((size_t)nq * CNT_STRIDE));
+    HIP_TRY(ix->cand_key.ensure((size_t)(nq * cap)));
+    HIP_TRY(ix->cand_idx.ensure((size_t)(nq * cap)));
+    return SVL_OK;
+}
+
+// Short lists: enqueued whole. The entries are in the host page, or in
+// out_index / out_score of the device for a large one.
+svl_status enqueue_short_lists(svl_vector_index *ix, const Selection &p, int32_t nq, int64_t offset,
+                               int64_t limit, hipStream_t s) {
+    HIP_TRY(launch_sample_threshold(ix->keys.p, nq, ix->n, p.rank, ix->thresh.p, ix->cnt.p, s));
+    HIP_TRY(launch_collect_candidates(ix->keys.p, nq, ix->n, ix->thresh.p, p.cap, ix->cnt.p,
+                                      ix->cand_key.p, ix->cand_idx.p, s));
+    const bool direct = ix->page.index != nullptr;
+    HIP_TRY(launch_rank_candidates(ix->cand_key.p, ix->cand_idx.p, ix->cnt.p, nq, ix->n, p.cap,
+                                   ix->perm.p, offset, limit, ix->page.take, ix->page.found,
+                                   direct ? ix->page.index : ix->out_index.p,
+                                   direct ? ix->page.score : ix->out_score.p, s));
+    return SVL_OK;
+}
+
+svl_status select_long_lists(svl_vector_index *ix, const Selection &p, int32_t nq, int64_t offset,
+                             int64_t limit, const std::vector<int64_t> &pass, int64_t *out_index,
+                             double *out_score, hipStream_t s, bool &selected) {
+    const int64_t n = ix->n, cap = p.cap;
+    HIP_TRY(ix->cand_key_alt.ensure((size_t)(nq * cap)));
+    HIP_TRY(ix->cand_idx_alt.ensure((size_t)(nq * cap)));
+    HIP_TRY(ix->blk_count.ensure((size_t)nq * (size_t)candidate_blocks(n)));
+    HIP_TRY(launch_sample_threshold(ix->keys.p, nq, n, p.rank, ix->thresh.p, ix->cnt.p, s));
+    HIP_TRY(launch_compact_keys(ix->keys.p, nq, n, ix->thresh.p, cap, ix->blk_count.p, ix->cnt.p,
+                                ix->page.found, ix->cand_key.p, ix->cand_idx.p, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    int64_t most;
+    if (!lists_hold_pages(ix->page.found, pass, offset + limit, cap, most)) return SVL_OK;
     if (most <= CAND_LDS) {
-        HIP_TRY(sort_candidates_lds(ix->cand_key.p, ix->cand_idx.p, ix->cand_key_alt.p,
-                                    ix->cand_idx_alt.p, ix->cnt.p, nq, cap, most, s));
+        HIP_TRY(launch_rank_candidates(ix->cand_key.p, ix->cand_idx.p, ix->cnt.p, nq, n, cap,
+                                       ix->perm.p, offset, limit, ix->page.take, ix->page.found,
+                                       ix->out_index.p, ix->out_score.p, s));
     } else {
         HIP_TRY(ix->seg_begin.ensure((size_t)nq));
         HIP_TRY(ix->seg_end.ensure((size_t)nq));
@@ -155,28 +260,31 @@ svl_status select_top(svl_vector_index *ix, int32_t nq, int64_t offset, int64_t 
         HIP_TRY(sort_candidates(ix->cand_key.p, ix->cand_idx.p, ix->cand_key_alt.p,
                                 ix->cand_idx_alt.p, ix->cnt.p, ix->seg_begin.p, ix->seg_end.p, nq,
                                 cap, ix->tmp.p, &b, s));
+        HIP_TRY(launch_gather_candidates(ix->cand_key_alt.p, ix->cand_idx_alt.p, nq, n, cap,
+                                         ix->perm.p, offset, limit, ix->page.take,
+                                         ix->out_index.p, ix->out_score.p, s));
     }
-    HIP_TRY(launch_gather_candidates(ix->cand_key_alt.p, ix->cand_idx_alt.p, nq, n, cap, ix->perm.p,
-                                     offset, limit, ix->take.p, ix->out_index.p,
-                                     ix->out_score.p, s));
-    HIP_TRY(hipMemcpyAsync(out_index, ix->out_index.p, (size_t)(nq * limit) * 8,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(out_score, ix->out_score.p, (size_t)(nq * limit) * 8,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    (void)take;
+    ST_TRY(copy_page(ix, nq, limit, out_index, out_score, s));
     selected = true;
     return SVL_OK;
 }
 
-// The ranking of `nq` validated queries already in ix->Q / ix->qnorm.
-svl_status rank_loaded(svl_vector_index *ix, int32_t nq, const uint8_t *mask, int64_t mask_stride,
-                       int64_t offset, int64_t limit, int64_t *out_index, double *out_score,
-                       int64_t *out_count, hipStream_t s) {
-    const int64_t n = ix->n;
+// The ranking of `nq` queries [nq, D] in HBM. With `norms` null their norms
+// are taken and checked on the device here (the first wait reports them),
+// otherwise `norms` holds those of queries that were checked on the host.
+svl_status rank_queries(svl_vector_index *ix, const float *queries, const double *norms,
+                        int32_t nq, int64_t query_dim, const uint8_t *mask, int64_t mask_stride,
+                        int64_t offset, int64_t limit, int64_t *out_index, double *out_score,
+                        int64_t *out_count, hipStream_t s) {
+    const int64_t n = ix->n, count = (int64_t)nq * n;
+    HIP_TRY(ix->qnorm.ensure((size_t)nq));
+    HIP_TRY(ix->page.ensure(nq, limit));
+    int *flags = norms ? nullptr : ix->page.flags;
     // admitted chunks per query, and the first admitted bad chunk (vector.rs:77-82)
-    std::vector<int64_t> take((size_t)nq), pass((size_t)nq, n);
-    for (int32_t q = 0; q < nq; ++q) {
+    std::vector<int64_t> pass((size_t)nq, n);
+    int64_t bad = -1;
+    int32_t bad_query = nq;
+    for (int32_t q = 0; q < nq && bad < 0; ++q) {
         if (mask) {
             const uint8_t *m = mask + (int64_t)q * mask_stride;
             int64_t cnt = 0;
@@ -184,23 +292,33 @@ svl_status rank_loaded(svl_vector_index *ix, int32_t nq, const uint8_t *mask, in
             pass[(size_t)q] = cnt;
         }
         for (int64_t b : ix->bad_list)
-            if (!mask || mask[(int64_t)q * mask_stride + b])
-                return fail(SVL_INTERNAL, "query %d: chunk %llu has a zero or non-finite embedding norm",
-                            q, (unsigned long long)ix->ids[(size_t)b]);
-        take[(size_t)q] = std::max<int64_t>(0, std::min(limit, pass[(size_t)q] - offset));
-        out_count[q] = take[(size_t)q];
+            if (!mask || mask[(int64_t)q * mask_stride + b]) {
+                bad = b;
+                bad_query = q;
+                break;
+            }
+        ix->page.take[q] = std::max<int64_t>(0, std::min(limit, pass[(size_t)q] - offset));
     }
-    if (n == 0 || limit == 0) return SVL_OK;
-    const int64_t count = (int64_t)nq * n;
-    if (count > (int64_t)UINT32_MAX) return fail(SVL_LIMIT, "queries x chunks exceeds 2^32 pairs");
+    if (bad >= 0 || n == 0 || limit == 0 || query_dim != ix->D || count > (int64_t)UINT32_MAX) {
+        // nothing to rank: the queries' own errors come first
+        if (flags) {
+            HIP_TRY(launch_prepare_queries(queries, nq, (int)query_dim, nullptr, ix->qnorm.p,
+                                           flags, s));
+            HIP_TRY(hipStreamSynchronize(s));
+            ST_TRY(check_flags(flags, nq, query_dim, ix->D, n > 0));
+        }
+        for (int32_t q = 0; q < bad_query; ++q) out_count[q] = ix->page.take[q];
+        if (bad >= 0)
+            return fail(SVL_INTERNAL, "query %d: chunk %llu has a zero or non-finite embedding norm",
+                        bad_query, (unsigned long long)ix->ids[(size_t)bad]);
+        if (n == 0 || limit == 0) return SVL_OK;
+        return fail(SVL_LIMIT, "queries x chunks exceeds 2^32 pairs");
+    }
     HIP_TRY(ix->keys.ensure((size_t)count));
-    HIP_TRY(ix->keys_alt.ensure((size_t)count));
-    HIP_TRY(ix->idx.ensure((size_t)count));
-    HIP_TRY(ix->idx_alt.ensure((size_t)count));
-    HIP_TRY(ix->qkey.ensure((size_t)count));
-    HIP_TRY(ix->take.ensure((size_t)nq));
     HIP_TRY(ix->out_index.ensure((size_t)(nq * limit)));
     HIP_TRY(ix->out_score.ensure((size_t)(nq * limit)));
+    const int qb = cosine_query_block(nq);
+    HIP_TRY(ix->Qd.ensure((size_t)(ix->D * ((nq + qb - 1) / qb * qb))));
     const uint8_t *d_mask = nullptr;
     int64_t d_stride = 0;
     if (mask) {
@@ -212,14 +330,37 @@ svl_status rank_loaded(svl_vector_index *ix, int32_t nq, const uint8_t *mask, in
         d_mask = ix->mask.p;
         d_stride = mask_stride == 0 ? 0 : n;
     }
-    const int qb = cosine_query_block(nq);
-    HIP_TRY(ix->Qd.ensure((size_t)(ix->D * ((nq + qb - 1) / qb * qb))));
-    HIP_TRY(launch_cosine_keys(ix->V.p, ix->cnorm.p, ix->Q.p, ix->qnorm.p, nq, n, (int)ix->D,
-                               d_mask, d_stride, ix->perm.p, ix->Qd.p, ix->keys.p, s));
-    HIP_TRY(hipMemcpyAsync(ix->take.p, take.data(), (size_t)nq * 8, hipMemcpyHostToDevice, s));
+    if (norms)
+        HIP_TRY(hipMemcpyAsync(ix->qnorm.p, norms, (size_t)nq * 8, hipMemcpyHostToDevice, s));
+    const Selection plan = plan_selection(n, offset + limit, nq);
+    if (plan.runs) ST_TRY(ensure_candidates(ix, nq, plan.cap));
+    HIP_TRY(launch_prepare_queries(queries, nq, (int)ix->D, ix->Qd.p, ix->qnorm.p, flags, s));
+    HIP_TRY(launch_cosine_keys(ix->V.p, ix->cnorm.p, ix->Qd.p, ix->qnorm.p, nq, n, (int)ix->D,
+                               d_mask, d_stride, ix->perm.p, ix->keys.p, s));
+    const bool small = plan.runs && plan.small;
+    if (small) ST_TRY(enqueue_short_lists(ix, plan, nq, offset, limit, s));
+    if (small || flags) HIP_TRY(hipStreamSynchronize(s));
+    ST_TRY(check_flags(flags, nq, query_dim, ix->D, true));
+    std::copy(ix->page.take, ix->page.take + nq, out_count);
+    int64_t most;
+    if (small && lists_hold_pages(ix->page.found, pass, offset + limit, plan.cap, most)) {
+        if (!ix->page.index) return copy_page(ix, nq, limit, out_index, out_score, s);
+        for (int32_t q = 0; q < nq; ++q) {
+            const int64_t at = (int64_t)q * limit, m = ix->page.take[q];
+            std::copy(ix->page.index + at, ix->page.index + at + m, out_index + at);
+            std::copy(ix->page.score + at, ix->page.score + at + m, out_score + at);
+        }
+        return SVL_OK;
+    }
     bool selected = false;
-    ST_TRY(select_top(ix, nq, offset, limit, take, pass, out_index, out_score, s, selected));
+    if (plan.runs && !plan.small)
+        ST_TRY(select_long_lists(ix, plan, nq, offset, limit, pass, out_index, out_score, s,
+                                 selected));
     if (selected) return SVL_OK;
+    HIP_TRY(ix->keys_alt.ensure((size_t)count));
+    HIP_TRY(ix->idx.ensure((size_t)count));
+    HIP_TRY(ix->idx_alt.ensure((size_t)count));
+    HIP_TRY(ix->qkey.ensure((size_t)count));
     size_t tmp_bytes = 0;
     const uint32_t *sorted = nullptr;
     HIP_TRY(rank_sort(ix->keys.p, ix->keys_alt.p, ix->idx.p, ix->idx_alt.p, ix->qkey.p, nq, n,
@@ -227,14 +368,9 @@ svl_status rank_loaded(svl_vector_index *ix, int32_t nq, const uint8_t *mask, in
     HIP_TRY(ix->tmp.ensure(std::max<size_t>(tmp_bytes, 1)));
     HIP_TRY(rank_sort(ix->keys.p, ix->keys_alt.p, ix->idx.p, ix->idx_alt.p, ix->qkey.p, nq, n,
                       ix->tmp.p, &tmp_bytes, &sorted, s));
-    HIP_TRY(launch_gather_hits(ix->keys.p, sorted, nq, n, ix->perm.p, offset, limit, ix->take.p,
+    HIP_TRY(launch_gather_hits(ix->keys.p, sorted, nq, n, ix->perm.p, offset, limit, ix->page.take,
                                ix->out_index.p, ix->out_score.p, s));
-    HIP_TRY(hipMemcpyAsync(out_index, ix->out_index.p, (size_t)(nq * limit) * 8,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(out_score, ix->out_score.p, (size_t)(nq * limit) * 8,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return SVL_OK;
+    return copy_page(ix, nq, limit, out_index, out_score, s);
 }
 
 svl_status check_page(int32_t nq, int64_t offset, int64_t limit, int64_t *out_index,
@@ -349,11 +485,10 @@ svl_status svl_vector_rank(svl_vector_index *ix, const float *queries, int32_t n
     hipStream_t s = ix->stream;
     if (ix->n > 0) {
         HIP_TRY(ix->Q.ensure((size_t)(nq * ix->D)));
-        HIP_TRY(ix->qnorm.ensure((size_t)nq));
         HIP_TRY(hipMemcpyAsync(ix->Q.p, queries, (size_t)(nq * ix->D) * 4, hipMemcpyHostToDevice, s));
-        HIP_TRY(hipMemcpyAsync(ix->qnorm.p, qn.data(), (size_t)nq * 8, hipMemcpyHostToDevice, s));
     }
-    return rank_loaded(ix, nq, mask, mask_stride, offset, limit, out_index, out_score, out_count, s);
+    return rank_queries(ix, ix->Q.p, qn.data(), nq, ix->D, mask, mask_stride, offset, limit,
+                        out_index, out_score, out_count, s);
 }
 
 svl_status svl_vector_rank_device(svl_vector_index *ix, const float *d_queries, int32_t nq,
@@ -372,27 +507,8 @@ svl_status svl_vector_rank_device(svl_vector_index *ix, const float *d_queries, 
     if (nq == 0) return SVL_OK;
     HIP_TRY(hipSetDevice(ix->device));
     hipStream_t s = stream ? (hipStream_t)stream : ix->stream;
-    HIP_TRY(ix->qnorm.ensure((size_t)nq));
-    HIP_TRY(ix->qflags.ensure((size_t)nq));
-    HIP_TRY(launch_query_norms(d_queries, nq, (int)query_dim, ix->qnorm.p, ix->qflags.p, s));
-    std::vector<int> flags((size_t)nq);
-    HIP_TRY(hipMemcpyAsync(flags.data(), ix->qflags.p, (size_t)nq * 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    for (int32_t q = 0; q < nq; ++q) {
-        if (flags[(size_t)q] & 1)
-            return fail(SVL_USAGE, "query %d: query embedding contains a non-finite value", q);
-        if (flags[(size_t)q] & 2)
-            return fail(SVL_USAGE,
-                        "query %d: query embedding norm is zero or non-finite; cosine similarity is undefined", q);
-        if (ix->n > 0 && query_dim != ix->D)
-            return fail(SVL_USAGE, "query %d: query embedding dimension %lld does not match the index dimension %lld",
-                        q, (long long)query_dim, (long long)ix->D);
-    }
-    if (ix->n > 0) {
-        HIP_TRY(ix->Q.ensure((size_t)(nq * ix->D)));
-        HIP_TRY(hipMemcpyAsync(ix->Q.p, d_queries, (size_t)(nq * ix->D) * 4, hipMemcpyDeviceToDevice, s));
-    }
-    return rank_loaded(ix, nq, mask, mask_stride, offset, limit, out_index, out_score, out_count, s);
+    return rank_queries(ix, d_queries, nullptr, nq, query_dim, mask, mask_stride, offset, limit,
+                        out_index, out_score, out_count, s);
 }
 
 }  // extern "C"

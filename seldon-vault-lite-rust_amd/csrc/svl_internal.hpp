@@ -364,49 +364,54 @@ hipError_t launch_log_mel(const float *x, const MelClip *clips, int n_clips, int
 // keys[q, c] = descending total-order key of dot(Q[q], V[c]) / (qnorm[q] *
 // cnorm[c]) accumulated in double in d order; all ones when mask (indexed
 // mask[q * mask_stride + perm[c]]) is given and zero.
-// Qd: scratch of D * round_up(nq, cosine_query_block(nq)) doubles.
+// Qd: the queries as launch_prepare_queries laid them out.
 int cosine_query_block(int nq);
-hipError_t launch_cosine_keys(const float *V, const double *cnorm, const float *Q,
+hipError_t launch_cosine_keys(const float *V, const double *cnorm, const double *Qd,
                               const double *qnorm, int nq, int64_t n, int D, const uint8_t *mask,
-                              int64_t mask_stride, const int64_t *perm, double *Qd,
-                              uint64_t *keys, hipStream_t s);
-// qnorm[q] = sqrt(sum Q[q, d]^2) in d order; flag bit 1: a non-finite value,
-// bit 2: a zero or non-finite norm (per query: flags[q]).
-hipError_t launch_query_norms(const float *Q, int nq, int D, double *qnorm, int *flags,
+                              int64_t mask_stride, const int64_t *perm, uint64_t *keys,
                               hipStream_t s);
+// Qd (D * round_up(nq, cosine_query_block(nq)) doubles, or null): the queries
+// in the score kernels' layout. With flags also qnorm[q] = sqrt(sum Q[q, d]^2)
+// in d order and the checks, flag bit 1: a non-finite value, bit 2: a zero or
+// non-finite norm (per query: flags[q], which may be host memory).
+hipError_t launch_prepare_queries(const float *Q, int nq, int D, double *Qd, double *qnorm,
+                                  int *flags, hipStream_t s);
 // Stable ranking of all nq * n keys by (query, key, position). With tmp ==
 // nullptr only *tmp_bytes is computed. *sorted receives the buffer (idx or
 // idx_alt) that holds the flat pair indices q * n + c in ranked order.
 hipError_t rank_sort(const uint64_t *keys, uint64_t *keys_alt, uint32_t *idx, uint32_t *idx_alt,
                      uint32_t *qkey, int nq, int64_t n, void *tmp, size_t *tmp_bytes,
                      const uint32_t **sorted, hipStream_t s);
-// Top-K selection for pages far smaller than the index: SAMPLE_COUNT samples
-// per query (every (n / SAMPLE_COUNT)-th key, n >= SAMPLE_COUNT), sorted per
-// query into sorted[q * SAMPLE_COUNT ...]; candidates are the admitted keys
-// <= sorted sample `rank`, in position order (at most cap stored per query,
-// cnt[q] counts all); the candidates sorted by (key, position); and the page
-// gathered.
+// Top-K selection for pages far smaller than the index. thresh[q] = the key of
+// rank `rank` among SAMPLE_COUNT samples of query q (every (n / SAMPLE_COUNT)-th
+// key); candidates are the admitted keys <= thresh[q], at most cap stored per
+// query. Query q's counter is cnt[q * CNT_STRIDE] (a cache line each: they are
+// counted with atomics), set to 0 here.
 constexpr int SAMPLE_COUNT = 4096;
-hipError_t sort_samples(const uint64_t *keys, int nq, int64_t n, uint64_t *sorted,
-                        hipStream_t s);
-// Only the sample of rank `rank` (into sorted[q * SAMPLE_COUNT + rank]), by
-// counting; the faster choice up to SELECT_SAMPLE_MAX_QUERIES queries.
-constexpr int SELECT_SAMPLE_MAX_QUERIES = 4;
-hipError_t select_sample(const uint64_t *keys, int nq, int64_t n, int rank, uint64_t *sorted,
-                         hipStream_t s);
-// blk_count: candidate_blocks(n) * nq counters.
+constexpr int CNT_STRIDE = 64;
+hipError_t launch_sample_threshold(const uint64_t *keys, int nq, int64_t n, int rank,
+                                   uint64_t *thresh, unsigned int *cnt, hipStream_t s);
+// Candidates in any order; the counters (zero before) count all.
+hipError_t launch_collect_candidates(const uint64_t *keys, int nq, int64_t n,
+                                     const uint64_t *thresh, int64_t cap, unsigned int *cnt,
+                                     uint64_t *cand_key, uint32_t *cand_idx, hipStream_t s);
+// Candidates in position order; the counters and found[q], which may be host
+// memory, count all. blk_count: candidate_blocks(n) * nq words.
 int candidate_blocks(int64_t n);
-hipError_t launch_compact_keys(const uint64_t *keys, int nq, int64_t n,
-                               const uint64_t *sorted_samples, int S, int rank, int64_t cap,
-                               unsigned int *blk_count, unsigned int *cnt, uint64_t *cand_key,
-                               uint32_t *cand_idx, hipStream_t s);
-// Candidates sorted on chip when every query has at most CAND_LDS of them
-// (cnt[q] <= min(cap, most), most = the longest list <= CAND_LDS), into
-// key_alt / idx_alt.
+hipError_t launch_compact_keys(const uint64_t *keys, int nq, int64_t n, const uint64_t *thresh,
+                               int64_t cap, unsigned int *blk_count, unsigned int *cnt,
+                               unsigned int *found, uint64_t *cand_key, uint32_t *cand_idx,
+                               hipStream_t s);
+// Lists of at most min(cap, CAND_LDS) candidates, in any order, sorted by
+// (key, position) on chip and the page written; found[q] = the count, and a query
+// whose list is longer, or shorter than its page, gets no entries. take, found
+// and the outputs may be host memory.
 constexpr int CAND_LDS = 8192;
-hipError_t sort_candidates_lds(const uint64_t *cand_key, const uint32_t *cand_idx,
-                               uint64_t *key_alt, uint32_t *idx_alt, const unsigned int *cnt,
-                               int nq, int64_t cap, int64_t most, hipStream_t s);
+hipError_t launch_rank_candidates(const uint64_t *cand_key, const uint32_t *cand_idx,
+                                  const unsigned int *cnt, int nq, int64_t n, int64_t cap,
+                                  const int64_t *perm, int64_t offset, int64_t limit,
+                                  const int64_t *take, unsigned int *found, int64_t *out_index,
+                                  double *out_score, hipStream_t s);
 // Stable sort of each query's candidates by key into key_alt / idx_alt.
 hipError_t sort_candidates(const uint64_t *cand_key, const uint32_t *cand_idx, uint64_t *key_alt,
                            uint32_t *idx_alt, const unsigned int *cnt, unsigned int *begin,

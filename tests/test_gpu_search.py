@@ -189,14 +189,46 @@ def test_top_k_selection_path():
         for q in range(6):
             check_query(ix, emb, ids, qs[q], got[q], mask=masks[q], offset=offset, limit=limit,
                         label=f"query {q} page ({offset}, {limit})")
-            # one query alone takes the threshold by counting instead of the
-            # sample sort of the 6-query call: the same page, bit for bit
+            # one query alone: the same page, bit for bit
             one = ix.rank(qs[q:q + 1], masks=masks[q:q + 1], offset=offset, limit=limit)[0]
             assert np.array_equal(one[0], got[q][0]), f"query {q} alone ({offset}, {limit})"
             assert np.array_equal(one[1].view(np.uint64), got[q][1].view(np.uint64))
-        # three and four queries count too, one block row per query
+        # and three and four queries
         for k in (3, 4):
             few = ix.rank(qs[:k], masks=masks[:k], offset=offset, limit=limit)
             for q in range(k):
                 assert np.array_equal(few[q][0], got[q][0]), f"{k} queries, query {q}"
                 assert np.array_equal(few[q][1].view(np.uint64), got[q][1].view(np.uint64))
+
+
+@pytest.mark.parametrize("n,offset,limit", [(70_001, 0, 10), (70_001, 390, 10), (70_001, 5, 1000),
+                                            (70_001, 0, 2150), (140_000, 8000, 700)])
+@pytest.mark.parametrize("nq,d", [(1, 36), (5, 37), (70, 36)])
+def test_candidate_lists_of_every_length(n, offset, limit, nq, d):
+    """Pages whose candidate lists take one, two, four and eight entries per
+    lane of the block that sorts them, and more than it holds; queries in HBM
+    at an address that is a multiple of 4 bytes only, padded to a block of 4,
+    8 and 128; pages above and below the size that is written into host memory."""
+    import torch
+    emb, ids = corpus(n, d, seed=n + limit)
+    ix = V.VectorIndex(emb, ids)
+    rng = np.random.default_rng(nq + limit)
+    qs = rng.standard_normal((nq, d)).astype(np.float32)
+    buf = torch.zeros(nq * d + 1, device="cuda:0")
+    buf[1:] = torch.from_numpy(qs.reshape(-1)).to("cuda:0")
+    torch.cuda.synchronize()
+    got = ix.rank_device(buf.data_ptr() + 4, nq, d, offset=offset, limit=limit)
+    host = ix.rank(qs, offset=offset, limit=limit)
+    for q in range(nq):
+        assert np.array_equal(got[q][0], host[q][0])
+        assert np.array_equal(got[q][1].view(np.uint64), host[q][1].view(np.uint64))
+    for q in {0, nq // 2, nq - 1}:
+        check_query(ix, emb, ids, qs[q], got[q], offset=offset, limit=limit, label=f"query {q}")
+    # a query that must be refused does not disturb the next call
+    buf[1 + (nq - 1) * d] = float("nan")
+    torch.cuda.synchronize()
+    with pytest.raises(S.SvlError) as e:
+        ix.rank_device(buf.data_ptr() + 4, nq, d, offset=offset, limit=limit)
+    assert e.value.kind == "Usage" and f"query {nq - 1}" in str(e.value)
+    again = ix.rank(qs, offset=offset, limit=limit)
+    assert all(np.array_equal(a[0], h[0]) for a, h in zip(again, host))
