@@ -828,9 +828,32 @@ __global__ __launch_bounds__(256) void add_kernel(const float *a, const float *b
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) y[i] = a[i] + b[i];
 }
+// 16 values a thread, four loads in flight, where x is 16-byte aligned (VEC;
+// the last n % 4 values go to the last block), one a thread otherwise. Bound
+// by the read (a linear call of 3001 x 4096 outputs: 208 us, 220 with one value
+// a thread and the flag cleared by a memset).
+template <bool VEC>
 __global__ __launch_bounds__(256) void finite_kernel(const float *x, int64_t n, int *flag) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n && !isfinite(x[i])) raise_flag(flag, FLAG_NONFINITE);
+    bool ok = true;
+    if constexpr (VEC) {
+        const int64_t n4 = n / 4, i0 = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+        f32x4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (i0 + 256 * j < n4) v[j] = reinterpret_cast<const f32x4 *>(x)[i0 + 256 * j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ok &= (bool)isfinite(v[j][r]);
+        if (blockIdx.x == gridDim.x - 1 && threadIdx.x < n % 4)
+            ok &= (bool)isfinite(x[4 * n4 + threadIdx.x]);
+    } else {
+        const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (i < n) ok = isfinite(x[i]);
+    }
+    if (!ok) raise_flag(flag, FLAG_NONFINITE);
 }
 
 static dim3 grid1d(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
@@ -852,7 +875,11 @@ hipError_t launch_add(const float *a, const float *b, float *y, int64_t n, hipSt
 }
 hipError_t launch_finite_check(const float *x, int64_t n, int *flag, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(finite_kernel, grid1d(n), dim3(256), 0, s, x, n, flag);
+    if ((uintptr_t)x % 16 == 0)
+        hipLaunchKernelGGL(finite_kernel<true>, dim3((unsigned)((n + 4095) / 4096)), dim3(256), 0,
+                           s, x, n, flag);
+    else
+        hipLaunchKernelGGL(finite_kernel<false>, grid1d(n), dim3(256), 0, s, x, n, flag);
     return hipGetLastError();
 }
 

