@@ -35,6 +35,9 @@ for p in (ROOT, os.path.join(ROOT, "seldon-vault-lite-rust_amd")):
 
 METRIC = "text embeddings/sec at batch 64×seq 512 FP32; % FP32-MFMA peak; p50 latency"
 PEAK_FP32_MFMA_TFLOPS = 157.3  # MI355X published dense FP32 matrix peak
+# The projections take an FP32 product as three F16 MFMA products (operands
+# split into pairs of halves): a third of the published dense F16 matrix peak.
+PEAK_SPLIT_TFLOPS = 2516.6 / 3
 PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFLOPS = 78.6  # MI355X published FP64 peak
 BATCH, LEN_LO, LEN_HI = 64, 64, 512
@@ -636,9 +639,11 @@ def main():
             lat.append((time.perf_counter() - a) * 1e3)
 
     traffic = gemm_traffic()
-    roofline = {"kernel": "gemm_nt_dma<64,128,16,EPI_GEGLU,4,2,2> (gate/up projection + GeGLU)",
-                "bound": "mfma", "achieved": round(gu_tflops, 3), "peak": PEAK_FP32_MFMA_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(gu_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
+    roofline = {"kernel": "gemm_split<128,128,1,EPI_GEGLU,2,2,2,2> (gate/up projection + GeGLU, FP32 "
+                          "products as three F16 MFMA products)",
+                "bound": "mfma", "achieved": round(gu_tflops, 3),
+                "peak": round(PEAK_SPLIT_TFLOPS, 1),
+                "unit": "TFLOP/s", "frac": round(gu_tflops / PEAK_SPLIT_TFLOPS, 4),
                 "traffic": traffic,
                 "flops_per_launch": gu_flops, "avg_launch_ms": round(gu_ms, 4),
                 "launches": gu["launches"]}
