@@ -169,11 +169,13 @@ svl_status svl_measure_peaks(svl_ctx *ctx, double *fp32_mfma_tflops, double *hbm
  * on every SIMD; best of three timed launches of about 12 ms each. */
 svl_status svl_measure_fp64_peak(svl_ctx *ctx, double *fp64_mfma_tflops);
 
-/* Batches of 4096 tokens or more run as `groups` groups of rows (1..4,
- * default 1), group 0 on the caller's stream and the others on streams of
- * the model that wait for it and are joined back into it, so one group's
- * kernels can fill the GPU while another's drain. groups <= 1 runs every batch
- * as one group on one stream, the fastest setting for most batches. Results are bit-identical for any setting. */
+/* Batches of 4096 tokens or more run as `groups` groups of rows (1..4), group
+ * 0 on the caller's stream and the others on streams of the model that wait
+ * for it and are joined back into it, so one group's kernels can fill the GPU
+ * while another's drain. groups <= 1 runs every batch as one group on one
+ * stream. The default is one group for models whose projections run on split
+ * operands (the fastest setting for most batches) and three for the others.
+ * Results are bit-identical for any setting. */
 svl_status svl_text_model_set_stream_split(svl_text_model *model, int groups);
 
 /* Every forward entry point (svl_text_forward_batch, svl_text_forward_device,

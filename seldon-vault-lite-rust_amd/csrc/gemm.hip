@@ -1,10 +1,9 @@
 // FP32 GEMM on CDNA4 matrix cores: C = epilogue(A[M,K] . W[N,K]^T).
 //
 // This is the reference's `linear` (src/tensor/kernels.rs:577-685,
-// out[r,c] = sum_k in[r,k] * w[c,k]) on FP32 operands: the linear entry point,
-// and the projections of models whose widths are not multiples of 32 (all
-// others run on split operands, gemm_split.hip):
-// A is the packed activation matrix (all valid tokens of the batch, row
+// out[r,c] = sum_k in[r,k] * w[c,k]) on FP32 operands: the linear entry point
+// and the projections of every model that does not run on split operands
+// (gemm_split.hip). A is the packed activation matrix (all valid tokens of the batch, row
 // major, K contiguous) and W the weight in the reference's [out, in] layout,
 // so both operands are K-contiguous and no transpose is ever materialised.
 //
@@ -30,9 +29,17 @@
 //    over k is unchanged. Every output element sees the same MFMA sequence
 //    over k whatever the tile shape, so results do not depend on the tile
 //    chosen or on a row's position in the batch.
-//  * The tile shape is chosen per launch from the grid's per-CU work (below).
+//  * The tile shape is chosen per launch from the grid's per-CU work:
+//    128x128 (3 workgroups per CU) for large grids, 128x64 or 64x64 (4 per
+//    CU) when bigger tiles would leave CUs idle or unevenly loaded, 32x32
+//    when even 64x64 tiles would not cover the GPU once.
 //  * Tiles are remapped so each XCD runs a contiguous range of the tile
-//    list, N fastest (the N tiles that share an A block hit that XCD's L2).
+//    list, N fastest (the N tiles that share an A block hit that XCD's L2);
+//    launches of 128 M blocks or more with the whole GPU (32 or more when
+//    the launch shares the GPU with other streams) order the range in
+//    groups of 8 M blocks, M fastest within an N block and the N blocks of
+//    every second group in reverse, so the tiles in flight on an XCD share a
+//    few A blocks and W panels.
 //  * Epilogues fuse the elementwise op that follows each projection in
 //    text.rs (PLE scale, GeGLU, GELU-gate x per-layer input).
 #include <algorithm>
@@ -362,10 +369,21 @@ __global__ __launch_bounds__(256, MINB) void gemm_nt_mfma(GemmArgs p, int tiles_
     gemm_epilogue<S::TM, S::TN, EPI>(p, acc, m0 + wm * S::WM, n0 + wn * S::WN, l16, g, seg);
 }
 
+// M blocks per rasterization group of the DMA kernel's tile order, and the
+// fewest M blocks of a launch that takes the grouped order: 128 for a launch
+// with the whole GPU (below that the 1 x 128-token forward went from 2.00 to
+// 2.04 ms and the audio tower lost 1 % with it; the T2 launches kept their
+// time and fetched 2.6x less), 32 for one that shares the GPU with other
+// streams (the T2 row groups, about 98 M blocks each: 1695-1696 against
+// 1680-1690 embeddings/s, and the image tower 29.31-29.37 against
+// 29.48-29.64 ms; 16 and 64 measured the same as 32).
+constexpr int RASTER_M = 8, RASTER_MIN_TILES_M = 128, RASTER_MIN_TILES_M_SHARED = 32;
+
 // Direct-to-LDS variant; requires K % BK == 0 and 16-byte aligned rows. NS
 // LDS stages: NS - 1 slices are in flight while one is consumed. WMW waves
 // along M, 4 / WMW along N.
-template <int BM, int BN, int BK, int EPI, int MINB, int NS, int WMW, bool CONV = false>
+template <int BM, int BN, int BK, int EPI, int MINB, int NS, int WMW, bool CONV = false,
+          bool RASTER = false>
 __global__ __launch_bounds__(256, MINB) void gemm_nt_dma(GemmArgs p, int tiles_m, int tiles_n) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int WNW = 4 / WMW;                // waves along N
@@ -417,8 +435,23 @@ __global__ __launch_bounds__(256, MINB) void gemm_nt_dma(GemmArgs p, int tiles_m
     const int xcd = bid & 7, local = bid >> 3;
     const int q8 = ntiles >> 3, r8 = ntiles & 7;
     const int tile = xcd * q8 + min(xcd, r8) + local;
-    const int tm = uniform(tile / tiles_n);
-    const int tn = tile - tm * tiles_n;
+    int tm, tn;
+    if constexpr (RASTER) {
+        // Within that range, groups of RASTER_M M blocks run N block by N
+        // block, M fastest: the tiles in flight together on an XCD then share
+        // a few W panels and A blocks in its L2 (the T2 gate/up launch fetched
+        // 188 against 491 MiB with N fastest, at the same speed). Odd groups
+        // run the N blocks in reverse, so a group starts on the W panels the
+        // one before it ended on (the same launch fetched 187 against 217 MiB,
+        // at the same speed).
+        const int gsize = RASTER_M * tiles_n, grp = tile / gsize, first = grp * RASTER_M;
+        const int gm = min(RASTER_M, tiles_m - first), in = tile - grp * gsize;
+        tm = uniform(first + in % gm);
+        tn = uniform(grp & 1 ? tiles_n - 1 - in / gm : in / gm);
+    } else {
+        tm = uniform(tile / tiles_n);
+        tn = tile - tm * tiles_n;
+    }
     const int m0 = tm * BM, n0 = tn * BN;
     // The wave index through v_readfirstlane: the LDS destinations of the
     // DMA instructions (M0) then come from scalar registers, set by one
@@ -740,18 +773,53 @@ __global__ __launch_bounds__(256) void gemm_nt_simple(GemmArgs p) {
 template <int BM, int BN, int BK, int EPI, int MINB, int NS, int WMW = 2, bool CONV = false>
 static hipError_t launch_dma(const GemmArgs &a, hipStream_t s) {
     const int tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
+    if constexpr (!CONV) {
+        if (tm >= (a.cus > 0 ? RASTER_MIN_TILES_M_SHARED : RASTER_MIN_TILES_M)) {
+            hipLaunchKernelGGL((gemm_nt_dma<BM, BN, BK, EPI, MINB, NS, WMW, false, true>),
+                               dim3(tm * tn), dim3(256), 0, s, a, tm, tn);
+            return hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL((gemm_nt_dma<BM, BN, BK, EPI, MINB, NS, WMW, CONV>), dim3(tm * tn),
                        dim3(256), 0, s, a, tm, tn);
     return hipGetLastError();
 }
 
-// Grids of at least two workgroups per CU keep two stages (their co-resident
-// workgroups hide each other's DMA latency, and a deeper pipeline measured
-// slower there); short grids, whose few workgroups run the K loop alone, take
-// as many stages as the LDS budget allows. Grids that do not fill the GPU once
-// also take 64-wide K slices, so each barrier is amortised over four times more
-// MFMAs (the k order, set by the 16-k groups, is the same for any slice
-// width).
+// Tile choice.
+//  * A launch with the whole GPU: workgroups are spread round-robin over the
+//    256 CUs, so it takes about ceil(tiles / 256) tile-times on its busiest
+//    CU; the cost of a tile shape is that count times the tile's MAC count
+//    over the shape's measured efficiency (128x128 at 3 per CU and 64x64 at
+//    4 per CU: 1.0; 128x64 at 4 per CU: 0.95; 64x32 at 4 per CU: 0.93),
+//    ties going to the larger tile (the audio tower's M = 3000 x 4096
+//    projection: 250 us at 128x128, 275 us at 64x64). With 16x16 fragments
+//    64x64 tiles keep up with larger ones (the 18688-token O projection:
+//    168 us against 202 us for 128x64 tiles), and their finer grid wastes
+//    less of the last round.
+//  * A launch that shares the GPU with other streams (a.cus > 0, the text
+//    path's row groups): 64x64 (O and down per group: 65 and 93 us against
+//    75 and 110 us for 128x64); the other streams' work fills the partial
+//    rounds that the cost model above optimises for.
+//  * Grids that 64x64 tiles would not cover once (one short row, 128 tokens:
+//    QKV at 6.9 us against 15.9 us for 64x64 tiles): 32x32 tiles, one 16x16
+//    block per wave; paired epilogues 32x64 tiles whose two wave columns
+//    hold the x and y halves of the pair block (two 16x16 blocks per wave),
+//    joined through LDS for the epilogue.
+//  * Otherwise paired epilogues keep the 32 + 32 columns of a pair in one
+//    wave: 64x128 tiles (4 per CU; the 18688-token gate/up: 481 us against
+//    502 us for 128x128), for the row groups too, with deeper pipelines below
+//    two rounds of 128x128 tiles.
+//  * Outputs of at most 32 columns (the audio subsampling's 32 channels):
+//    128x32 tiles, the four waves stacked along M, instead of 64x64 tiles
+//    that would spend half their MFMAs on zero columns.
+//  * Stages: grids of at least two workgroups per CU keep two stages (their
+//    co-resident workgroups hide each other's DMA latency, and a deeper
+//    pipeline measured slower there); short grids, whose few workgroups run
+//    the K loop alone, take as many stages as the LDS budget allows.
+//    Grids that do not fill the GPU once (fewer tiles than CUs) also take
+//    64-wide K slices, so each barrier is amortised over four times more
+//    MFMAs (the k order, set by the 16-k groups, is the same for any slice
+//    width).
 template <int BM, int BN, int BK, int EPI, int MINB, int NS_DEEP>
 static hipError_t launch_dma_staged(const GemmArgs &a, hipStream_t s) {
     // workgroups per CU that the deep pipeline's LDS allows (160 KB per CU)
@@ -764,64 +832,96 @@ static hipError_t launch_dma_staged(const GemmArgs &a, hipStream_t s) {
     return launch_dma<BM, BN, BK, EPI, MINB, 2>(a, s);
 }
 
-// Tile choice for plain products (the linear entry point, and models whose
-// widths keep them off the split operands):
-//  * Grids that 64x64 tiles would not cover once (a few short rows): 32x32
-//    tiles, one 16x16 block per wave, so each wave's MFMA chain is K / 4
-//    instructions long, with wide K slices (fewer DMA round trips and barriers
-//    on a chain that is mostly memory latency): 256-wide slices in one
-//    workgroup per CU (128 x 768 x 768: 7.0 us, against 7.6 us for 64-wide),
-//    64-wide slices in three where the grid passes one round (1040 x 768 x
-//    768: 15.7 against 20.8 us).
-//  * Outputs of at most 32 columns: 128x32 tiles, the four waves stacked along
-//    M, instead of 64x64 tiles that would spend half their MFMAs on zero
-//    columns.
-//  * Otherwise the least work on the busiest CU: ceil(tiles / 256) times the
-//    tile's MACs over the shape's measured efficiency (128x128 at 3 per CU,
-//    its count rounded up to whole rounds of three, and 64x64 at 4 per CU: 1.0;
-//    128x64: 0.95; 64x32: 0.93), ties to the larger (3000 x 4096 x 1024: 250
-//    us at 128x128, 275 us at 64x64; 3000 x 768 x 1536: 63.7 us at 64x32, 70.9
-//    us at 64x64).
-static hipError_t launch_dma_store(const GemmArgs &a, hipStream_t s) {
-    constexpr int EPI = EPI_STORE;
+template <int EPI>
+static hipError_t launch_dma_auto(const GemmArgs &a, hipStream_t s) {
     auto tiles = [&](int bm, int bn) {
         return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
     };
-    if (tiles(64, 64) < 256 && a.K % 32 == 0) {
-        if (tiles(32, 32) <= 256) {
-            if (a.K % 256 == 0) return launch_dma<32, 32, 256, EPI, 1, 2>(a, s);
-            if (a.K % 128 == 0) return launch_dma<32, 32, 128, EPI, 1, 2>(a, s);
-        }
-        if (a.K % 64 == 0) return launch_dma<32, 32, 64, EPI, 1, 3>(a, s);
-        return launch_dma<32, 32, 32, EPI, 1, 4>(a, s);
-    }
-    if (a.N <= 32 && a.K % 32 == 0) return launch_dma<128, 32, 32, EPI, 4, 2, 4>(a, s);
-    auto per_cu = [&](int bm, int bn) { return (double)((tiles(bm, bn) + 255) / 256); };
-    const double c128 = std::ceil(per_cu(128, 128) / 3.0) * 3.0 * (128.0 * 128.0);
-    const double c12864 = per_cu(128, 64) * (128.0 * 64.0) / 0.95;
-    const double c64 = per_cu(64, 64) * (64.0 * 64.0);
-    const double c6432 = a.K % 32 == 0 ? per_cu(64, 32) * (64.0 * 32.0) / 0.93 : 1e300;
-    if (c6432 < c64 && c6432 < c128 && c6432 < c12864) return launch_dma<64, 32, 32, EPI, 4, 2, 2>(a, s);
-    if (c64 < c128 && c64 < c12864) {
-        if (a.K % 32 == 0) return launch_dma_staged<64, 64, 32, EPI, 4, 3>(a, s);
-        return launch_dma_staged<64, 64, 16, EPI, 4, 4>(a, s);
-    }
-    if (c12864 < c128) return launch_dma_staged<128, 64, 16, EPI, 4, 3>(a, s);
-    return launch_dma_staged<128, 128, 16, EPI, 3, 3>(a, s);
-}
-
-// The other epilogues run here only in models whose widths are not multiples
-// of 32 (every other model's projections are split): one tile shape per grid
-// size.
-template <int EPI>
-static hipError_t launch_dma_fused(const GemmArgs &a, hipStream_t s) {
-    const int64_t t64 = (int64_t)((a.M + 63) / 64) * ((a.N + 63) / 64);
+    // Grids that 64x64 tiles would not cover once (a few short rows): the
+    // smallest tiles, one 16x16 block per wave (paired: two, the x or the y
+    // half of the pair), so each wave's MFMA chain is K / 4 (2 x K / 4)
+    // instructions long.
+    const bool tiny = tiles(64, 64) < 256 && a.K % 32 == 0;
     if constexpr (paired_epi<EPI>()) {
-        if (t64 < 256 && a.K % 32 == 0) return launch_dma<32, 64, 32, EPI, 1, 4, 2>(a, s);
+        if (tiny && tiles(32, 64) <= 256) {
+            // 32x64 tiles: the x and y halves of each pair on two waves, so a
+            // wave's chain is 2 x K / 4 MFMAs (gate/up at 128 tokens: 12.1 us
+            // against 17.6 us for 64x64 tiles with one 16x64 block per wave;
+            // three or four stages measured no faster). They fill the GPU
+            // once at one workgroup per CU; larger grids take the rules below
+            // (gate/up at 256 tokens 17.2 against 20.0 us).
+            if (a.K % 128 == 0) return launch_dma<32, 64, 128, EPI, 1, 2, 2>(a, s);
+            if (a.K % 64 == 0) return launch_dma<32, 64, 64, EPI, 1, 3, 2>(a, s);
+            return launch_dma<32, 64, 32, EPI, 1, 4, 2>(a, s);
+        }
+        // concurrent row groups: 64x128x16 tiles at four per CU, as for the
+        // whole batch (the T2 step 37.57-37.64 against 37.98-38.04 ms with
+        // 128x128x16 tiles at three per CU, which had led before the DMA
+        // issue moved behind the MFMAs; same box)
+        if (a.cus > 0 && a.K % 16 == 0) return launch_dma<64, 128, 16, EPI, 4, 2>(a, s);
+        if (tiles(128, 128) < 2 * 256) {
+            // grids of a few thousand rows: tiles small enough to spread over
+            // every CU (gate/up at 1040 / 2000 / 3016 rows: 34.7 / 63.8 / 88.0
+            // us against 53.9 / 76.6 / 104.2 us for 64x128 tiles)
+            if (a.K % 32 == 0) {
+                if (tiles(64, 64) < 1280) return launch_dma<32, 64, 32, EPI, 4, 2, 2>(a, s);
+                return launch_dma<64, 64, 32, EPI, 4, 2, 4>(a, s);
+            }
+            return launch_dma<64, 128, 16, EPI, 3, 4>(a, s);
+        }
         return launch_dma<64, 128, 16, EPI, 4, 2>(a, s);
     } else {
-        if (t64 < 256 && a.K % 32 == 0) return launch_dma<32, 32, 32, EPI, 1, 4>(a, s);
-        return launch_dma<64, 64, 16, EPI, 4, 2>(a, s);
+        if (tiny) {
+            // Wide K slices: fewer DMA round trips and barriers on a chain
+            // that is mostly memory latency. 256-wide slices (two 64 KB
+            // stages) took the 1 x 128-token forward from 1.837 to 1.811 ms
+            // against 128-wide ones; 128-wide took O at 128 tokens from 7.6
+            // to 7.0 us against 64-wide. Those hold one workgroup per CU, so
+            // they serve grids of one round; larger ones take 64-wide slices
+            // in three stages, three workgroups per CU (at 1040 tokens the
+            // N = 768 projections 15.7 against 20.8 us, the PLE gate 9.1
+            // against 11.3 us; at 520 tokens QKV 12.8 against 16.7 us).
+            if (tiles(32, 32) <= 256) {
+                if (a.K % 256 == 0) return launch_dma<32, 32, 256, EPI, 1, 2>(a, s);
+                if (a.K % 128 == 0) return launch_dma<32, 32, 128, EPI, 1, 2>(a, s);
+            }
+            if (a.K % 64 == 0) return launch_dma<32, 32, 64, EPI, 1, 3>(a, s);
+            return launch_dma<32, 32, 32, EPI, 1, 4>(a, s);
+        }
+        // The PLE gate (N = 256, K = 768, GELU x per-layer input): 64x32 tiles
+        // at six per CU, whole batch or row group (T2 whole batch 68 against
+        // 76 us for 64x64 tiles; three row groups together 62 against 66-73 us)
+        if constexpr (EPI == EPI_GELU_MUL)
+            if (a.K % 32 == 0) return launch_dma<64, 32, 32, EPI, 6, 2, 2>(a, s);
+        if (a.cus > 0) {
+            if (a.K % 32 == 0) return launch_dma<64, 64, 32, EPI, 4, 2>(a, s);
+            if (tiles(128, 128) < 4 * 256) return launch_dma_staged<128, 64, 16, EPI, 4, 3>(a, s);
+            return launch_dma_staged<128, 128, 16, EPI, 3, 3>(a, s);
+        }
+        if (a.N <= 32 && a.K % 32 == 0) return launch_dma<128, 32, 32, EPI, 4, 2, 4>(a, s);
+        // The least work on the busiest CU, over the shape's efficiency. 64x32
+        // tiles (one or two accumulator blocks per wave) run at 0.93 of 64x64
+        // ones, and their finer grid evens out grids of a few thousand rows: at
+        // 3000 rows N = 768 (K = 1536) took 63.7 against 70.9 us for 64x64
+        // tiles (564 of them leave CUs with two or three) and N = 1536 74.6
+        // against 79.4 us, while N = 1024 (752 64x64 tiles, three per CU)
+        // took 190.6 against 205.8 us at K = 4096 on 64x64 tiles.
+        auto per_cu = [&](int bm, int bn) { return (double)((tiles(bm, bn) + 255) / 256); };
+        // 128x128 tiles run three at a time per CU, and a CU's last round
+        // holds its remainder: their count is rounded up to whole rounds (the
+        // 16384-row QKV, five per CU: 268 us against 230 us for 64x64 tiles;
+        // the 3016-row QKV, one per CU: 52.6 against 49.0 us)
+        const double c128 = std::ceil(per_cu(128, 128) / 3.0) * 3.0 * (128.0 * 128.0);
+        const double c12864 = per_cu(128, 64) * (128.0 * 64.0) / 0.95;
+        const double c64 = per_cu(64, 64) * (64.0 * 64.0);
+        const double c6432 = a.K % 32 == 0 ? per_cu(64, 32) * (64.0 * 32.0) / 0.93 : 1e300;
+        if (c6432 < c64 && c6432 < c128 && c6432 < c12864) return launch_dma<64, 32, 32, EPI, 4, 2, 2>(a, s);
+        if (c64 < c128 && c64 < c12864) {
+            if (a.K % 32 == 0) return launch_dma_staged<64, 64, 32, EPI, 4, 3>(a, s);
+            return launch_dma_staged<64, 64, 16, EPI, 4, 4>(a, s);
+        }
+        if (c12864 < c128) return launch_dma_staged<128, 64, 16, EPI, 4, 3>(a, s);
+        return launch_dma_staged<128, 128, 16, EPI, 3, 3>(a, s);
     }
 }
 
@@ -852,14 +952,14 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t s) {
     const bool dma_ok = a.K % 16 == 0 && (int64_t)128 * std::max(a.lda, a.ldw) * 4 < INT32_MAX;
     if (dma_ok) {
         switch (a.epi) {
-            case EPI_STORE: return launch_dma_store(a, s);
-            case EPI_SCALE: return launch_dma_fused<EPI_SCALE>(a, s);
-            case EPI_GEGLU: return launch_dma_fused<EPI_GEGLU>(a, s);
-            case EPI_GELU_MUL: return launch_dma_fused<EPI_GELU_MUL>(a, s);
-            case EPI_BIAS: return launch_dma_fused<EPI_BIAS>(a, s);
-            case EPI_CLIP_STORE: return launch_dma_fused<EPI_CLIP_STORE>(a, s);
-            case EPI_CLIP_SILU: return launch_dma_fused<EPI_CLIP_SILU>(a, s);
-            case EPI_CLIP_GLU: return launch_dma_fused<EPI_CLIP_GLU>(a, s);
+            case EPI_STORE: return launch_dma_auto<EPI_STORE>(a, s);
+            case EPI_SCALE: return launch_dma_auto<EPI_SCALE>(a, s);
+            case EPI_GEGLU: return launch_dma_auto<EPI_GEGLU>(a, s);
+            case EPI_GELU_MUL: return launch_dma_auto<EPI_GELU_MUL>(a, s);
+            case EPI_BIAS: return launch_dma_auto<EPI_BIAS>(a, s);
+            case EPI_CLIP_STORE: return launch_dma_auto<EPI_CLIP_STORE>(a, s);
+            case EPI_CLIP_SILU: return launch_dma_auto<EPI_CLIP_SILU>(a, s);
+            case EPI_CLIP_GLU: return launch_dma_auto<EPI_CLIP_GLU>(a, s);
         }
         return hipErrorInvalidValue;
     }

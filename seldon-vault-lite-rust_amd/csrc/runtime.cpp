@@ -121,7 +121,7 @@ struct svl_text_model {
     static constexpr int MAX_GROUPS = 4;
     hipStream_t extra[MAX_GROUPS - 1] = {};  // streams of row groups 1..3
     hipEvent_t ev_fork = nullptr, ev_join[MAX_GROUPS - 1] = {};
-    int row_groups = 1;                      // row groups per large batch
+    int row_groups = 0;                      // row groups per large batch (0: the default)
     int64_t pass_tokens = 0;                 // tokens per pass (0: from PASS_BYTES)
     std::mutex mu;
 
@@ -527,6 +527,8 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     int32_t *pos = m->pos.p + t0, *rowlen = m->rowlen.p + t0;
     const int64_t *offs = m->offsets.p + grp.off_slot;
     const int64_t T_all = b.hidden_stride > 0 ? b.hidden_stride : b.T;
+    // CUs each launch can expect while the batch's groups run side by side
+    const int cus = b.groups.size() > 1 ? (int)(256 / b.groups.size()) : 0;
     // split models: the split copy of h that the PLE projections read
     const SplitRows hs = m->split ? SplitRows{attn, m->rs.p + t0} : SplitRows();
     const float *h_in = m->split ? attn : h, *h_rs = hs.descale;
@@ -548,6 +550,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         // (the split descale carries ple_scale)
         GemmArgs g{h_in, H, m->ple_model, H, ple, L * P, (int)T, (int)(L * P), (int)H,
                    m->split ? EPI_STORE : EPI_SCALE, m->ple_scale, nullptr, 0, 0};
+        g.cus = cus;
         g.wd = m->d_ple_model;
         g.rs = h_rs;
         Timer tm(m, s, KC_GEMM_PLE_MODEL, 2.0 * Td * H * L * P);
@@ -564,6 +567,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{n, H, ly.w_qkv, H, qkv, ldqkv, (int)T, (int)ldqkv, (int)H, EPI_STORE, 1.f,
                        nullptr, 0, 0};
+            g.cus = cus;
             g.wd = ly.d_qkv;
             Timer tm(m, s, KC_GEMM_QKV, 2.0 * Td * H * ldqkv);
             HIP_TRY(launch_gemm(g, s));
@@ -611,6 +615,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{attn, qd, ly.w_o, qd, tmp, H, (int)T, (int)H, (int)qd, EPI_STORE, 1.f,
                        nullptr, 0, 0};
+            g.cus = cus;
             g.wd = ly.d_o;
             Timer tm(m, s, KC_GEMM_O, 2.0 * Td * qd * H);
             HIP_TRY(launch_gemm(g, s));
@@ -623,6 +628,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{n, H, ly.w_gu, H, act, m->I, (int)T, (int)(2 * m->I_pad), (int)H, EPI_GEGLU,
                        1.f, nullptr, 0, (int)m->I};
+            g.cus = cus;
             g.wd = ly.d_gu;
             g.out_scale = ly.s_act;
             Timer tm(m, s, KC_GEMM_GATE_UP, 2.0 * Td * H * 2 * m->I);
@@ -631,6 +637,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{act, m->I, ly.w_down, m->I, tmp, H, (int)T, (int)H, (int)m->I, EPI_STORE,
                        1.f, nullptr, 0, 0};
+            g.cus = cus;
             g.wd = ly.d_down;
             Timer tm(m, s, KC_GEMM_DOWN, 2.0 * Td * m->I * H);
             HIP_TRY(launch_gemm(g, s));
@@ -643,6 +650,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{h_in, H, ly.w_pg, H, pg, P, (int)T, (int)P, (int)H, EPI_GELU_MUL, 1.f,
                        ple + l * P, L * P, 0};
+            g.cus = cus;
             g.wd = ly.d_pg;
             g.rs = h_rs;
             g.out_scale = ly.s_pg;
@@ -652,6 +660,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             GemmArgs g{pg, P, ly.w_pp, P, tmp, H, (int)T, (int)H, (int)P, EPI_STORE, 1.f, nullptr,
                        0, 0};
+            g.cus = cus;
             g.wd = ly.d_pp;
             g.rs = h_rs;
             Timer tm(m, s, KC_GEMM_PLE_PROJ, 2.0 * Td * P * H);
@@ -673,6 +682,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     {
         GemmArgs g{n, H, m->out_proj, H, proj, E, (int)T, (int)E, (int)H, EPI_STORE, 1.f, nullptr,
                    0, 0};
+        g.cus = cus;
         g.wd = m->d_out_proj;
         Timer tm(m, s, KC_GEMM_OUT, 2.0 * Td * H * E);
         HIP_TRY(launch_gemm(g, s));
@@ -773,7 +783,7 @@ svl_status prepare_batch(svl_text_model *m, const int64_t *offsets, int32_t r0, 
     for (int32_t r = r0; r <= r1; ++r) b.offsets[(size_t)(r - r0)] = offsets[r] - offsets[r0];
     b.T = b.offsets.back();
     if (b.T > (int64_t)INT32_MAX / 8) return fail(SVL_LIMIT, "batch holds too many tokens");
-    build_groups(m, b, m->row_groups);
+    build_groups(m, b, m->row_groups > 0 ? m->row_groups : m->split ? 1 : 3);
     return SVL_OK;
 }
 

@@ -47,6 +47,7 @@ struct GemmArgs {
     const float *aux;
     int64_t ldaux;
     int n_out;  // EPI_GEGLU / EPI_CLIP_GLU: number of real output columns
+    int cus = 0;               // > 0: the launch shares the GPU with other streams
     int clip_cols = 0;         // output columns per clip segment (0: one segment)
     float clip[4][4] = {};     // per segment: input min, input max, output min, output max
     int64_t a_seg = 0;         // floats from one clip segment's A operand to the next's

@@ -455,6 +455,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
     if (R <= 0) return SVL_OK;
     int *flag = v->flag.p;
     const int64_t ldqkv = v->qd + 2 * v->kd;
+    const int cus = b.groups.size() > 1 ? (int)(256 / b.groups.size()) : 0;
     // attention on split head rows; its windows span one image
     int64_t longest = 0;
     for (size_t i = 0; i + 1 < b.offsets.size(); ++i)
@@ -467,6 +468,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         {
             GemmArgs ga{n, H, ly.w_qkv, H, qkv, ldqkv, (int)R, (int)ldqkv, (int)H, EPI_STORE, 1.f,
                         nullptr, 0, 0};
+            ga.cus = cus;
             ga.wd = ly.d_qkv;
             HIP_TRY(launch_gemm(ga, s));
         }
@@ -504,6 +506,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         {
             GemmArgs ga{attn, v->qd, ly.w_o, v->qd, tmp, H, (int)R, (int)H, (int)v->qd, EPI_STORE,
                         1.f, nullptr, 0, 0};
+            ga.cus = cus;
             ga.wd = ly.d_o;
             HIP_TRY(launch_gemm(ga, s));
         }
@@ -512,6 +515,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         {
             GemmArgs ga{n, H, ly.w_gu, H, act, v->I, (int)R, (int)(2 * v->I_pad), (int)H, EPI_GEGLU,
                         1.f, nullptr, 0, (int)v->I};
+            ga.cus = cus;
             ga.wd = ly.d_gu;
             ga.out_scale = ly.s_act;
             HIP_TRY(launch_gemm(ga, s));
@@ -519,6 +523,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         {
             GemmArgs ga{act, v->I, ly.w_down, v->I, tmp, H, (int)R, (int)H, (int)v->I, EPI_STORE,
                         1.f, nullptr, 0, 0};
+            ga.cus = cus;
             ga.wd = ly.d_down;
             HIP_TRY(launch_gemm(ga, s));
         }

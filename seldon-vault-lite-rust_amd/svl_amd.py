@@ -594,7 +594,7 @@ class TextModel:
         _check(lib().svl_text_model_create(self.device.handle, ctypes.byref(cfg), arr, n,
                                            ctypes.byref(h)))
         self.handle = h
-        self.row_groups = 1   # the library's default: large batches are not split
+        self.row_groups = 0   # 0: the library's default
 
     @classmethod
     def load(cls, model_dir: str, device: Device | None = None) -> "TextModel":
@@ -705,7 +705,8 @@ class TextModel:
 
     def set_stream_split(self, groups):
         """Row groups (1..4, each on its own stream) for batches of 4096+
-        tokens; True = 3, False = 1 (the default)."""
+        tokens; True = 3, False = 1. The default is one for models on split
+        operands, three for the others."""
         g = 3 if groups is True else (1 if groups is False else int(groups))
         _check(lib().svl_text_model_set_stream_split(self.handle, g))
         self.row_groups = max(1, min(g, 4))
