@@ -62,11 +62,6 @@ struct AuLayer {
           *lc_norm = nullptr;
     Bounds bstart = {}, bend = {};
     float *norm_pre_attn = nullptr, *norm_post_attn = nullptr, *norm_out = nullptr;
-    // split towers: descale of each projection's outputs, and the scales of
-    // its split operand (indexed by feed-forward, by Q / K / V)
-    float *d_w1[2] = {}, *d_w2[2] = {}, *d_qkv = nullptr, *d_post = nullptr, *d_start = nullptr,
-          *d_end = nullptr;
-    float s_up[2] = {}, s_down[2] = {}, s_qkv[3] = {}, s_post = 0.f, s_start = 0.f, s_end = 0.f;
 };
 
 // Typed view into the model's metadata block (set by upload_au_meta).
@@ -85,13 +80,6 @@ struct svl_audio_model {
     std::vector<float *> allocations;
     float *w_conv0 = nullptr, *ln0 = nullptr, *w_conv1 = nullptr, *ln1 = nullptr,
           *w_in = nullptr, *w_out = nullptr, *b_out = nullptr, *w_emb = nullptr;
-    // Every projection and the layer-1 convolution run on split operands
-    // (gemm_split.hip): 128 layer-0 and 32 or 64 layer-1 channels, a hidden size
-    // that is a multiple of 128 (the Q/K/V segments are whole tiles) and an
-    // output projection that is one of 32. Other towers take the FP32 GEMMs.
-    bool split = false;
-    float *d_conv1 = nullptr, *d_in = nullptr, *d_out = nullptr, *d_emb = nullptr;
-    float s_l0 = 0.f, s_l1 = 0.f, s_out = 0.f, s_emb = 0.f;
     std::vector<AuLayer> layers;
     // workspace
     DevBuf<float> mel, l0, l1, h, n, tmp, act, qkv, att, gated, proj, projn, soft;
@@ -262,62 +250,35 @@ std::vector<float> position_table(int64_t hidden, int64_t positions) {
 
 // A clipped linear (audio.rs:558-601). Its A operand is written already
 // clamped to b's input bounds by the kernel that produces it (in_clamp).
-GemmArgs clipped(const float *A, int64_t lda, const float *W, const float *descale, int64_t ldw,
-                 float *C, int64_t ldc, int64_t M, int64_t N, int64_t K, int epi, const Bounds &b) {
+GemmArgs clipped(const float *A, int64_t lda, const float *W, int64_t ldw, float *C, int64_t ldc,
+                 int64_t M, int64_t N, int64_t K, int epi, const Bounds &b) {
     GemmArgs g{A, lda, W, ldw, C, ldc, (int)M, (int)N, (int)K, epi, 1.f, nullptr, 0, 0};
-    g.wd = descale;
     for (int k = 0; k < 4; ++k) g.clip[0][k] = b.v[k];
     return g;
 }
 
 // Store clamp that makes a row kernel's output the A operand of the clipped
-// linears with input bounds b[0 .. n-1] (one copy each, `stride` floats apart),
-// split and scaled by scale[0 .. n-1] where that is positive.
-OutClamp in_clamp(const Bounds *const *b, const float *scale, int n, int64_t stride) {
+// linears with input bounds b[0 .. n-1] (one copy each, `stride` floats apart).
+OutClamp in_clamp(const Bounds *const *b, int n, int64_t stride) {
     OutClamp oc;
     oc.copies = n;
     oc.stride = stride;
     for (int k = 0; k < n; ++k) {
         oc.lo[k] = b[k]->v[0];
         oc.hi[k] = b[k]->v[1];
-        oc.scale[k] = scale[k];
     }
     return oc;
 }
 
-OutClamp in_clamp(const Bounds &b, float scale) {
+OutClamp in_clamp(const Bounds &b) {
     const Bounds *p = &b;
-    return in_clamp(&p, &scale, 1, 0);
-}
-
-// Largest magnitude of clamp(x, lo, hi) for |x| <= bound: the clamp only
-// shrinks values when zero lies between its bounds.
-double clamp_bound(double bound, float lo, float hi) {
-    const double most = std::max(std::fabs((double)lo), std::fabs((double)hi));
-    return lo <= 0.f && hi >= 0.f ? std::min(bound, most) : most;
-}
-
-// Largest magnitude of a clipped linear's outputs over inputs clamp(x, in)
-// with x = RMSNorm(.) * norm of width K, for its uploaded FP32 weight.
-svl_status clipped_bound(const float *w, int64_t rows, int64_t K, const float *norm,
-                         const Bounds &b, float *scratch, double *out) {
-    std::vector<float> each;
-    ST_TRY(product_bounds(w, rows, K, nullptr, scratch, each));
-    double bound = largest(each) * std::max(std::fabs((double)b.v[0]), std::fabs((double)b.v[1]));
-    if (b.v[0] <= 0.f && b.v[1] >= 0.f) {  // the clamp only shrinks
-        ST_TRY(product_bounds(w, rows, K, norm, scratch, each));
-        bound = std::min(bound, largest(each));
-    }
-    *out = clamp_bound(bound, b.v[2], b.v[3]);
-    return SVL_OK;
+    return in_clamp(&p, 1, 0);
 }
 
 // The FFN up projection's SiLU output is the down projection's A operand.
-GemmArgs ffn_up(const float *A, int64_t lda, const float *W, const float *descale, float *C,
-                int64_t M, int64_t N, int64_t K, const Bounds &up, const Bounds &down,
-                float out_scale) {
-    GemmArgs g = clipped(A, lda, W, descale, K, C, N, M, N, K, EPI_CLIP_SILU, up);
-    g.out_scale = out_scale;
+GemmArgs ffn_up(const float *A, int64_t lda, const float *W, float *C, int64_t M, int64_t N,
+                int64_t K, const Bounds &up, const Bounds &down) {
+    GemmArgs g = clipped(A, lda, W, K, C, N, M, N, K, EPI_CLIP_SILU, up);
     g.post_lo = down.v[0];
     g.post_hi = down.v[1];
     return g;
@@ -513,7 +474,7 @@ svl_status enqueue_audio(svl_audio_model *m, const AuBatch &b, const float *d_me
     HIP_TRY(launch_positions(m->offsets.p, b.B, m->pos.p, m->rowlen.p, s));
     // Subsampling (audio.rs:1136-1255).
     HIP_TRY(launch_sscp_conv0(d_mel, m->mask.p, m->rows0.p, b.T0, m->w_conv0, m->ln0, (int)m->C0,
-                              m->eps, m->l0.p, flag, s, m->s_l0));
+                              m->eps, m->l0.p, flag, s));
     // layer 1: the 3x3 stride-2 convolution as an implicit-im2col GEMM against
     // the tap-major [C1, 9 C0] weight, then LayerNorm + ReLU. C0 is 128 in
     // every configuration that reaches this point (prepare_clips), and a pass
@@ -523,7 +484,6 @@ svl_status enqueue_audio(svl_audio_model *m, const AuBatch &b, const float *d_me
         const int64_t K = 9 * m->C0;
         GemmArgs g{m->l0.p, K, m->w_conv1, K, m->l1.p, m->C1, (int)(T * FREQ1), (int)m->C1,
                    (int)K, EPI_STORE, 1.f, nullptr, 0, 0};
-        g.wd = m->d_conv1;
         g.conv_rows = reinterpret_cast<const int32_t *>(m->rows1.p);
         g.conv_mask = m->mask0.p;
         g.conv_c0 = (int)m->C0;
@@ -533,12 +493,11 @@ svl_status enqueue_audio(svl_audio_model *m, const AuBatch &b, const float *d_me
         if (!gemm_conv_ok(g)) return fail(SVL_INTERNAL, "audio subsampling launch out of bounds");
         HIP_TRY(launch_gemm_conv(g, s));
     }
-    HIP_TRY(launch_sscp_ln_relu(m->l1.p, m->ln1, (int)m->C1, T * FREQ1, m->eps, flag, s, m->s_l1));
+    HIP_TRY(launch_sscp_ln_relu(m->l1.p, m->ln1, (int)m->C1, T * FREQ1, m->eps, flag, s));
     {
         const int64_t K = FREQ1 * m->C1;
         GemmArgs g{m->l1.p, K, m->w_in, K, m->h.p, H, (int)T, (int)H, (int)K, EPI_STORE, 1.f,
                    nullptr, 0, 0};
-        g.wd = m->d_in;
         HIP_TRY(launch_gemm(g, s));
     }
     if (h_sscp)
@@ -546,23 +505,23 @@ svl_status enqueue_audio(svl_audio_model *m, const AuBatch &b, const float *d_me
     if (m->L > 0)  // feed_forward1's input clamp + pre norm of layer 0
         HIP_TRY(launch_audio_rows(m->h.p, m->clip, m->layers[0].ff_pre[0], nullptr, 1.f, m->n.p,
                                   inf, nullptr, nullptr, T, W, m->eps, flag, s,
-                                  in_clamp(m->layers[0].ff_b1[0], m->layers[0].s_up[0])));
+                                  in_clamp(m->layers[0].ff_b1[0])));
     for (int64_t l = 0; l < m->L; ++l) {
         const AuLayer &ly = m->layers[(size_t)l];
         // feed_forward1 (audio.rs:1374-1433): n holds rms(clamp(h), pre).
-        HIP_TRY(launch_gemm(ffn_up(m->n.p, H, ly.ff_w1[0], ly.d_w1[0], m->act.p, T, I, H,
-                                   ly.ff_b1[0], ly.ff_b2[0], ly.s_down[0]), s));
-        HIP_TRY(launch_gemm(clipped(m->act.p, I, ly.ff_w2[0], ly.d_w2[0], I, m->tmp.p, H, T, H, I,
+        HIP_TRY(launch_gemm(ffn_up(m->n.p, H, ly.ff_w1[0], m->act.p, T, I, H, ly.ff_b1[0],
+                                   ly.ff_b2[0]), s));
+        HIP_TRY(launch_gemm(clipped(m->act.p, I, ly.ff_w2[0], I, m->tmp.p, H, T, H, I,
                                     EPI_CLIP_STORE, ly.ff_b2[0]), s));
         // h += rms(clamp(ff), post) * rw; n = rms(h, norm_pre_attn), one copy
         // per projection of Q, K and V, each clamped to its input bounds
         const Bounds *bs[3] = {&ly.bq, &ly.bk, &ly.bv};
         HIP_TRY(launch_audio_rows(m->tmp.p, m->clip, ly.ff_post[0], m->h.p, m->rw, m->h.p, inf,
                                   ly.norm_pre_attn, m->n.p, T, W, m->eps, flag, s,
-                                  in_clamp(bs, ly.s_qkv, 3, T * H)));
+                                  in_clamp(bs, 3, T * H)));
         // chunked attention (audio.rs:1529-1669)
         if (H % 128 == 0) {
-            GemmArgs g = clipped(m->n.p, H, ly.w_qkv, ly.d_qkv, H, m->qkv.p, 3 * H, T, 3 * H, H,
+            GemmArgs g = clipped(m->n.p, H, ly.w_qkv, H, m->qkv.p, 3 * H, T, 3 * H, H,
                                  EPI_CLIP_STORE, ly.bq);
             g.clip_cols = (int)H;
             g.a_seg = T * H;
@@ -574,7 +533,7 @@ svl_status enqueue_audio(svl_audio_model *m, const AuBatch &b, const float *d_me
         } else {
             for (int j = 0; j < 3; ++j)
                 HIP_TRY(launch_gemm(clipped(m->n.p + (int64_t)j * T * H, H,
-                                            ly.w_qkv + (int64_t)j * H * H, nullptr, H,
+                                            ly.w_qkv + (int64_t)j * H * H, H,
                                             m->qkv.p + (int64_t)j * H, 3 * H, T, H, H,
                                             EPI_CLIP_STORE, *bs[j]), s));
         }
@@ -604,68 +563,56 @@ svl_status enqueue_audio(svl_audio_model *m, const AuBatch &b, const float *d_me
             a.flag = flag;
             a.out_lo = ly.bpost.v[0];
             a.out_hi = ly.bpost.v[1];
-            a.out_scale = ly.s_post;
             HIP_TRY(launch_audio_attention(a, s));
         }
-        HIP_TRY(launch_gemm(clipped(m->att.p, H, ly.w_post, ly.d_post, H, m->tmp.p, H, T, H, H,
-                                    EPI_CLIP_STORE, ly.bpost), s));
+        HIP_TRY(launch_gemm(clipped(m->att.p, H, ly.w_post, H, m->tmp.p, H, T, H, H, EPI_CLIP_STORE,
+                                    ly.bpost), s));
         // h += rms(post, norm_post_attn); n = rms(h, lconv pre)
         HIP_TRY(launch_audio_rows(m->tmp.p, inf, ly.norm_post_attn, m->h.p, 1.f, m->h.p, inf,
-                                  ly.lc_pre, m->n.p, T, W, m->eps, flag, s,
-                                  in_clamp(ly.bstart, ly.s_start)));
+                                  ly.lc_pre, m->n.p, T, W, m->eps, flag, s, in_clamp(ly.bstart)));
         // light conv (audio.rs:1448-1527)
         {
-            GemmArgs g = clipped(m->n.p, H, ly.w_start, ly.d_start, H, m->gated.p, H, T,
-                                 2 * m->H_pad, H, EPI_CLIP_GLU, ly.bstart);
+            GemmArgs g = clipped(m->n.p, H, ly.w_start, H, m->gated.p, H, T, 2 * m->H_pad, H,
+                                 EPI_CLIP_GLU, ly.bstart);
             g.n_out = (int)H;
             HIP_TRY(launch_gemm(g, s));
         }
         HIP_TRY(launch_lconv(m->gated.p, ly.dw, (int)m->K, m->pos.p, m->clip, ly.lc_norm, m->n.p,
-                             T, W, m->eps, flag, s, ly.bend.v[0], ly.bend.v[1], ly.s_end));
-        HIP_TRY(launch_gemm(clipped(m->n.p, H, ly.w_end, ly.d_end, H, m->tmp.p, H, T, H, H,
-                                    EPI_CLIP_STORE, ly.bend), s));
+                             T, W, m->eps, flag, s, ly.bend.v[0], ly.bend.v[1]));
+        HIP_TRY(launch_gemm(clipped(m->n.p, H, ly.w_end, H, m->tmp.p, H, T, H, H, EPI_CLIP_STORE,
+                                    ly.bend), s));
         // h += end; n = rms(clamp(h), feed_forward2 pre)
         HIP_TRY(launch_audio_rows(m->tmp.p, inf, nullptr, m->h.p, 1.f, m->h.p, m->clip,
-                                  ly.ff_pre[1], m->n.p, T, W, m->eps, flag, s,
-                                  in_clamp(ly.ff_b1[1], ly.s_up[1])));
+                                  ly.ff_pre[1], m->n.p, T, W, m->eps, flag, s, in_clamp(ly.ff_b1[1])));
         // feed_forward2
-        HIP_TRY(launch_gemm(ffn_up(m->n.p, H, ly.ff_w1[1], ly.d_w1[1], m->act.p, T, I, H,
-                                   ly.ff_b1[1], ly.ff_b2[1], ly.s_down[1]), s));
-        HIP_TRY(launch_gemm(clipped(m->act.p, I, ly.ff_w2[1], ly.d_w2[1], I, m->tmp.p, H, T, H, I,
+        HIP_TRY(launch_gemm(ffn_up(m->n.p, H, ly.ff_w1[1], m->act.p, T, I, H, ly.ff_b1[1],
+                                   ly.ff_b2[1]), s));
+        HIP_TRY(launch_gemm(clipped(m->act.p, I, ly.ff_w2[1], I, m->tmp.p, H, T, H, I,
                                     EPI_CLIP_STORE, ly.ff_b2[1]), s));
-        // h = rms(h + rms(clamp(ff), post) * rw, norm_out); the last layer's
-        // split copy is the output projection's operand
-        OutClamp last;
-        if (m->split && l + 1 == m->L) {
-            last.split = m->n.p;
-            last.split_scale = m->s_out;
-        }
+        // h = rms(h + rms(clamp(ff), post) * rw, norm_out)
         HIP_TRY(launch_audio_rows(m->tmp.p, m->clip, ly.ff_post[1], m->h.p, m->rw, nullptr, inf,
-                                  ly.norm_out, m->h.p, T, W, m->eps, flag, s, last));
+                                  ly.norm_out, m->h.p, T, W, m->eps, flag, s));
         if (h_hidden)
             HIP_TRY(hipMemcpyAsync(h_hidden + (size_t)(l * T * H), m->h.p, (size_t)(T * H) * 4,
                                    hipMemcpyDeviceToHost, s));
         if (l + 1 < m->L)
             HIP_TRY(launch_audio_rows(m->h.p, m->clip, m->layers[(size_t)l + 1].ff_pre[0], nullptr,
                                       1.f, m->n.p, inf, nullptr, nullptr, T, W, m->eps, flag, s,
-                                      in_clamp(m->layers[(size_t)l + 1].ff_b1[0],
-                                               m->layers[(size_t)l + 1].s_up[0])));
+                                      in_clamp(m->layers[(size_t)l + 1].ff_b1[0])));
     }
     // Output projection + bias, unscaled RMSNorm of the valid rows, text
     // projection (audio.rs:1085-1133).
     {
-        GemmArgs g{m->split ? m->n.p : m->h.p, H, m->w_out, H, m->proj.p, m->P, (int)T, (int)m->P,
-                   (int)H, EPI_BIAS, 1.f, m->b_out, 0, 0};
-        g.wd = m->d_out;
+        GemmArgs g{m->h.p, H, m->w_out, H, m->proj.p, m->P, (int)T, (int)m->P, (int)H, EPI_BIAS,
+                   1.f, m->b_out, 0, 0};
         HIP_TRY(launch_gemm(g, s));
     }
     HIP_TRY(launch_finite_check(m->proj.p, T * m->P, flag, s));
     HIP_TRY(launch_compact_rms(m->proj.p, m->valid_idx.p, m->projn.p, b.tokens, (int)m->P, m->eps,
-                               flag, s, m->s_emb));
+                               flag, s));
     {
         GemmArgs g{m->projn.p, m->P, m->w_emb, m->P, d_soft, m->text_hidden, (int)b.tokens,
                    (int)m->text_hidden, (int)m->P, EPI_STORE, 1.f, nullptr, 0, 0};
-        g.wd = m->d_emb;
         HIP_TRY(launch_gemm(g, s));
     }
     HIP_TRY(launch_finite_check(d_soft, b.tokens * m->text_hidden, flag, s));
@@ -897,30 +844,14 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
     if (m->C0 > 512)
         return fail(SVL_UNSUPPORTED, "audio subsampling channels above 512 are not supported");
 
-    m->split = m->L > 0 && m->C0 == 128 && (m->C1 == 32 || m->C1 == 64) && m->H % 128 == 0 &&
-               m->P % 32 == 0;
-    std::vector<float> a, b2, nw;
+    std::vector<float> a, b2;
     auto up = [&](const std::string &name, float **dst) -> svl_status {
         ST_TRY(decode_named(by_name, name, a));
         return upload_owned(m->allocations, a.data(), a.size(), dst);
     };
-    // The projection weight [rows, K] in `w`, for an A operand scaled by a_scale.
-    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, float **dst,
-                   float **descale) -> svl_status {
-        if (!m->split) return upload_owned(m->allocations, w.data(), w.size(), dst);
-        return upload_split(m->allocations, w.data(), (int64_t)w.size() / K, K, a_scale, dst,
-                            descale);
-    };
-    auto norm_scale = [&](const std::string &name, const Bounds *b, float *scale) -> svl_status {
-        ST_TRY(decode_named(by_name, name, nw));
-        const double bound = norm_bound(nw);
-        if (m->split) *scale = split_scale(b ? clamp_bound(bound, b->v[0], b->v[1]) : bound);
-        return SVL_OK;
-    };
     const std::string sp = "audio_tower.subsample_conv_projection.";
     ST_TRY(up(sp + "layer0.conv.weight", &m->w_conv0));
     ST_TRY(up(sp + "layer0.norm.weight", &m->ln0));
-    ST_TRY(norm_scale(sp + "layer0.norm.weight", nullptr, &m->s_l0));
     // Layer-1 convolution weight [C1][C0][3][3]; the implicit-im2col GEMM
     // takes it tap-major, [C1][3 x 3][C0].
     ST_TRY(decode_named(by_name, sp + "layer1.conv.weight", a));
@@ -930,20 +861,12 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             for (int64_t t = 0; t < 9; ++t)
                 b2[(size_t)((o * 9 + t) * m->C0 + c)] = a[(size_t)((o * m->C0 + c) * 9 + t)];
     a.swap(b2);
-    ST_TRY(put(a, 9 * m->C0, m->s_l0, &m->w_conv1, &m->d_conv1));
+    ST_TRY(upload_owned(m->allocations, a.data(), a.size(), &m->w_conv1));
     ST_TRY(up(sp + "layer1.norm.weight", &m->ln1));
-    ST_TRY(norm_scale(sp + "layer1.norm.weight", nullptr, &m->s_l1));
-    ST_TRY(decode_named(by_name, sp + "input_proj_linear.weight", a));
-    ST_TRY(put(a, (int64_t)a.size() / m->H, m->s_l1, &m->w_in, &m->d_in));
-    if (m->L > 0)
-        ST_TRY(norm_scale("audio_tower.layers." + std::to_string(m->L - 1) + ".norm_out.weight",
-                          nullptr, &m->s_out));
-    ST_TRY(decode_named(by_name, "audio_tower.output_proj.weight", a));
-    ST_TRY(put(a, m->H, m->s_out, &m->w_out, &m->d_out));
+    ST_TRY(up(sp + "input_proj_linear.weight", &m->w_in));
+    ST_TRY(up("audio_tower.output_proj.weight", &m->w_out));
     ST_TRY(up("audio_tower.output_proj.bias", &m->b_out));
-    if (m->split) m->s_emb = split_scale(std::sqrt((double)m->P));
-    ST_TRY(decode_named(by_name, "embed_audio.embedding_projection.weight", a));
-    ST_TRY(put(a, m->P, m->s_emb, &m->w_emb, &m->d_emb));
+    ST_TRY(up("embed_audio.embedding_projection.weight", &m->w_emb));
 
     const std::vector<float> table = position_table(m->H, m->positions);
     float *d_table = nullptr;
@@ -958,24 +881,10 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             const std::string q = p + ffs[f];
             ST_TRY(up(q + "pre_layer_norm.weight", &ly.ff_pre[f]));
             ST_TRY(up(q + "post_layer_norm.weight", &ly.ff_post[f]));
+            ST_TRY(up(q + "ffw_layer_1.linear.weight", &ly.ff_w1[f]));
+            ST_TRY(up(q + "ffw_layer_2.linear.weight", &ly.ff_w2[f]));
             ST_TRY(read_bounds(by_name, q + "ffw_layer_1", ly.ff_b1[f]));
             ST_TRY(read_bounds(by_name, q + "ffw_layer_2", ly.ff_b2[f]));
-            ST_TRY(norm_scale(q + "pre_layer_norm.weight", &ly.ff_b1[f], &ly.s_up[f]));
-            ST_TRY(decode_named(by_name, q + "ffw_layer_1.linear.weight", a));
-            if (m->split) {
-                // |silu(x)| <= |x|, then the down projection's input clamp
-                double up_bound;
-                ST_TRY(upload_rows(m->allocations, a.data(), m->I, m->H, &ly.ff_w1[f], &ly.d_w1[f]));
-                ST_TRY(clipped_bound(ly.ff_w1[f], m->I, m->H, ly.ff_pre[f], ly.ff_b1[f],
-                                     ly.d_w1[f], &up_bound));
-                ly.s_down[f] =
-                    split_scale(clamp_bound(up_bound, ly.ff_b2[f].v[0], ly.ff_b2[f].v[1]));
-                ST_TRY(split_weight(ly.ff_w1[f], m->I, m->H, ly.s_up[f], ly.d_w1[f]));
-            } else {
-                ST_TRY(upload_owned(m->allocations, a.data(), a.size(), &ly.ff_w1[f]));
-            }
-            ST_TRY(decode_named(by_name, q + "ffw_layer_2.linear.weight", a));
-            ST_TRY(put(a, m->I, ly.s_down[f], &ly.ff_w2[f], &ly.d_w2[f]));
         }
         std::vector<float> qkv((size_t)(3 * m->H * m->H));
         const char *projs[3] = {"q_proj", "k_proj", "v_proj"};
@@ -984,24 +893,10 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             ST_TRY(decode_named(by_name, p + "self_attn." + projs[j] + ".linear.weight", a));
             std::copy(a.begin(), a.end(), qkv.begin() + (int64_t)j * m->H * m->H);
             ST_TRY(read_bounds(by_name, p + "self_attn." + projs[j], *bs[j]));
-            ST_TRY(norm_scale(p + "norm_pre_attn.weight", bs[j], &ly.s_qkv[j]));
         }
-        ST_TRY(up(p + "norm_pre_attn.weight", &ly.norm_pre_attn));
-        double v_bound = 0;  // attention outputs are convex sums of value rows (or zero)
-        if (m->split) {
-            const int64_t H = m->H;
-            ST_TRY(upload_rows(m->allocations, qkv.data(), 3 * H, H, &ly.w_qkv, &ly.d_qkv));
-            ST_TRY(clipped_bound(ly.w_qkv + 2 * H * H, H, H, ly.norm_pre_attn, ly.bv, ly.d_qkv,
-                                 &v_bound));
-            for (int j = 0; j < 3; ++j)
-                ST_TRY(split_weight(ly.w_qkv + j * H * H, H, H, ly.s_qkv[j], ly.d_qkv + j * H));
-        } else {
-            ST_TRY(upload_owned(m->allocations, qkv.data(), qkv.size(), &ly.w_qkv));
-        }
+        ST_TRY(upload_owned(m->allocations, qkv.data(), qkv.size(), &ly.w_qkv));
+        ST_TRY(up(p + "self_attn.post.linear.weight", &ly.w_post));
         ST_TRY(read_bounds(by_name, p + "self_attn.post", ly.bpost));
-        if (m->split) ly.s_post = split_scale(clamp_bound(v_bound, ly.bpost.v[0], ly.bpost.v[1]));
-        ST_TRY(decode_named(by_name, p + "self_attn.post.linear.weight", a));
-        ST_TRY(put(a, m->H, ly.s_post, &ly.w_post, &ly.d_post));
         // per-dimension query scale q_scale * softplus(per_dim_scale) (audio.rs:1565-1576)
         ST_TRY(decode_named(by_name, p + "self_attn.per_dim_scale", a));
         std::vector<float> qf((size_t)m->hd);
@@ -1025,21 +920,16 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             ly.relk = relk;
         }
         ST_TRY(up(p + "lconv1d.pre_layer_norm.weight", &ly.lc_pre));
-        ST_TRY(read_bounds(by_name, p + "lconv1d.linear_start", ly.bstart));
-        ST_TRY(norm_scale(p + "lconv1d.pre_layer_norm.weight", &ly.bstart, &ly.s_start));
         ST_TRY(decode_named(by_name, p + "lconv1d.linear_start.linear.weight", a));
         {   // rows [0, H) are the gated values, [H, 2H) the gates
             std::vector<float> first(a.begin(), a.begin() + m->H * m->H),
                 second(a.begin() + m->H * m->H, a.end());
-            const std::vector<float> il =
-                interleave_gate_up(first, second, m->H, m->H_pad, m->H, m->split ? 16 : 32);
-            ST_TRY(put(il, m->H, ly.s_start, &ly.w_start, &ly.d_start));
+            const std::vector<float> il = interleave_gate_up(first, second, m->H, m->H_pad, m->H, 32);
+            ST_TRY(upload_owned(m->allocations, il.data(), il.size(), &ly.w_start));
         }
+        ST_TRY(read_bounds(by_name, p + "lconv1d.linear_start", ly.bstart));
+        ST_TRY(up(p + "lconv1d.linear_end.linear.weight", &ly.w_end));
         ST_TRY(read_bounds(by_name, p + "lconv1d.linear_end", ly.bend));
-        // |silu(x)| <= |x| of the convolution's norm
-        ST_TRY(norm_scale(p + "lconv1d.conv_norm.weight", &ly.bend, &ly.s_end));
-        ST_TRY(decode_named(by_name, p + "lconv1d.linear_end.linear.weight", a));
-        ST_TRY(put(a, m->H, ly.s_end, &ly.w_end, &ly.d_end));
         // depthwise weight [H, 1, K] uploaded tap-major, [K, H]: the kernel
         // reads four channels' weights of one tap as one float4
         ST_TRY(decode_named(by_name, p + "lconv1d.depthwise_conv1d.weight", a));
@@ -1053,10 +943,10 @@ svl_status svl_audio_model_create(svl_ctx *ctx, const svl_audio_config *cfg, int
             ST_TRY(upload_owned(m->allocations, dwt.data(), dwt.size(), &ly.dw));
         }
         ST_TRY(up(p + "lconv1d.conv_norm.weight", &ly.lc_norm));
+        ST_TRY(up(p + "norm_pre_attn.weight", &ly.norm_pre_attn));
         ST_TRY(up(p + "norm_post_attn.weight", &ly.norm_post_attn));
         ST_TRY(up(p + "norm_out.weight", &ly.norm_out));
     }
-    if (m->split) HIP_TRY(hipStreamSynchronize(nullptr));  // the weights' conversion
     HIP_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
     HIP_TRY(hipHostMalloc((void **)&m->h_flag, sizeof(int), hipHostMallocDefault));
     *out = guard.release();

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void sscp_conv0_kernel(const float *__restrict
                                                          const float *__restrict__ w,
                                                          const float *__restrict__ ln, int C0,
                                                          float eps, float *__restrict__ out,
-                                                         int *flag, float out_scale) {
+                                                         int *flag) {
     __shared__ float taps[3][SSCP_TAPS_W];
     __shared__ float ws[4 * CPT * 9];
     const int64_t r = blockIdx.x;
@@ -84,21 +84,6 @@ __global__ __launch_bounds__(256) void sscp_conv0_kernel(const float *__restrict
     const float inv = 1.0f / sqrtf(var + eps);
     ok = ok && isfinite(inv);
     float *o = out + (r * FREQ0 + f) * C0 + c0;
-    if constexpr (CPT == 32) {
-        if (out_scale > 0.f) {  // the thread's 32 channels are one split block
-            auto four = [&](int j) {
-                f32x4 y;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    y[e] = fmaxf((v[j + e] - mean) * inv * ln[c0 + j + e], 0.0f) * out_scale;
-                return y;
-            };
-#pragma unroll
-            for (int c = 0; c < 4; ++c) split_store8(o, 0, c, four(4 * c), four(16 + 4 * c));
-            if (!ok) raise_flag(flag, FLAG_NONFINITE);
-            return;
-        }
-    }
     if (CPT % 4 == 0 && C0 == 4 * CPT) {
 #pragma unroll
         for (int j = 0; j < CPT; j += 4)
@@ -116,13 +101,13 @@ __global__ __launch_bounds__(256) void sscp_conv0_kernel(const float *__restrict
 
 hipError_t launch_sscp_conv0(const float *mel, const uint8_t *mask, const SscpRow *rows,
                              int64_t n_rows, const float *w, const float *ln, int C0, float eps,
-                             float *out, int *flag, hipStream_t s, float out_scale) {
+                             float *out, int *flag, hipStream_t s) {
     if (n_rows <= 0) return hipSuccess;
-    if (n_rows > INT32_MAX || C0 < 1 || (out_scale > 0.f && C0 != 128)) return hipErrorInvalidValue;
+    if (n_rows > INT32_MAX || C0 < 1) return hipErrorInvalidValue;
     static_assert(FREQ0 * 4 == 256, "four threads per output frequency");
 #define C0_LAUNCH(CPT)                                                                       \
     hipLaunchKernelGGL(sscp_conv0_kernel<CPT>, dim3((unsigned)n_rows), dim3(256), 0, s, mel, \
-                       mask, rows, w, ln, C0, eps, out, flag, out_scale)
+                       mask, rows, w, ln, C0, eps, out, flag)
     const int cpt = (C0 + 3) / 4;
     if (cpt <= 8) C0_LAUNCH(8);
     else if (cpt <= 16) C0_LAUNCH(16);
@@ -138,8 +123,7 @@ hipError_t launch_sscp_conv0(const float *mel, const uint8_t *mask, const SscpRo
 // positions, in place; one wave per position.
 __global__ __launch_bounds__(256) void sscp_ln_relu_kernel(float *__restrict__ x,
                                                            const float *__restrict__ ln, int C,
-                                                           int64_t n, float eps, int *flag,
-                                                           float out_scale) {
+                                                           int64_t n, float eps, int *flag) {
     const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (p >= n) return;
@@ -159,23 +143,15 @@ __global__ __launch_bounds__(256) void sscp_ln_relu_kernel(float *__restrict__ x
     var = wave_sum(var) / (float)C;
     const float inv = 1.0f / sqrtf(var + eps);
     ok = ok && isfinite(inv);
-    if (out_scale > 0.f) {
-        // at most one channel per lane: the wave has read the row before it
-        // stores the split values over it
-        if (lane < C)
-            split_store1(row, lane, fmaxf((row[lane] - mean) * inv * ln[lane], 0.0f) * out_scale);
-    } else {
-        for (int c = lane; c < C; c += 64) row[c] = fmaxf((row[c] - mean) * inv * ln[c], 0.0f);
-    }
+    for (int c = lane; c < C; c += 64) row[c] = fmaxf((row[c] - mean) * inv * ln[c], 0.0f);
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
 }
 
 hipError_t launch_sscp_ln_relu(float *x, const float *ln, int C, int64_t n, float eps, int *flag,
-                               hipStream_t s, float out_scale) {
+                               hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    if (out_scale > 0.f && C != 32 && C != 64) return hipErrorInvalidValue;
     hipLaunchKernelGGL(sscp_ln_relu_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, x, ln,
-                       C, n, eps, flag, out_scale);
+                       C, n, eps, flag);
     return hipGetLastError();
 }
 
@@ -238,8 +214,8 @@ __global__ __launch_bounds__(256) void audio_rows_kernel(
                     ((f32x4 *)(h_out + row * width))[i] = v[c];
                 } else {
                     for (int k = 0; k < oc.copies; ++k)
-                        store_row4(h_out + k * oc.stride + row * width, i,
-                                   clamp4(v[c], oc.lo[k], oc.hi[k]), oc.scale[k]);
+                        ((f32x4 *)(h_out + k * oc.stride + row * width))[i] =
+                            clamp4(v[c], oc.lo[k], oc.hi[k]);
                 }
             }
             if (w2) {
@@ -260,9 +236,7 @@ __global__ __launch_bounds__(256) void audio_rows_kernel(
                 const f32x4 y = v[c] * inv * w2v[c];
                 ok = ok && finite4(y);
                 for (int k = 0; k < oc.copies; ++k)
-                    store_row4(n_out + k * oc.stride + row * width, i,
-                               clamp4(y, oc.lo[k], oc.hi[k]), oc.scale[k]);
-                if (oc.split) store_row4(oc.split + row * width, i, y, oc.split_scale);
+                    ((f32x4 *)(n_out + k * oc.stride + row * width))[i] = clamp4(y, oc.lo[k], oc.hi[k]);
             }
         }
     }
@@ -274,8 +248,6 @@ hipError_t launch_audio_rows(const float *x, float c1, const float *w1, const fl
                              int width, float eps, int *flag, hipStream_t s, const OutClamp &oc) {
     if (rows <= 0) return hipSuccess;
     if (width <= 0 || width % 4 || width > 2048 || oc.copies < 1 || oc.copies > 3)
-        return hipErrorInvalidValue;
-    if (width % 32 && (oc.split || oc.scale[0] > 0.f || oc.scale[1] > 0.f || oc.scale[2] > 0.f))
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)((rows + 3) / 4));
 #define AR_LAUNCH(NC)                                                                        \
@@ -510,16 +482,14 @@ __global__ __launch_bounds__(64 * AW) void audio_attn_kernel(AudioAttnArgs p) {
                 const int q = gg + G * j;
                 if (q >= nb) continue;
                 const bool on = __builtin_amdgcn_readlane((int)live[j], KL * gg) != 0;
-                float *orow = p.out + (r0 + q0 + q) * p.ldo;
+                float *orow = p.out + (r0 + q0 + q) * p.ldo + (int64_t)h * hd;
 #pragma unroll
                 for (int t = 0; t < TD; ++t) {
                     const int d = lane + 64 * t;
                     if (d < hd) {
                         const float y = on ? acc[q][t] : 0.0f;
                         ok = ok && isfinite(y);
-                        const float z = clamp_ref(y, p.out_lo, p.out_hi);
-                        if (p.out_scale > 0.f) split_store1(orow, h * hd + d, z * p.out_scale);
-                        else orow[h * hd + d] = z;
+                        orow[d] = clamp_ref(y, p.out_lo, p.out_hi);
                     }
                 }
             }
@@ -586,7 +556,7 @@ __global__ __launch_bounds__(256) void lconv_kernel(const float *__restrict__ ga
                                                     const int32_t *__restrict__ pos, float clip,
                                                     const float *__restrict__ w, float *__restrict__ out,
                                                     int64_t rows, int width, float eps, int *flag,
-                                                    float out_lo, float out_hi, float out_scale) {
+                                                    float out_lo, float out_hi) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
@@ -626,7 +596,7 @@ __global__ __launch_bounds__(256) void lconv_kernel(const float *__restrict__ ga
             y.z = silu_ref(y.z);
             y.w = silu_ref(y.w);
             ok = ok && finite4(y);
-            store_row4(out + row * width, i, clamp4(y, out_lo, out_hi), out_scale);
+            ((f32x4 *)(out + row * width))[i] = clamp4(y, out_lo, out_hi);
         }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
@@ -634,13 +604,13 @@ __global__ __launch_bounds__(256) void lconv_kernel(const float *__restrict__ ga
 
 hipError_t launch_lconv(const float *gated, const float *dw, int K, const int32_t *pos, float clip,
                         const float *w, float *out, int64_t rows, int width, float eps, int *flag,
-                        hipStream_t s, float out_lo, float out_hi, float out_scale) {
+                        hipStream_t s, float out_lo, float out_hi) {
     if (rows <= 0) return hipSuccess;
-    if (width % 4 || width > 2048 || (out_scale > 0.f && width % 32)) return hipErrorInvalidValue;
+    if (width % 4 || width > 2048) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((rows + 3) / 4));
 #define LC_LAUNCH(NC)                                                                           \
     hipLaunchKernelGGL(lconv_kernel<NC>, grid, dim3(256), 0, s, gated, dw, K, pos, clip, w, out, \
-                       rows, width, eps, flag, out_lo, out_hi, out_scale)
+                       rows, width, eps, flag, out_lo, out_hi)
     switch ((width + 255) / 256) {
         case 1: LC_LAUNCH(1); break;
         case 2: LC_LAUNCH(2); break;
@@ -659,8 +629,7 @@ template <int NC>
 __global__ __launch_bounds__(256) void compact_rms_kernel(const float *__restrict__ x,
                                                           const int32_t *__restrict__ idx,
                                                           float *__restrict__ out, int64_t rows,
-                                                          int width, float eps, int *flag,
-                                                          float out_scale) {
+                                                          int width, float eps, int *flag) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
@@ -685,20 +654,19 @@ __global__ __launch_bounds__(256) void compact_rms_kernel(const float *__restric
         if (i < nv) {
             const f32x4 y = v[c] * inv;
             ok = ok && finite4(y);
-            store_row4(out + row * width, i, y, out_scale);
+            ((f32x4 *)(out + row * width))[i] = y;
         }
     }
     if (!ok) raise_flag(flag, FLAG_NONFINITE);
 }
 
 hipError_t launch_compact_rms(const float *x, const int32_t *idx, float *out, int64_t rows,
-                              int width, float eps, int *flag, hipStream_t s, float out_scale) {
+                              int width, float eps, int *flag, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    if (width % 4 || width > 2048 || (out_scale > 0.f && width % 32)) return hipErrorInvalidValue;
+    if (width % 4 || width > 2048) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((rows + 3) / 4));
 #define CR_LAUNCH(NC) \
-    hipLaunchKernelGGL(compact_rms_kernel<NC>, grid, dim3(256), 0, s, x, idx, out, rows, width, eps, flag, \
-                       out_scale)
+    hipLaunchKernelGGL(compact_rms_kernel<NC>, grid, dim3(256), 0, s, x, idx, out, rows, width, eps, flag)
     switch ((width + 255) / 256) {
         case 1: CR_LAUNCH(1); break;
         case 2: CR_LAUNCH(2); break;

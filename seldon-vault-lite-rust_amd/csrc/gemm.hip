@@ -992,7 +992,6 @@ bool gemm_conv_ok(const GemmArgs &a) {
 hipError_t launch_gemm_conv(const GemmArgs &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
     if (!gemm_conv_ok(a)) return hipErrorInvalidValue;
-    if (a.wd) return launch_gemm_conv_split(a, s);
     if (a.N <= 32) return launch_dma<128, 32, 32, EPI_STORE, 4, 2, 4, true>(a, s);
     return launch_dma<64, 64, 32, EPI_STORE, 4, 2, 2, true>(a, s);
 }

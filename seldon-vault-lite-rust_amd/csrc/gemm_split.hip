@@ -45,20 +45,10 @@
 
 namespace svl {
 
-template <int EPI>
-constexpr bool split_paired() {
-    return EPI == EPI_GEGLU || EPI == EPI_CLIP_GLU;
-}
-
-template <int EPI>
-constexpr bool split_clipped() {
-    return EPI == EPI_CLIP_STORE || EPI == EPI_CLIP_SILU || EPI == EPI_CLIP_GLU;
-}
-
 // Outputs that only another GEMM reads: stored as split rows.
 template <int EPI>
 constexpr bool split_output() {
-    return EPI == EPI_GEGLU || EPI == EPI_GELU_MUL || EPI == EPI_CLIP_SILU;
+    return EPI == EPI_GEGLU || EPI == EPI_GELU_MUL;
 }
 
 // Stores `lim` (<= 4) consecutive floats of a row.
@@ -72,7 +62,7 @@ __device__ __forceinline__ void store_run(float *p, const f32x4 &v, int lim, boo
     }
 }
 
-template <int BM, int BN, int KB, int EPI, int MINB, int NS, int WMW, int WNW, bool CONV, bool RASTER>
+template <int BM, int BN, int KB, int EPI, int MINB, int NS, int WMW, int WNW, bool RASTER>
 __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, int tiles_m,
                                                                    int tiles_n) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -87,7 +77,8 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
     constexpr int A_CH = BM / RPK / NW, W_CH = BN / RPK / NW;  // DMA instructions per wave
     // the narrowest wave tile (one 16-column run per lane) has no pairs
     constexpr bool NARROW = WTN == 16;
-    static_assert(!NARROW || !split_paired<EPI>(), "paired epilogues take 32-column wave tiles");
+    constexpr bool PAIRED = EPI == EPI_GEGLU;
+    static_assert(!NARROW || !PAIRED, "paired epilogues take 32-column wave tiles");
     static_assert(WTM % 16 == 0 && (WTN % 32 == 0 || NARROW) && A_CH >= 1 && W_CH >= 1 &&
                       A_CH * RPK * NW == BM && W_CH * RPK * NW == BN,
                   "tile shape");
@@ -139,47 +130,20 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
     const int wm = wave / WNW, wn = wave % WNW;
     const int lr = lane & 15, lc = lane >> 4;  // fragment row and chunk of this lane
     const int M = p.M, N = p.N;
-    const int seg = uniform(split_clipped<EPI>() && p.clip_cols > 0 ? n0 / p.clip_cols : 0);
 
     // operand windows: reads past the last valid row return zero
-    const __amdgpu_buffer_rsrc_t ra = CONV
-        ? __builtin_amdgcn_make_buffer_rsrc((void *)uniform(p.A), (short)0,
-                                            uniform((int)(p.conv_a_floats * 4)), 0x00020000)
-        : __builtin_amdgcn_make_buffer_rsrc(
-              (void *)uniform(p.A + (int64_t)seg * p.a_seg + (int64_t)m0 * p.lda), (short)0,
-              uniform((int)(min(BM, M - m0) * p.lda * 4)), 0x00020000);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)uniform(p.A + (int64_t)m0 * p.lda), (short)0,
+        uniform((int)(min(BM, M - m0) * p.lda * 4)), 0x00020000);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         (void *)uniform(p.W + (int64_t)n0 * p.ldw), (short)0,
         uniform((int)(min(BN, N - n0) * p.ldw * 4)), 0x00020000);
     int a_off[A_CH], w_off[W_CH];
-    // implicit im2col: per A row of this lane, the layer-0 float offset of
-    // tap (0, 0) channel 0 and the valid kt (bits 0-2) and kf (bits 3-5)
-    int a_taps[CONV ? A_CH : 1];
 #pragma unroll
     for (int q = 0; q < A_CH; ++q) {
         const int row = (wave * A_CH + q) * RPK + lane / CPR;
         const int c = (lane % CPR) ^ ((row / RPL) % SWZ);
-        if constexpr (CONV) {
-            a_off[q] = 0;
-            a_taps[q] = 0;
-            const int m = m0 + row;
-            if (m < M) {
-                const int r = m / p.conv_f1, f = m - r * p.conv_f1;
-                const int base = p.conv_rows[3 * r], t = p.conv_rows[3 * r + 1],
-                          len = p.conv_rows[3 * r + 2];
-                int bits = 0;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const int it = 2 * t + k - 1, iff = 2 * f + k - 1;
-                    if (it >= 0 && it < len && p.conv_mask[base + it]) bits |= 1 << k;
-                    if (iff >= 0 && iff < p.conv_f0) bits |= 8 << k;
-                }
-                a_off[q] = ((base + 2 * t - 1) * p.conv_f0 + 2 * f - 1) * p.conv_c0 + 4 * c;
-                a_taps[q] = bits;
-            }
-        } else {
-            a_off[q] = (row * (int)p.lda + 4 * c) * 4;
-        }
+        a_off[q] = (row * (int)p.lda + 4 * c) * 4;
     }
 #pragma unroll
     for (int q = 0; q < W_CH; ++q) {
@@ -192,20 +156,9 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
         float *as = stage_a(st);
         float *ws = stage_w(st);
         if (q < A_CH) {
-            if constexpr (CONV) {
-                // a slice lies within one tap; a tap outside the clip, the
-                // mask or the frequencies reads past the window, as zero
-                const int tap = k0 / p.conv_c0, kt = tap / 3, kf = tap - 3 * kt;
-                const int delta = (kt * p.conv_f0 + kf) * p.conv_c0 + (k0 - tap * p.conv_c0);
-                const bool ok = (a_taps[q] >> kt & 1) && (a_taps[q] >> (3 + kf) & 1);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    ra, (__attribute__((address_space(3))) void *)&as[(wave * A_CH + q) * 256], 16,
-                    ok ? (a_off[q] + delta) * 4 : 0x7FFFFFF0, 0, 0, 0);
-            } else {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    ra, (__attribute__((address_space(3))) void *)&as[(wave * A_CH + q) * 256], 16,
-                    a_off[q], k0 * 4, 0, 0);
-            }
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                ra, (__attribute__((address_space(3))) void *)&as[(wave * A_CH + q) * 256], 16,
+                a_off[q], k0 * 4, 0, 0);
         } else {
             const int r = q - A_CH;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -341,13 +294,8 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
     }
 
     // ---- epilogue ----
-    float olo = 0.f, ohi = 0.f;
-    if constexpr (split_clipped<EPI>()) {
-        olo = p.clip[seg][2];
-        ohi = p.clip[seg][3];
-    }
     // column limit of C; vector stores need aligned rows
-    const int limit = split_paired<EPI>() ? p.n_out : N;
+    const int limit = PAIRED ? p.n_out : N;
     const bool vec = (p.ldc & 3) == 0 && ((uintptr_t)p.C & 15) == 0;
     auto value = [&](int i, int j) { return (acc[i][j] + acl[i][j]) * rs[i] * wd[j]; };
     constexpr int NBLK = NARROW ? 1 : WTN / 32;
@@ -358,38 +306,24 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
         float *crow = p.C + (int64_t)m * p.ldc;
         // split outputs: the row's scale (1 / rs for rows with their own)
         const float os = SOUT ? (p.rs ? p.out_scale / rs[i] : p.out_scale) : 1.f;
-        if constexpr (split_paired<EPI>()) {
+        if constexpr (PAIRED) {
 #pragma unroll
             for (int b = 0; b < NBLK; ++b) {
                 const f32x4 x = value(i, 2 * b), y = value(i, 2 * b + 1);
                 f32x4 o;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if constexpr (EPI == EPI_GEGLU)
-                        o[r] = gelu_tanh(x[r]) * y[r];
-                    else
-                        o[r] = clamp_ref(x[r], olo, ohi) * sigmoid_ref(clamp_ref(y[r], olo, ohi));
-                }
+                for (int r = 0; r < 4; ++r) o[r] = gelu_tanh(x[r]) * y[r];
                 const int n = nw / 2 + 16 * b + 4 * lc;  // output columns n .. n + 3
-                if constexpr (SOUT) {
-                    if (n < limit) split_store4(crow, n, o * os);
-                } else {
-                    store_run(crow + n, o, limit - n, vec);
-                }
+                if (n < limit) split_store4(crow, n, o * os);
             }
         } else {
             // block j with its epilogue applied, columns col(j) .. + 3
             auto out = [&](int j) {
-                const int n = col(j);
                 f32x4 v = value(i, j);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     float x = v[r];
                     if constexpr (EPI == EPI_GELU_MUL) x = gelu_tanh(x) * aux[i][j][r];
-                    if constexpr (EPI == EPI_BIAS) x = x + (n + r < N ? p.aux[n + r] : 0.f);
-                    if constexpr (EPI == EPI_CLIP_STORE) x = clamp_ref(x, olo, ohi);
-                    if constexpr (EPI == EPI_CLIP_SILU)
-                        x = clamp_ref(silu_ref(clamp_ref(x, olo, ohi)), p.post_lo, p.post_hi);
                     v[r] = SOUT ? x * os : x;
                 }
                 return v;
@@ -417,17 +351,15 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
 // (6230 x 768 x 768 26.5 against 27.2 us, 3000 x 1024 x 4096 75.7 against 79.4).
 constexpr int SPLIT_RASTER_MIN_N = 1280;
 
-template <int BM, int BN, int KB, int EPI, int MINB, int NS, int WMW, int WNW, bool CONV = false>
+template <int BM, int BN, int KB, int EPI, int MINB, int NS, int WMW, int WNW>
 static hipError_t launch_split_tile(const GemmArgs &a, hipStream_t s) {
     const int tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-    if constexpr (!CONV)
-        if (a.N >= SPLIT_RASTER_MIN_N) {
-            hipLaunchKernelGGL((gemm_split<BM, BN, KB, EPI, MINB, NS, WMW, WNW, false, true>),
-                               dim3(tm * tn), dim3(64 * WMW * WNW), 0, s, a, tm, tn);
-            return hipGetLastError();
-        }
-    hipLaunchKernelGGL((gemm_split<BM, BN, KB, EPI, MINB, NS, WMW, WNW, CONV, false>),
-                       dim3(tm * tn), dim3(64 * WMW * WNW), 0, s, a, tm, tn);
+    if (a.N >= SPLIT_RASTER_MIN_N)
+        hipLaunchKernelGGL((gemm_split<BM, BN, KB, EPI, MINB, NS, WMW, WNW, true>), dim3(tm * tn),
+                           dim3(64 * WMW * WNW), 0, s, a, tm, tn);
+    else
+        hipLaunchKernelGGL((gemm_split<BM, BN, KB, EPI, MINB, NS, WMW, WNW, false>), dim3(tm * tn),
+                           dim3(64 * WMW * WNW), 0, s, a, tm, tn);
     return hipGetLastError();
 }
 
@@ -455,22 +387,23 @@ static hipError_t launch_split_auto(const GemmArgs &a, hipStream_t s) {
     auto tiles = [&](int bm, int bn) {
         return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
     };
+    constexpr bool PAIRED = EPI == EPI_GEGLU;
     const bool k128 = a.K % 128 == 0;
     if (tiles(64, 64) <= 256 && k128) {
-        if constexpr (!split_paired<EPI>())
+        if constexpr (!PAIRED)
             if (tiles(32, 16) <= 256) {
                 if (a.K % 256 == 0) return launch_split_tile<32, 16, 8, EPI, 1, 3, 2, 1>(a, s);
                 return launch_split_tile<32, 16, 4, EPI, 1, 4, 2, 1>(a, s);
             }
         if (tiles(32, 32) <= 256) {
-            if constexpr (split_paired<EPI>()) {
+            if constexpr (PAIRED) {
                 if (a.K % 256 == 0) return launch_split_tile<32, 32, 8, EPI, 1, 2, 2, 1>(a, s);
             } else {
                 if (a.K % 256 == 0) return launch_split_tile<32, 32, 8, EPI, 1, 2, 2, 2>(a, s);
                 return launch_split_tile<32, 32, 4, EPI, 1, 3, 2, 2>(a, s);
             }
         }
-        if constexpr (split_paired<EPI>()) {
+        if constexpr (PAIRED) {
             if (tiles(64, 32) <= 256) return launch_split_tile<64, 32, 4, EPI, 1, 3, 4, 1>(a, s);
         } else if (tiles(32, 32) <= 512) {
             return launch_split_tile<32, 32, 4, EPI, 2, 2, 2, 2>(a, s);
@@ -500,20 +433,8 @@ hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s) {
         case EPI_STORE: return launch_split_auto<EPI_STORE>(a, s);
         case EPI_GEGLU: return launch_split_auto<EPI_GEGLU>(a, s);
         case EPI_GELU_MUL: return launch_split_auto<EPI_GELU_MUL>(a, s);
-        case EPI_BIAS: return launch_split_auto<EPI_BIAS>(a, s);
-        case EPI_CLIP_STORE: return launch_split_auto<EPI_CLIP_STORE>(a, s);
-        case EPI_CLIP_SILU: return launch_split_auto<EPI_CLIP_SILU>(a, s);
-        case EPI_CLIP_GLU: return launch_split_auto<EPI_CLIP_GLU>(a, s);
     }
     return hipErrorInvalidValue;
-}
-
-// The implicit-im2col convolution (gemm_conv_ok holds): 32-k slices that each
-// lie within one tap; the waves stacked along M for at most 32 channels.
-hipError_t launch_gemm_conv_split(const GemmArgs &a, hipStream_t s) {
-    if (a.K % 32 || (uintptr_t)a.wd % 16) return hipErrorInvalidValue;
-    if (a.N <= 32) return launch_split_tile<128, 32, 1, EPI_STORE, 4, 2, 4, 1, true>(a, s);
-    return launch_split_tile<64, 64, 1, EPI_STORE, 4, 2, 2, 2, true>(a, s);
 }
 
 // ---- split rows -----------------------------------------------------------------

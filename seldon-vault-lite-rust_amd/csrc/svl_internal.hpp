@@ -86,12 +86,10 @@ hipError_t launch_gemm_simple(const GemmArgs &a, hipStream_t s);
 // K % 32 == 0), and every epilogue value is first descaled by wd[n] (and
 // rs[m] where rows carry scales of their own): C = epilogue((A . W^T) *
 // rs[m] * wd[n]). Paired epilogues take W rows interleaved in 16-row blocks.
-// The epilogues whose output only another GEMM reads (GEGLU, GELU_MUL,
-// CLIP_SILU) store split rows scaled by out_scale (out_scale / rs[m] with row
-// scales; ldc % 32 == 0, the output width a multiple of 32).
+// EPI_STORE, and the epilogues whose output only another GEMM reads (GEGLU,
+// GELU_MUL), which store split rows scaled by out_scale (out_scale / rs[m] with
+// row scales; ldc % 32 == 0, the output width a multiple of 32).
 hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s);
-// launch_gemm_conv on split operands.
-hipError_t launch_gemm_conv_split(const GemmArgs &a, hipStream_t s);
 constexpr int SPLIT_RASTER_M = 8;  // M blocks per rasterization group
 // x [rows, K] (leading dimension ldx) to split rows of K_pad >= K, each
 // scaled by its own power of two; descale[row] = also / scale.
@@ -280,24 +278,18 @@ static_assert(sizeof(SscpRow) == 3 * sizeof(int32_t), "GemmArgs::conv_rows reads
 // masked frames skipped, LayerNorm + ReLU). C0 <= 512.
 hipError_t launch_sscp_conv0(const float *mel, const uint8_t *mask, const SscpRow *rows,
                              int64_t n_rows, const float *w, const float *ln, int C0, float eps,
-                             float *out, int *flag, hipStream_t s, float out_scale = 0.f);
+                             float *out, int *flag, hipStream_t s);
 // In place: x[p] = relu(layernorm(x[p], ln)) over C channels, n positions.
-// Both store split values times out_scale when it is positive (C0 = 128,
-// C = 32 or 64).
 hipError_t launch_sscp_ln_relu(float *x, const float *ln, int C, int64_t n, float eps, int *flag,
-                               hipStream_t s, float out_scale = 0.f);
+                               hipStream_t s);
 // Clamped stores of a row kernel's last output (the A operand of a clipped
 // linear): copy c goes to out + c * stride clamped to [lo[c], hi[c]]. The
-// default is one unclamped copy. A copy with a positive scale is stored as
-// split rows; `split` receives a further, unclamped split copy.
+// default is one unclamped copy.
 struct OutClamp {
     int copies = 1;
     int64_t stride = 0;
     float lo[3] = {-__builtin_huge_valf(), -__builtin_huge_valf(), -__builtin_huge_valf()};
     float hi[3] = {__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
-    float scale[3] = {0.f, 0.f, 0.f};
-    float *split = nullptr;
-    float split_scale = 0.f;
 };
 // t = w1 ? rms(clamp(x, +-c1), w1) : x; h = res ? res + t * rw : t (-> h_out);
 // if w2: n_out = rms(clamp(h, +-c2), w2). `oc` applies to the last output
@@ -323,7 +315,6 @@ struct AudioAttnArgs {
     int *flag;
     // the output projection's input bounds, applied as the output is stored
     float out_lo = -__builtin_huge_valf(), out_hi = __builtin_huge_valf();
-    float out_scale = 0.f;  // > 0: out holds split rows scaled by it
 };
 hipError_t launch_audio_attention(const AudioAttnArgs &a, hipStream_t s);
 // Causal depthwise conv (dw tap-major, [K, width]) within each clip, clamp, RMSNorm(w), SiLU,
@@ -331,12 +322,10 @@ hipError_t launch_audio_attention(const AudioAttnArgs &a, hipStream_t s);
 hipError_t launch_lconv(const float *gated, const float *dw, int K, const int32_t *pos, float clip,
                         const float *w, float *out, int64_t rows, int width, float eps, int *flag,
                         hipStream_t s, float out_lo = -__builtin_huge_valf(),
-                        float out_hi = __builtin_huge_valf(), float out_scale = 0.f);
-// out[j] = unscaled_rms(x[idx[j]]). Both store split rows times out_scale when
-// it is positive (width % 32 == 0).
+                        float out_hi = __builtin_huge_valf());
+// out[j] = unscaled_rms(x[idx[j]]).
 hipError_t launch_compact_rms(const float *x, const int32_t *idx, float *out, int64_t rows,
-                              int width, float eps, int *flag, hipStream_t s,
-                              float out_scale = 0.f);
+                              int width, float eps, int *flag, hipStream_t s);
 
 // ---- log-mel front end ---------------------------------------------------------
 // One clip of packed 16 kHz samples: samples [sample_base, sample_base +

@@ -118,6 +118,40 @@ def test_config_au_two_layers_matches_oracle(au2):
         check(g_.pooled(), o["pooled"], f"config AU clip {i} soft tokens")
 
 
+def test_channel_gains_that_cancel_leave_the_bits(au2):
+    """A norm weight times 2^k and the same column of the projections that read
+    it times 2^-k is the same function, and in 32-bit operands and sums every
+    product is the same number (the clamps in between are opened): the tower's
+    outputs are equal bit for bit, however far a channel stands out."""
+    c, w, _, _ = au2
+    w = dict(w)
+    for l in range(2):
+        p = f"audio_tower.layers.{l}."
+        for name in ("feed_forward1.ffw_layer_1", "feed_forward2.ffw_layer_1", "self_attn.q_proj",
+                     "self_attn.k_proj", "self_attn.v_proj", "lconv1d.linear_start"):
+            w[f"{p}{name}.input_min"] = np.full_like(w[f"{p}{name}.input_min"], -1e30)
+            w[f"{p}{name}.input_max"] = np.full_like(w[f"{p}{name}.input_max"], 1e30)
+    gained = dict(w)
+    for l in range(2):
+        p = f"audio_tower.layers.{l}."
+        for i, (norm, readers) in enumerate((
+                ("feed_forward1.pre_layer_norm", ["feed_forward1.ffw_layer_1"]),
+                ("norm_pre_attn", [f"self_attn.{x}_proj" for x in "qkv"]),
+                ("lconv1d.pre_layer_norm", ["lconv1d.linear_start"]),
+                ("feed_forward2.pre_layer_norm", ["feed_forward2.ffw_layer_1"]))):
+            gain = np.ones(w[f"{p}{norm}.weight"].shape, np.float32)
+            gain[[3 + i, 500 + l, 1023]] = [2.0 ** 20, 2.0 ** 12, 2.0 ** -14]
+            gained[f"{p}{norm}.weight"] = w[f"{p}{norm}.weight"] * gain
+            for r in readers:
+                gained[f"{p}{r}.linear.weight"] = w[f"{p}{r}.linear.weight"] / gain
+    ac = A.AudioConfig.from_json_value(c)
+    mels = _masked_clips()
+    want = A.AudioModel(ac, w, 768).forward_batch(mels)
+    got = A.AudioModel(ac, gained, 768).forward_batch(mels)
+    for a, b in zip(got, want):
+        assert np.array_equal(a.pooled(), b.pooled())
+
+
 def test_batch_and_device_paths_are_bit_identical(au2):
     import torch
     c, w, gpu, om = au2
