@@ -126,6 +126,10 @@ __device__ __forceinline__ float sigmoid_ref(float v) {
 // rows are unchanged): the eight values a GEMM lane's accumulators hold.
 // Scales are powers of two that keep every |x * scale| at most 2^14 or so:
 // halves reach 65504, and the low half's last bit is 2^-24, 2^-38 of that.
+// Values within 2^-16 of that keep 22 bits, smaller ones an error of 2^-25:
+// operands of known bounds (norm outputs, activations) have one scale per
+// channel, undone in the columns of the weight that reads them, others (hidden
+// rows, patches, weights) one per row from its largest value.
 __device__ __forceinline__ void split4(const f32x4 v, f16x4 &hi, f16x4 &lo) {
     hi = __builtin_convertvector(v, f16x4);
     lo = __builtin_convertvector(v - __builtin_convertvector(hi, f32x4), f16x4);

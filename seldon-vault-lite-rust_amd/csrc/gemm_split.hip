@@ -304,8 +304,7 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
         const int m = mw + 16 * i + lr;
         if (m >= M) continue;
         float *crow = p.C + (int64_t)m * p.ldc;
-        // split outputs: the row's scale (1 / rs for rows with their own)
-        const float os = SOUT ? (p.rs ? p.out_scale / rs[i] : p.out_scale) : 1.f;
+        const float row_scale = 1.f / rs[i];  // of a GELU_MUL output (a power of two)
         if constexpr (PAIRED) {
 #pragma unroll
             for (int b = 0; b < NBLK; ++b) {
@@ -314,17 +313,16 @@ __global__ __launch_bounds__(64 * WMW * WNW, MINB) void gemm_split(GemmArgs p, i
 #pragma unroll
                 for (int r = 0; r < 4; ++r) o[r] = gelu_tanh(x[r]) * y[r];
                 const int n = nw / 2 + 16 * b + 4 * lc;  // output columns n .. n + 3
-                if (n < limit) split_store4(crow, n, o * os);
+                if (n < limit) split_store4(crow, n, o);
             }
         } else {
             // block j with its epilogue applied, columns col(j) .. + 3
             auto out = [&](int j) {
                 f32x4 v = value(i, j);
+                if constexpr (EPI == EPI_GELU_MUL) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float x = v[r];
-                    if constexpr (EPI == EPI_GELU_MUL) x = gelu_tanh(x) * aux[i][j][r];
-                    v[r] = SOUT ? x * os : x;
+                    for (int r = 0; r < 4; ++r)
+                        v[r] = gelu_tanh(v[r]) * aux[i][j][r] * row_scale;
                 }
                 return v;
             };
@@ -439,29 +437,53 @@ hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s) {
 
 // ---- split rows -----------------------------------------------------------------
 
-// One wave per row: x [rows, K] to split rows of K_pad (a multiple of 32,
-// zeros past K), each scaled by the power of two that brings its largest
-// magnitude into [2^13, 2^14); descale[row] is the inverse, times `also`.
-// `out` may be x itself (K_pad == ldx): a wave reads the 256 values of a pass
-// before it stores their blocks.
-__global__ __launch_bounds__(256) void split_rows_kernel(const float *x, int64_t ldx, int64_t rows,
-                                                         int K, int K_pad, float also, float *out,
-                                                         float *__restrict__ descale) {
+// One wave per row of w [rows, K], in place: the row times `cols`, scaled by the
+// power of two that brings its largest magnitude into [2^13, 2^14). A wave
+// reads the 256 values of a pass before it stores their blocks.
+//
+// A value scaled to 2^-2 or more keeps 22 bits; below that its low half ends in
+// the half's denormals, 2^-25 being its error whatever its size. The flag is
+// raised where that holds for more than a quarter of a row's nonzero values (a
+// spread of 2^16 between most of the row and its largest value; a few small
+// values beside many large ones lose nothing a sum would show), or where the
+// largest lies outside what the scale's range brings there.
+__global__ __launch_bounds__(256) void split_rows_kernel(float *w, int64_t rows, int K,
+                                                         const float *__restrict__ cols, float also,
+                                                         const float *__restrict__ row_mul,
+                                                         float *__restrict__ descale, int *flag) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
-    const float *xr = x + row * ldx;
+    float *wr = w + row * K;
     float mx = 0.f;
-    for (int k = lane; k < K; k += 64) mx = fmaxf(mx, fabsf(xr[k]));
-    const float sc = split_scale_of(wave_max(mx));
-    float *orow = out + row * K_pad;
-    for (int k = 4 * lane; k < K_pad; k += 256) {
-        f32x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = k + r < K ? xr[k + r] : 0.f;
-        split_store4(orow, k, v * sc);
+    bool finite = true;
+    for (int k = lane; k < K; k += 64) {
+        const float v = cols ? wr[k] * cols[k] : wr[k];
+        finite = finite && isfinite(v);
+        mx = fmaxf(mx, fabsf(v));
     }
-    if (lane == 0) descale[row] = also / sc;
+    mx = wave_max(mx);
+    const float sc = split_scale_of(mx);
+    int small = 0, some = 0;
+    for (int k = 4 * lane; k < K; k += 256) {
+        f32x4 v = *(const f32x4 *)(wr + k);
+        if (cols) v = v * *(const f32x4 *)(cols + k);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[r] *= sc;
+            some += v[r] != 0.f;
+            small += v[r] != 0.f && fabsf(v[r]) < 0.25f;
+        }
+        split_store4(wr, k, v);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        some += __shfl_xor(some, o);
+        small += __shfl_xor(small, o);
+    }
+    const bool scaled = mx == 0.f || (mx * sc >= 8192.f && mx * sc < 16384.f);
+    if (!finite || !scaled || 4 * small > some) raise_flag(flag, 1);
+    if (lane == 0) descale[row] = (row_mul ? also * row_mul[row] : also) / sc;
 }
 
 // One wave per row; the squares are summed in double (no overflow or underflow
@@ -490,11 +512,12 @@ hipError_t launch_row_bounds(const float *x, int64_t rows, int K, const float *w
     return hipGetLastError();
 }
 
-hipError_t launch_split_rows(const float *x, int64_t ldx, int64_t rows, int K, int K_pad,
-                             float also, float *out, float *descale, hipStream_t s) {
+hipError_t launch_split_rows(float *w, int64_t rows, int K, const float *cols, float also,
+                             const float *row_mul, float *descale, int *flag, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x, ldx,
-                       rows, K, K_pad, also, out, descale);
+    if (K % 32 || (uintptr_t)w % 16 || (uintptr_t)cols % 16) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, w, rows,
+                       K, cols, also, row_mul, descale, flag);
     return hipGetLastError();
 }
 

@@ -193,74 +193,178 @@ inline float split_scale(double bound) {
     return std::ldexp(1.f, std::max(-100, std::min(100, 14 - e)));
 }
 
-// Largest magnitude of RMSNorm(x) * w over rows of w.size() values: each
-// normalised value is at most sqrt(n) (w empty: unscaled, n = width).
-inline double norm_bound(const std::vector<float> &w) {
+// True where split_scale does bring it there (or there is nothing to bring).
+inline bool split_scalable(double bound) {
+    return bound == 0 || (bound >= std::ldexp(1.0, -80) && bound <= std::ldexp(1.0, 80));
+}
+
+// One scale per channel of a split operand, from a bound on each channel's
+// magnitude. A channel that stands out would otherwise set the scale of all,
+// and the others' low halves would end in the half's denormals. The inverse
+// scales go into the columns of the weight that reads the operand (0 for a
+// channel that is always zero).
+struct ChannelScales {
+    std::vector<float> scale, inverse;
+    bool ok = true;
+    explicit ChannelScales(const std::vector<double> &bounds) {
+        for (double b : bounds) {
+            ok = ok && split_scalable(b);
+            scale.push_back(split_scale(b));
+            inverse.push_back(b > 0 ? 1.f / scale.back() : 0.f);
+        }
+    }
+};
+
+// Largest magnitude of each channel of RMSNorm(x) * w: a normalised value is at
+// most sqrt(n).
+inline std::vector<double> norm_bounds(const std::vector<float> &w) {
+    std::vector<double> b;
+    for (float v : w) b.push_back(std::sqrt((double)w.size()) * std::fabs((double)v));
+    return b;
+}
+
+template <class T>
+inline double largest(const std::vector<T> &v) {
     double mx = 0;
-    for (float v : w) mx = std::max(mx, (double)std::fabs(v));
-    return std::sqrt((double)w.size()) * mx;
-}
-
-// A weight [rows, K] (K % 32 == 0) in device memory, still FP32, with room for
-// the descale of each row behind it (K % 32 == 0 keeps it aligned).
-inline svl_status upload_rows(std::vector<float *> &owned, const float *host, int64_t rows,
-                              int64_t K, float **w, float **wd) {
-    const size_t count = (size_t)(rows * K);
-    float *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, (count + (size_t)std::max<int64_t>(rows, 1)) * sizeof(float)));
-    owned.push_back(d);
-    HIP_TRY(hipMemcpy(d, host, count * sizeof(float), hipMemcpyHostToDevice));
-    *w = d;
-    *wd = d + count;
-    return SVL_OK;
-}
-
-// Its rows become split rows in place, with the per-output descale of its
-// GEMM: factor / (row scale * a_scale), a_scale the A operand's scale. On the
-// null stream; the caller waits for it before other streams read them.
-inline svl_status split_weight(float *w, int64_t rows, int64_t K, float a_scale, float *wd,
-                               float factor = 1.f) {
-    HIP_TRY(launch_split_rows(w, K, rows, (int)K, (int)K, factor / a_scale, w, wd, nullptr));
-    return SVL_OK;
-}
-
-inline svl_status upload_split(std::vector<float *> &owned, const float *host, int64_t rows,
-                               int64_t K, float a_scale, float **w, float **wd,
-                               float factor = 1.f) {
-    ST_TRY(upload_rows(owned, host, rows, K, w, wd));
-    return split_weight(*w, rows, K, a_scale, *wd, factor);
-}
-
-// Largest |RMSNorm(x) * norm . row| of each row of an uploaded FP32 weight
-// (Cauchy-Schwarz: sqrt(K) * |norm o row|; norm null: K-vectors of norm
-// sqrt(K)). `scratch`: rows floats on the device (the weight's descales).
-inline svl_status product_bounds(const float *w, int64_t rows, int64_t K, const float *norm,
-                                 float *scratch, std::vector<float> &each) {
-    each.resize((size_t)rows);
-    HIP_TRY(launch_row_bounds(w, rows, (int)K, norm, scratch, nullptr));
-    HIP_TRY(hipMemcpy(each.data(), scratch, (size_t)rows * sizeof(float), hipMemcpyDeviceToHost));
-    return SVL_OK;
-}
-
-inline double largest(const std::vector<float> &v) {
-    double mx = 0;
-    for (float x : v) mx = std::max(mx, (double)x);
+    for (T x : v) mx = std::max(mx, (double)x);
     return mx;
 }
 
-// Largest |gelu(g) u| (at most |g| |u|) of a fused gate/up weight [2 I, K]
-// (16-row blocks) over RMSNorm(x) * norm.
-inline svl_status geglu_bound(const float *w, int64_t I, int64_t K, const float *norm,
-                              float *scratch, double *bound) {
-    std::vector<float> b;
-    ST_TRY(product_bounds(w, 2 * I, K, norm, scratch, b));
-    *bound = 0;
-    for (int64_t j = 0; j < I; ++j) {
-        const size_t at = (size_t)(32 * (j / 16) + j % 16);
-        *bound = std::max(*bound, (double)b[at] * (double)b[at + 16]);
-    }
-    return SVL_OK;
+// Query and key norm weights of a head, rotated in pairs (i, i + group / 2) of
+// each `group` values: powers of two move between them so that both sides of a
+// pair's products have like bounds (the products, and so the scores, stay the
+// same numbers). False if the pairs' products still differ so much that more
+// than a quarter would lose bits beside the largest (2^11 below it on each
+// side, where a normalised value of 1 is scaled to about 2^-2).
+inline bool balance_heads(std::vector<float> &qn, std::vector<float> &kn, size_t group) {
+    std::vector<double> size;
+    const size_t half = group / 2;
+    for (size_t g = 0; g + group <= qn.size(); g += group)
+        for (size_t i = g; i < g + half; ++i) {
+            const float q = std::max(std::fabs(qn[i]), std::fabs(qn[i + half])),
+                        k = std::max(std::fabs(kn[i]), std::fabs(kn[i + half]));
+            if (q == 0.f || k == 0.f) {  // products of zero
+                qn[i] = qn[i + half] = kn[i] = kn[i + half] = 0.f;
+                continue;
+            }
+            if (!split_scalable(q) || !split_scalable(k)) return false;
+            const int e = (std::ilogb(k) - std::ilogb(q)) >> 1;
+            for (size_t j : {i, i + half}) {
+                qn[j] = std::ldexp(qn[j], e);
+                kn[j] = std::ldexp(kn[j], -e);
+            }
+            size.push_back(std::max(std::ldexp((double)q, e), std::ldexp((double)k, -e)));
+        }
+    const double least = std::ldexp(largest(size), -11);
+    const int64_t small = std::count_if(size.begin(), size.end(), [&](double v) { return v < least; });
+    return 4 * small <= (int64_t)size.size();
 }
+
+// Brings a model's projection weights to the device as split rows while the
+// model is created (on the null stream; finish() waits). `fits` ends false when
+// the halves would hold some operand in fewer bits than they should
+// (split_rows_kernel and the bounds above say when): such a model is created
+// again on FP32 operands.
+struct SplitLoader {
+    std::vector<float *> &owned;
+    DevBuf<float> cols, mul;
+    DevBuf<int> flag;
+    bool fits = true;
+
+    explicit SplitLoader(std::vector<float *> &o) : owned(o) {}
+    SplitLoader(const SplitLoader &) = delete;
+    ~SplitLoader() {
+        cols.release();
+        mul.release();
+        flag.release();
+    }
+
+    svl_status put(DevBuf<float> &to, const std::vector<float> &v) {
+        HIP_TRY(to.ensure(v.size()));
+        HIP_TRY(hipMemcpy(to.p, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice));
+        return SVL_OK;
+    }
+
+    // A weight [rows, K] (K % 32 == 0), still FP32, with room for the descale
+    // of each row behind it (K % 32 == 0 keeps it aligned).
+    svl_status upload(const float *host, int64_t rows, int64_t K, float **w, float **wd) {
+        const size_t count = (size_t)(rows * K);
+        float *d = nullptr;
+        HIP_TRY(hipMalloc((void **)&d, (count + (size_t)std::max<int64_t>(rows, 1)) * sizeof(float)));
+        owned.push_back(d);
+        HIP_TRY(hipMemcpy(d, host, count * sizeof(float), hipMemcpyHostToDevice));
+        *w = d;
+        *wd = d + count;
+        return SVL_OK;
+    }
+
+    // Largest |RMSNorm(x) * norm . row| of each row of an uploaded FP32 weight
+    // (Cauchy-Schwarz: sqrt(K) * |norm o row|; norm null: K-vectors of norm
+    // sqrt(K)). `scratch`: rows floats on the device (the weight's descales).
+    svl_status bounds(const float *w, int64_t rows, int64_t K, const std::vector<float> *norm,
+                      float *scratch, std::vector<float> &each) {
+        each.resize((size_t)rows);
+        if (norm) ST_TRY(put(cols, *norm));
+        HIP_TRY(launch_row_bounds(w, rows, (int)K, norm ? cols.p : nullptr, scratch, nullptr));
+        HIP_TRY(hipMemcpy(each.data(), scratch, (size_t)rows * sizeof(float), hipMemcpyDeviceToHost));
+        return SVL_OK;
+    }
+
+    // An uploaded weight to split rows in place, its columns times a's inverse
+    // scales first (null: an A operand of one scale, a_scale); wd = the descale
+    // of each output of its GEMM, times factor and row_mul[row].
+    svl_status convert(float *w, int64_t rows, int64_t K, float a_scale, const ChannelScales *a,
+                       float *wd, float factor = 1.f, const std::vector<float> *row_mul = nullptr) {
+        if (!flag.p) {
+            const int zero = 0;
+            HIP_TRY(flag.ensure(1));
+            HIP_TRY(hipMemcpy(flag.p, &zero, sizeof zero, hipMemcpyHostToDevice));
+        }
+        if (a) {
+            fits = fits && a->ok;
+            ST_TRY(put(cols, a->inverse));
+        }
+        if (row_mul) ST_TRY(put(mul, *row_mul));
+        HIP_TRY(launch_split_rows(w, rows, (int)K, a ? cols.p : nullptr, factor / a_scale,
+                                  row_mul ? mul.p : nullptr, wd, flag.p, nullptr));
+        return SVL_OK;
+    }
+
+    svl_status weight(const std::vector<float> &host, int64_t K, float a_scale,
+                      const ChannelScales *a, float **w, float **wd, float factor = 1.f) {
+        const int64_t rows = (int64_t)host.size() / K;
+        ST_TRY(upload(host.data(), rows, K, w, wd));
+        return convert(*w, rows, K, a_scale, a, *wd, factor);
+    }
+
+    // A fused gate/up weight [2 I, K] (16-row blocks) over RMSNorm(x) * norm,
+    // whose channels carry `in`: one scale per activation channel, |gelu(g) u|
+    // being at most |g| |u|, applied by the up rows' descale.
+    svl_status geglu(const std::vector<float> &gu, int64_t I, int64_t K,
+                     const std::vector<float> &norm, const ChannelScales &in, float **w, float **wd,
+                     std::vector<double> &act) {
+        std::vector<float> b;
+        ST_TRY(upload(gu.data(), 2 * I, K, w, wd));
+        ST_TRY(bounds(*w, 2 * I, K, &norm, *wd, b));
+        act.clear();
+        std::vector<float> row_mul((size_t)(2 * I), 1.f);
+        for (int64_t j = 0; j < I; ++j) {
+            const size_t at = (size_t)(32 * (j / 16) + j % 16);
+            act.push_back((double)b[at] * (double)b[at + 16]);
+            fits = fits && split_scalable(b[at]) && split_scalable(b[at + 16]);
+            row_mul[at + 16] = split_scale(act.back());
+        }
+        return convert(*w, 2 * I, K, 1.f, &in, *wd, 1.f, &row_mul);
+    }
+
+    svl_status finish(bool *ok) {
+        int raised = 0;
+        HIP_TRY(hipStreamSynchronize(nullptr));
+        if (flag.p) HIP_TRY(hipMemcpy(&raised, flag.p, sizeof(int), hipMemcpyDeviceToHost));
+        *ok = fits && raised == 0;
+        return SVL_OK;
+    }
+};
 
 // Gate and up projections [I, H] interleaved in blocks of `block` rows
 // [g 0 .. block - 1, u 0 .. block - 1, g block .., ...], padded to I_pad rows

@@ -61,12 +61,14 @@ template <int NC>
 __global__ __launch_bounds__(256) void rms_rows_kernel(const float *__restrict__ x,
                                                        const float *__restrict__ w,
                                                        float *__restrict__ out, int64_t rows,
-                                                       int width, float eps, int *flag) {
+                                                       int width, float eps, int *flag,
+                                                       int w_rows) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
     const int nv = width >> 2;
     const f32x4 *xr = (const f32x4 *)(x + row * width);
+    if (w_rows > 1) w += (int64_t)((uint32_t)row % (uint32_t)w_rows) * width;
     // the row and the weights loaded together (chunks past the width load
     // its last chunk and take no part)
     f32x4 v[NC], wv[NC];
@@ -103,11 +105,12 @@ __global__ __launch_bounds__(256) void rms_rows_generic_kernel(const float *__re
                                                                const float *__restrict__ w,
                                                                float *__restrict__ out,
                                                                int64_t rows, int width, float eps,
-                                                               int *flag) {
+                                                               int *flag, int w_rows) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
     const float *xr = x + row * width;
+    if (w_rows > 1) w += (int64_t)((uint32_t)row % (uint32_t)w_rows) * width;
     float ss = 0.f;
     for (int i = lane; i < width; i += 64) ss += xr[i] * xr[i];
     ss = wave_sum(ss);
@@ -123,18 +126,19 @@ __global__ __launch_bounds__(256) void rms_rows_generic_kernel(const float *__re
 }
 
 hipError_t launch_rms_rows(const float *x, const float *w, float *out, int64_t rows, int width,
-                           float eps, int *flag, hipStream_t s) {
+                           float eps, int *flag, hipStream_t s, int w_rows) {
     if (rows <= 0) return hipSuccess;
+    if (w_rows > 1 && (!w || rows > UINT32_MAX)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((rows + 3) / 4));
     const bool vec = width > 0 && width % 4 == 0 && width <= 256 * ROW_CHUNKS &&
                      (uintptr_t)x % 16 == 0 &&
                      (uintptr_t)out % 16 == 0 && (!w || (uintptr_t)w % 16 == 0);
     if (vec) {
         SVL_DISPATCH_NC((width + 255) / 256, rms_rows_kernel, grid, s, x, w, out, rows, width, eps,
-                        flag);
+                        flag, w_rows);
     } else
         hipLaunchKernelGGL(rms_rows_generic_kernel, grid, dim3(256), 0, s, x, w, out, rows, width,
-                           eps, flag);
+                           eps, flag, w_rows);
     return hipGetLastError();
 }
 

@@ -72,12 +72,13 @@ struct DevLayer {
           *ln_post_ple = nullptr, *q_norm = nullptr, *k_norm = nullptr;
     float scalar = 1.f;
     int hd = 0, nkv = 0, full = 0;
-    // split models: descale of each projection's outputs, and the scales of
-    // its split operands (norm outputs, attention output, GeGLU and PLE
-    // activations)
+    // split models: descale of each projection's outputs and the attention
+    // output's scale (the norm weights, d_gu and ple_norm carry the scales of
+    // the norm outputs', the GeGLU and the PLE activation's channels, the
+    // weights that read them the inverses)
     float *d_qkv = nullptr, *d_o = nullptr, *d_gu = nullptr, *d_down = nullptr, *d_pg = nullptr,
           *d_pp = nullptr;
-    float s_in = 0.f, s_ff = 0.f, s_attn = 0.f, s_act = 1.f, s_pg = 1.f;
+    float s_attn = 0.f;
     QkvSplit s_heads;  // of the normalised and rotated Q, K and V rows
 };
 
@@ -103,10 +104,10 @@ struct svl_text_model {
     float embedding_scale = 1.f, ple_scale = 1.f;
     int64_t I_pad = 0;
     // Every projection runs on split operands (gemm_split.hip): the widths are
-    // multiples of 32. Other models take the FP32 GEMMs.
+    // multiples of 32 and the weights fit them (SplitLoader). Other models take
+    // the FP32 GEMMs.
     bool split = false;
     float *d_out_proj = nullptr, *d_ple_model = nullptr;
-    float s_final = 0.f;
     std::vector<DevLayer> layers;
     std::vector<float *> allocations;
     float *embed = nullptr, *out_proj = nullptr, *final_norm = nullptr, *ple_model = nullptr,
@@ -532,6 +533,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     // split models: the split copy of h that the PLE projections read
     const SplitRows hs = m->split ? SplitRows{attn, m->rs.p + t0} : SplitRows();
     const float *h_in = m->split ? attn : h, *h_rs = hs.descale;
+    const float split_n = m->split ? 1.f : 0.f;  // norm outputs as split rows
 
     HIP_TRY(launch_positions(offs, grp.nrows, pos, rowlen, s));
     {
@@ -539,7 +541,7 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         HIP_TRY(launch_gather(d_ids + t0, m->embed, m->V, d_featmap ? d_featmap + t0 : nullptr,
                               d_feats, m->embedding_scale,
                               m->layers[0].ln_in, h, n, T, (int)H, m->eps, flag, s,
-                              m->layers[0].s_in, hs));
+                              split_n, hs));
     }
     if (h_hidden)
         HIP_TRY(hipMemcpyAsync(h_hidden + t0 * H, h, (size_t)(T * H) * 4, hipMemcpyDeviceToHost,
@@ -558,7 +560,8 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
     }
     {
         Timer tm(m, s, KC_PLE_NORM, Td * L * P * 8);
-        HIP_TRY(launch_rms_rows(ple, m->ple_norm, ple, T * L, (int)P, m->eps, flag, s));
+        HIP_TRY(launch_rms_rows(ple, m->ple_norm, ple, T * L, (int)P, m->eps, flag, s,
+                                m->split ? (int)L : 1));
     }
 
     for (int64_t l = 0; l < L; ++l) {
@@ -623,14 +626,13 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         {
             Timer tm(m, s, KC_RESNORM, Td * H * 4 * 4);
             HIP_TRY(launch_resnorm(tmp, ly.ln_post_attn, h, h, ly.ln_pre_ff, n, 1.0f, T, (int)H,
-                                   m->eps, flag, s, ly.s_ff));
+                                   m->eps, flag, s, split_n));
         }
         {
             GemmArgs g{n, H, ly.w_gu, H, act, m->I, (int)T, (int)(2 * m->I_pad), (int)H, EPI_GEGLU,
                        1.f, nullptr, 0, (int)m->I};
             g.cus = cus;
             g.wd = ly.d_gu;
-            g.out_scale = ly.s_act;
             Timer tm(m, s, KC_GEMM_GATE_UP, 2.0 * Td * H * 2 * m->I);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -653,7 +655,6 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
             g.cus = cus;
             g.wd = ly.d_pg;
             g.rs = h_rs;
-            g.out_scale = ly.s_pg;
             Timer tm(m, s, KC_GEMM_PLE_GATE, 2.0 * Td * H * P);
             HIP_TRY(launch_gemm(g, s));
         }
@@ -668,10 +669,9 @@ svl_status enqueue_group(svl_text_model *m, const Batch &b, const Group &grp, hi
         }
         {
             const float *next = l + 1 < L ? m->layers[(size_t)l + 1].ln_in : m->final_norm;
-            const float s_next = l + 1 < L ? m->layers[(size_t)l + 1].s_in : m->s_final;
             Timer tm(m, s, KC_RESNORM, Td * H * 4 * 4);
             HIP_TRY(launch_resnorm(tmp, ly.ln_post_ple, h, h, next, n, ly.scalar, T, (int)H,
-                                   m->eps, flag, s, s_next));
+                                   m->eps, flag, s, split_n));
         }
         if (h_hidden)
             HIP_TRY(hipMemcpyAsync(h_hidden + (size_t)((l + 1) * T_all * H + t0 * H), h,
@@ -1003,9 +1003,9 @@ svl_status svl_shutdown(svl_ctx *ctx) {
 
 const char *svl_last_error(void) { return g_err.c_str(); }
 
-svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
-                                 const svl_tensor_view *tensors, size_t n_tensors,
-                                 svl_text_model **out) {
+static svl_status create_text(svl_ctx *ctx, const svl_text_config *cfg,
+                              const svl_tensor_view *tensors, size_t n_tensors, bool allow_split,
+                              bool *fits, svl_text_model **out) {
     if (!ctx || !out) return fail(SVL_USAGE, "context or output pointer is null");
     ST_TRY(validate_config(cfg));
     HIP_TRY(hipSetDevice(ctx->device));
@@ -1044,31 +1044,39 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
     auto get = [&](const std::string &name, std::vector<float> &buf) -> svl_status {
         return decode_named(by_name, name, buf);
     };
-    m->split = m->H % 32 == 0 && m->I % 32 == 0 && m->P % 32 == 0;
+    m->split = allow_split && m->H % 32 == 0 && m->I % 32 == 0 && m->P % 32 == 0;
     for (int64_t l = 0; l < m->L; ++l)
         m->split = m->split && (m->NH * cfg->head_dim[l]) % 32 == 0;
-    // A projection weight [rows, K], for an A operand scaled by a_scale.
-    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, float **dst,
-                   float **descale, float factor = 1.f) -> svl_status {
+    SplitLoader load(m->allocations);
+    // A projection weight [rows, K], for an A operand of one scale or of one
+    // per channel.
+    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, const ChannelScales *a,
+                   float **dst, float **descale, float factor = 1.f) -> svl_status {
         if (!m->split) return upload(m, w.data(), w.size(), dst);
-        return upload_split(m->allocations, w.data(), (int64_t)w.size() / K, K, a_scale, dst,
-                            descale, factor);
+        return load.weight(w, K, a_scale, a, dst, descale, factor);
+    };
+    // A norm weight whose outputs are a projection's operand: it carries their
+    // scales.
+    auto put_norm = [&](const std::vector<float> &w, const ChannelScales &c, float **dst) {
+        std::vector<float> v(w);
+        for (size_t i = 0; m->split && i < v.size(); ++i) v[i] *= c.scale[i];
+        return upload(m, v.data(), v.size(), dst);
     };
     std::vector<float> a, b2, c2, nw;
     ST_TRY(get("language_model.embed_tokens.weight", a));
     ST_TRY(upload(m, a.data(), a.size(), &m->embed));
-    ST_TRY(get("language_model.norm.weight", a));
-    ST_TRY(upload(m, a.data(), a.size(), &m->final_norm));
-    if (m->split) m->s_final = split_scale(norm_bound(a));
+    ST_TRY(get("language_model.norm.weight", nw));
+    const ChannelScales c_final(norm_bounds(nw));
+    ST_TRY(put_norm(nw, c_final, &m->final_norm));
     ST_TRY(get("language_model.embedding_projection.weight", a));
-    ST_TRY(put(a, m->H, m->s_final, &m->out_proj, &m->d_out_proj));
+    ST_TRY(put(a, m->H, 1.f, &c_final, &m->out_proj, &m->d_out_proj));
     // the hidden rows carry scales of their own (SplitRows); the descale also
     // applies the projection's 1 / sqrt(H)
     ST_TRY(get("language_model.ple.per_layer_model_projection.weight", a));
-    ST_TRY(put(a, m->H, 1.f, &m->ple_model, &m->d_ple_model, m->ple_scale));
-    ST_TRY(get("language_model.ple.per_layer_projection_norm.weight", a));
-    ST_TRY(upload(m, a.data(), a.size(), &m->ple_norm));
-    const double ple_bound = norm_bound(a);
+    ST_TRY(put(a, m->H, 1.f, nullptr, &m->ple_model, &m->d_ple_model, m->ple_scale));
+    std::vector<float> ple_norm, ple_norms;  // split models: [L, P] with the layers' scales
+    ST_TRY(get("language_model.ple.per_layer_projection_norm.weight", ple_norm));
+    const std::vector<double> ple_bounds = norm_bounds(ple_norm);
 
     m->layers.resize((size_t)m->L);
     for (int64_t l = 0; l < m->L; ++l) {
@@ -1082,76 +1090,83 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
         struct {
             const char *name;
             float **dst;
-        } norms[] = {{"input_layernorm.weight", &ly.ln_in},
-                     {"post_attention_layernorm.weight", &ly.ln_post_attn},
-                     {"pre_feedforward_layernorm.weight", &ly.ln_pre_ff},
+        } norms[] = {{"post_attention_layernorm.weight", &ly.ln_post_attn},
                      {"post_feedforward_layernorm.weight", &ly.ln_post_ff},
-                     {"ple_block.post_per_layer_input_norm.weight", &ly.ln_post_ple},
-                     {"self_attn.q_norm.weight", &ly.q_norm},
-                     {"self_attn.k_norm.weight", &ly.k_norm}};
+                     {"ple_block.post_per_layer_input_norm.weight", &ly.ln_post_ple}};
         for (auto &nm : norms) {
             ST_TRY(get(p + nm.name, a));
             ST_TRY(upload(m, a.data(), a.size(), nm.dst));
         }
+        ST_TRY(get(p + "input_layernorm.weight", nw));
+        const ChannelScales c_in(norm_bounds(nw));
+        ST_TRY(put_norm(nw, c_in, &ly.ln_in));
         // fused QKV weight: rows [q; k; v]
         std::vector<float> qkv((size_t)((qd + 2 * kd) * H));
-        ST_TRY(get(p + "input_layernorm.weight", nw));
-        if (m->split) ly.s_in = split_scale(norm_bound(nw));
         ST_TRY(get(p + "self_attn.q_proj.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin());
         ST_TRY(get(p + "self_attn.k_proj.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + qd * H);
         ST_TRY(get(p + "self_attn.v_proj.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + (qd + kd) * H);
-        ST_TRY(put(qkv, H, ly.s_in, &ly.w_qkv, &ly.d_qkv));
-        // attention outputs are convex sums of RMS-normalised value rows
-        if (m->split) ly.s_attn = split_scale(std::sqrt((double)ly.hd));
+        ST_TRY(put(qkv, H, 1.f, &c_in, &ly.w_qkv, &ly.d_qkv));
+        ST_TRY(get(p + "self_attn.q_norm.weight", b2));
+        ST_TRY(get(p + "self_attn.k_norm.weight", c2));
         if (m->split) {
+            // attention outputs are convex sums of RMS-normalised value rows
+            ly.s_attn = split_scale(std::sqrt((double)ly.hd));
             // a rotated row's values are at most the row's norm; scale 1.0
             // (text.rs:421) times log2(e) for scores in log2 units
-            ST_TRY(get(p + "self_attn.q_norm.weight", nw));
+            load.fits = load.fits && balance_heads(b2, c2, b2.size());
             ly.s_heads.q_mul = 1.4426950408889634f;
-            ly.s_heads.q = split_scale(norm_bound(nw) * ly.s_heads.q_mul);
-            ST_TRY(get(p + "self_attn.k_norm.weight", nw));
-            ly.s_heads.k = split_scale(norm_bound(nw));
+            ly.s_heads.q = split_scale(largest(norm_bounds(b2)) * ly.s_heads.q_mul);
+            ly.s_heads.k = split_scale(largest(norm_bounds(c2)));
             ly.s_heads.v = ly.s_attn;
         }
+        ST_TRY(upload(m, b2.data(), b2.size(), &ly.q_norm));
+        ST_TRY(upload(m, c2.data(), c2.size(), &ly.k_norm));
         ST_TRY(get(p + "self_attn.o_proj.weight", a));
-        ST_TRY(put(a, qd, ly.s_attn, &ly.w_o, &ly.d_o));
+        ST_TRY(put(a, qd, ly.s_attn, nullptr, &ly.w_o, &ly.d_o));
         ST_TRY(get(p + "mlp.gate_proj.weight", b2));
         ST_TRY(get(p + "mlp.up_proj.weight", c2));
         const std::vector<float> gu =
             interleave_gate_up(b2, c2, m->I, m->I_pad, m->H, m->split ? 16 : 32);
-        if (m->split) {
-            ST_TRY(get(p + "pre_feedforward_layernorm.weight", nw));
-            ly.s_ff = split_scale(norm_bound(nw));
-            ST_TRY(upload_rows(m->allocations, gu.data(), 2 * m->I, H, &ly.w_gu, &ly.d_gu));
-            double act;
-            ST_TRY(geglu_bound(ly.w_gu, m->I, H, ly.ln_pre_ff, ly.d_gu, &act));
-            ly.s_act = split_scale(act);
-            ST_TRY(split_weight(ly.w_gu, 2 * m->I, H, ly.s_ff, ly.d_gu));
-        } else {
+        ST_TRY(get(p + "pre_feedforward_layernorm.weight", nw));
+        const ChannelScales c_ff(norm_bounds(nw));
+        ST_TRY(put_norm(nw, c_ff, &ly.ln_pre_ff));
+        std::vector<double> act;
+        if (m->split)
+            ST_TRY(load.geglu(gu, m->I, H, nw, c_ff, &ly.w_gu, &ly.d_gu, act));
+        else
             ST_TRY(upload(m, gu.data(), gu.size(), &ly.w_gu));
-        }
+        const ChannelScales c_act(act);
         ST_TRY(get(p + "mlp.down_proj.weight", a));
-        ST_TRY(put(a, m->I, ly.s_act, &ly.w_down, &ly.d_down));
+        ST_TRY(put(a, m->I, 1.f, &c_act, &ly.w_down, &ly.d_down));
         ST_TRY(get(p + "ple_block.per_layer_input_gate.weight", a));
-        // A hidden row whose scale is 1 / rs has values below 2^14 rs, so its
-        // gates are at most 2^14 rs sqrt(H) |W row|; s_pg / rs brings gate x
-        // per-layer input below 2^14.
+        // A hidden row whose scale is 1 / rs has values below 2^14 rs, so a gate
+        // is at most 2^14 rs sqrt(H) |W row|; its channel's scale over rs brings
+        // gate x per-layer input below 2^14.
+        std::vector<double> gated;
         if (m->split) {
             std::vector<float> b;
-            ST_TRY(upload_rows(m->allocations, a.data(), m->P, H, &ly.w_pg, &ly.d_pg));
-            ST_TRY(product_bounds(ly.w_pg, m->P, H, nullptr, ly.d_pg, b));
-            ly.s_pg = split_scale(16384.0 * largest(b) * ple_bound);
-            ST_TRY(split_weight(ly.w_pg, m->P, H, 1.f, ly.d_pg));
+            ST_TRY(load.upload(a.data(), m->P, H, &ly.w_pg, &ly.d_pg));
+            ST_TRY(load.bounds(ly.w_pg, m->P, H, nullptr, ly.d_pg, b));
+            for (int64_t i = 0; i < m->P; ++i)
+                gated.push_back(16384.0 * b[(size_t)i] * ple_bounds[(size_t)i]);
+            ST_TRY(load.convert(ly.w_pg, m->P, H, 1.f, nullptr, ly.d_pg));
         } else {
             ST_TRY(upload(m, a.data(), a.size(), &ly.w_pg));
         }
+        const ChannelScales c_pg(gated);
+        for (size_t i = 0; m->split && i < ple_norm.size(); ++i)
+            ple_norms.push_back(ple_norm[i] * c_pg.scale[i]);
         ST_TRY(get(p + "ple_block.per_layer_projection.weight", a));
-        ST_TRY(put(a, m->P, ly.s_pg, &ly.w_pp, &ly.d_pp));
+        ST_TRY(put(a, m->P, 1.f, &c_pg, &ly.w_pp, &ly.d_pp));
         ST_TRY(get(p + "layer_scalar", a));
         ly.scalar = a[0];
+    }
+    {
+        const std::vector<float> &pn = m->split ? ple_norms : ple_norm;
+        ST_TRY(upload(m, pn.data(), pn.size(), &m->ple_norm));
     }
 
     // RoPE tables for every position a row may use.
@@ -1172,7 +1187,7 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
     }
     if (m->split) {
         m->max_q = std::max(m->max_q, m->H);
-        HIP_TRY(hipStreamSynchronize(nullptr));  // the weights' conversion
+        ST_TRY(load.finish(fits));
     }
     HIP_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming));
@@ -1183,6 +1198,17 @@ svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
     HIP_TRY(hipHostMalloc((void **)&m->h_flag, sizeof(int), hipHostMallocDefault));
     *out = guard.release();
     return SVL_OK;
+}
+
+svl_status svl_text_model_create(svl_ctx *ctx, const svl_text_config *cfg,
+                                 const svl_tensor_view *tensors, size_t n_tensors,
+                                 svl_text_model **out) {
+    bool fits = true;
+    ST_TRY(create_text(ctx, cfg, tensors, n_tensors, true, &fits, out));
+    if (fits) return SVL_OK;
+    delete *out;  // weights that the split operands would round: FP32 operands
+    *out = nullptr;
+    return create_text(ctx, cfg, tensors, n_tensors, false, &fits, out);
 }
 
 svl_status svl_text_model_destroy(svl_text_model *model) {

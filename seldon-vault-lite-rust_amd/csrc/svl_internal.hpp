@@ -69,7 +69,6 @@ struct GemmArgs {
     // split operands (launch_gemm_split)
     const float *wd = nullptr;  // [N] descale of each output column
     const float *rs = nullptr;  // [M] descale of each A row (null: 1)
-    float out_scale = 1.f;      // scale of a split output
 };
 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t s);
@@ -86,23 +85,27 @@ hipError_t launch_gemm_simple(const GemmArgs &a, hipStream_t s);
 // K % 32 == 0), and every epilogue value is first descaled by wd[n] (and
 // rs[m] where rows carry scales of their own): C = epilogue((A . W^T) *
 // rs[m] * wd[n]). Paired epilogues take W rows interleaved in 16-row blocks.
-// EPI_STORE, and the epilogues whose output only another GEMM reads (GEGLU,
-// GELU_MUL), which store split rows scaled by out_scale (out_scale / rs[m] with
-// row scales; ldc % 32 == 0, the output width a multiple of 32).
+// EPI_STORE, and the epilogues whose output only another GEMM reads, which
+// store split rows (ldc % 32 == 0, the output width a multiple of 32): GEGLU,
+// scaled by what the up rows' descales carry, and GELU_MUL, by what aux carries
+// over rs[m].
 hipError_t launch_gemm_split(const GemmArgs &a, hipStream_t s);
 constexpr int SPLIT_RASTER_M = 8;  // M blocks per rasterization group
-// x [rows, K] (leading dimension ldx) to split rows of K_pad >= K, each
-// scaled by its own power of two; descale[row] = also / scale.
-hipError_t launch_split_rows(const float *x, int64_t ldx, int64_t rows, int K, int K_pad,
-                             float also, float *out, float *descale, hipStream_t s);
+// w [rows, K] (K % 32 == 0) to split rows in place: each value times cols[k]
+// (null: 1), each row scaled by its own power of two; descale[row] = also *
+// row_mul[row] (null: 1) / scale. *flag is set where a row does not fit the
+// halves (split_rows_kernel).
+hipError_t launch_split_rows(float *w, int64_t rows, int K, const float *cols, float also,
+                             const float *row_mul, float *descale, int *flag, hipStream_t s);
 // out[r] >= sqrt(K * sum_k (x[r, k] * w[k])^2) (w == nullptr: ones), at most
 // 0.1 % above it.
 hipError_t launch_row_bounds(const float *x, int64_t rows, int K, const float *w, float *out,
                              hipStream_t s);
 
-// out = rms_norm_rows(x, w) (w == nullptr: unscaled).
+// out = rms_norm_rows(x, w) (w == nullptr: unscaled); w_rows > 1: row r takes
+// row r % w_rows of w [w_rows, width].
 hipError_t launch_rms_rows(const float *x, const float *w, float *out, int64_t rows, int width,
-                           float eps, int *flag, hipStream_t s);
+                           float eps, int *flag, hipStream_t s, int w_rows = 1);
 
 // A row kernel's split copy of its hidden rows: each row scaled by its own
 // power of two (rows == nullptr: none).
@@ -112,7 +115,8 @@ struct SplitRows {
 };
 
 // h_out = (res + rms(x, w1)) * scale ; if w2: n_out = rms(h_out, w2), stored
-// as split rows times n_scale when n_scale > 0. `hs`: split copy of h_out.
+// as split rows times n_scale when n_scale > 0 (1 where w2 carries the scales of
+// its channels). `hs`: split copy of h_out.
 hipError_t launch_resnorm(const float *x, const float *w1, const float *res, float *h_out,
                           const float *w2, float *n_out, float scale, int64_t rows, int width,
                           float eps, int *flag, hipStream_t s, float n_scale = 0.f,

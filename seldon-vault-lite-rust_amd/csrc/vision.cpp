@@ -47,9 +47,10 @@ struct VisLayer {
     float *w_qkv = nullptr, *w_o = nullptr, *w_gu = nullptr, *w_down = nullptr;
     float *ln_in = nullptr, *ln_post_attn = nullptr, *ln_pre_ff = nullptr, *ln_post_ff = nullptr,
           *q_norm = nullptr, *k_norm = nullptr;
-    // split towers: descale of each projection's outputs, scales of its operands
+    // split towers: descale of each projection's outputs (the norm weights and
+    // d_gu carry the scales of the norm outputs' and the GeGLU activation's
+    // channels, the weights that read them the inverses)
     float *d_qkv = nullptr, *d_o = nullptr, *d_gu = nullptr, *d_down = nullptr;
-    float s_in = 0.f, s_ff = 0.f, s_act = 1.f;
     QkvSplit s_heads;  // of the normalised and rotated Q, K and V rows
 };
 
@@ -64,7 +65,8 @@ struct svl_vision_model {
     std::vector<float *> allocations;
     float *w_in = nullptr, *pos_table = nullptr, *w_proj = nullptr;
     // Every projection runs on split operands (gemm_split.hip): the widths are
-    // multiples of 32. Other towers take the FP32 GEMMs.
+    // multiples of 32 and the weights fit them (SplitLoader). Other towers take
+    // the FP32 GEMMs.
     bool split = false;
     float *d_in = nullptr, *d_proj = nullptr;
     float s_attn = 0.f, s_pool = 0.f;
@@ -511,13 +513,12 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
             HIP_TRY(launch_gemm(ga, s));
         }
         HIP_TRY(launch_resnorm(tmp, ly.ln_post_attn, h, h, ly.ln_pre_ff, n, 1.0f, R, (int)H, v->eps,
-                               flag, s, ly.s_ff));
+                               flag, s, v->split ? 1.f : 0.f));
         {
             GemmArgs ga{n, H, ly.w_gu, H, act, v->I, (int)R, (int)(2 * v->I_pad), (int)H, EPI_GEGLU,
                         1.f, nullptr, 0, (int)v->I};
             ga.cus = cus;
             ga.wd = ly.d_gu;
-            ga.out_scale = ly.s_act;
             HIP_TRY(launch_gemm(ga, s));
         }
         {
@@ -529,7 +530,7 @@ svl_status enqueue_vis_layers(svl_vision_model *v, const VisBatch &b, const VisB
         }
         const float *next = l + 1 < v->L ? v->layers[(size_t)l + 1].ln_in : nullptr;
         HIP_TRY(launch_resnorm(tmp, ly.ln_post_ff, h, h, next, next ? n : nullptr, 1.0f, R, (int)H,
-                               v->eps, flag, s, next ? v->layers[(size_t)l + 1].s_in : 0.f));
+                               v->eps, flag, s, next && v->split ? 1.f : 0.f));
         if (h_hidden)
             HIP_TRY(hipMemcpyAsync(h_hidden + (size_t)((l + 1) * Ts * H), v->h.p,
                                    (size_t)(T * H) * 4, hipMemcpyDeviceToHost, s));
@@ -557,7 +558,7 @@ svl_status enqueue_vision(svl_vision_model *v, const VisBatch &b, float *d_pix, 
     }
     // position add fused with layer 0's input norm (the model has >= 1 layer)
     HIP_TRY(launch_patch_pos(v->h.p, v->coord.p, v->pos_table, v->pos_size, v->layers[0].ln_in,
-                             v->n.p, T, (int)H, v->eps, flag, s, v->layers[0].s_in));
+                             v->n.p, T, (int)H, v->eps, flag, s, v->split ? 1.f : 0.f));
     if (h_hidden)
         HIP_TRY(hipMemcpyAsync(h_hidden, v->h.p, (size_t)(T * H) * 4, hipMemcpyDeviceToHost, s));
 
@@ -735,9 +736,9 @@ svl_status image_embed(svl_vision_model *v, svl_text_model *text,
 
 extern "C" {
 
-svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, int64_t text_hidden,
-                                   const svl_tensor_view *tensors, size_t n_tensors,
-                                   svl_vision_model **out) {
+static svl_status create_vision(svl_ctx *ctx, const svl_vision_config *cfg, int64_t text_hidden,
+                                const svl_tensor_view *tensors, size_t n_tensors, bool allow_split,
+                                bool *fits, svl_vision_model **out) {
     if (!ctx || !out) return fail(SVL_USAGE, "context or output pointer is null");
     ST_TRY(validate_vision_config(cfg, text_hidden));
     const int device = ctx->device;
@@ -776,18 +777,26 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         v->inv_freq.push_back(value);
     }
 
-    v->split = v->H % 32 == 0 && v->I % 32 == 0 && v->qd % 32 == 0;
+    v->split = allow_split && v->H % 32 == 0 && v->I % 32 == 0 && v->qd % 32 == 0;
+    SplitLoader load(v->allocations);
     std::vector<float> a, b2, c2, nw;
     auto up = [&](const std::string &name, float **dst) -> svl_status {
         ST_TRY(decode_named(by_name, name, a));
         return upload_owned(v->allocations, a.data(), a.size(), dst);
     };
-    // A projection weight [rows, K], for an A operand scaled by a_scale.
-    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, float **dst,
-                   float **descale) -> svl_status {
+    // A projection weight [rows, K], for an A operand of one scale or of one
+    // per channel.
+    auto put = [&](const std::vector<float> &w, int64_t K, float a_scale, const ChannelScales *c,
+                   float **dst, float **descale) -> svl_status {
         if (!v->split) return upload_owned(v->allocations, w.data(), w.size(), dst);
-        return upload_split(v->allocations, w.data(), (int64_t)w.size() / K, K, a_scale, dst,
-                            descale);
+        return load.weight(w, K, a_scale, c, dst, descale);
+    };
+    // A norm weight whose outputs are a projection's operand: it carries their
+    // scales.
+    auto put_norm = [&](const std::vector<float> &w, const ChannelScales &c, float **dst) {
+        std::vector<float> s(w);
+        for (size_t i = 0; v->split && i < s.size(); ++i) s[i] *= c.scale[i];
+        return upload_owned(v->allocations, s.data(), s.size(), dst);
     };
     if (v->split) {
         // convex sums of RMS-normalised value rows; unscaled norms of the bins
@@ -795,60 +804,61 @@ svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, i
         v->s_pool = split_scale(std::sqrt((double)v->H));
     }
     ST_TRY(decode_named(by_name, "vision_tower.patch_embedder.input_proj.weight", a));
-    ST_TRY(put(a, PATCH_VALUES, 1.f, &v->w_in, &v->d_in));  // patches carry row scales
+    // patches carry row scales
+    ST_TRY(put(a, PATCH_VALUES, 1.f, nullptr, &v->w_in, &v->d_in));
     ST_TRY(up("vision_tower.patch_embedder.position_embedding_table", &v->pos_table));
     ST_TRY(decode_named(by_name, "embed_vision.embedding_projection.weight", a));
-    ST_TRY(put(a, v->H, v->s_pool, &v->w_proj, &v->d_proj));
+    ST_TRY(put(a, v->H, v->s_pool, nullptr, &v->w_proj, &v->d_proj));
     v->layers.resize((size_t)v->L);
     for (int64_t l = 0; l < v->L; ++l) {
         VisLayer &ly = v->layers[(size_t)l];
         const std::string p = "vision_tower.encoder.layers." + std::to_string(l) + ".";
         std::vector<float> qkv((size_t)((v->qd + 2 * v->kd) * v->H));
         ST_TRY(decode_named(by_name, p + "input_layernorm.weight", nw));
-        if (v->split) ly.s_in = split_scale(norm_bound(nw));
+        const ChannelScales c_in(norm_bounds(nw));
+        ST_TRY(put_norm(nw, c_in, &ly.ln_in));
         ST_TRY(decode_named(by_name, p + "self_attn.q_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin());
         ST_TRY(decode_named(by_name, p + "self_attn.k_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + v->qd * v->H);
         ST_TRY(decode_named(by_name, p + "self_attn.v_proj.linear.weight", a));
         std::copy(a.begin(), a.end(), qkv.begin() + (v->qd + v->kd) * v->H);
-        ST_TRY(put(qkv, v->H, ly.s_in, &ly.w_qkv, &ly.d_qkv));
+        ST_TRY(put(qkv, v->H, 1.f, &c_in, &ly.w_qkv, &ly.d_qkv));
+        ST_TRY(decode_named(by_name, p + "self_attn.q_norm.weight", b2));
+        ST_TRY(decode_named(by_name, p + "self_attn.k_norm.weight", c2));
         if (v->split) {
-            // a rotated row's values are at most the row's norm; scale 1.0
-            // (vision.rs:881) times log2(e) for scores in log2 units
-            ST_TRY(decode_named(by_name, p + "self_attn.q_norm.weight", nw));
+            // a rotated row's values are at most the row's norm, each half of a
+            // head rotating by itself; scale 1.0 (vision.rs:881) times log2(e)
+            // for scores in log2 units
+            load.fits = load.fits && balance_heads(b2, c2, b2.size() / 2);
             ly.s_heads.q_mul = 1.4426950408889634f;
-            ly.s_heads.q = split_scale(norm_bound(nw) * ly.s_heads.q_mul);
-            ST_TRY(decode_named(by_name, p + "self_attn.k_norm.weight", nw));
-            ly.s_heads.k = split_scale(norm_bound(nw));
+            ly.s_heads.q = split_scale(largest(norm_bounds(b2)) * ly.s_heads.q_mul);
+            ly.s_heads.k = split_scale(largest(norm_bounds(c2)));
             ly.s_heads.v = v->s_attn;
         }
+        ST_TRY(upload_owned(v->allocations, b2.data(), b2.size(), &ly.q_norm));
+        ST_TRY(upload_owned(v->allocations, c2.data(), c2.size(), &ly.k_norm));
         ST_TRY(decode_named(by_name, p + "self_attn.o_proj.linear.weight", a));
-        ST_TRY(put(a, v->qd, v->s_attn, &ly.w_o, &ly.d_o));
+        ST_TRY(put(a, v->qd, v->s_attn, nullptr, &ly.w_o, &ly.d_o));
         ST_TRY(decode_named(by_name, p + "mlp.gate_proj.linear.weight", b2));
         ST_TRY(decode_named(by_name, p + "mlp.up_proj.linear.weight", c2));
         const std::vector<float> gu =
             interleave_gate_up(b2, c2, v->I, v->I_pad, v->H, v->split ? 16 : 32);
-        ST_TRY(up(p + "pre_feedforward_layernorm.weight", &ly.ln_pre_ff));
-        if (v->split) {
-            ly.s_ff = split_scale(norm_bound(a));  // `up` left the norm weights in a
-            ST_TRY(upload_rows(v->allocations, gu.data(), 2 * v->I, v->H, &ly.w_gu, &ly.d_gu));
-            double act;
-            ST_TRY(geglu_bound(ly.w_gu, v->I, v->H, ly.ln_pre_ff, ly.d_gu, &act));
-            ly.s_act = split_scale(act);
-            ST_TRY(split_weight(ly.w_gu, 2 * v->I, v->H, ly.s_ff, ly.d_gu));
-        } else {
+        ST_TRY(decode_named(by_name, p + "pre_feedforward_layernorm.weight", nw));
+        const ChannelScales c_ff(norm_bounds(nw));
+        ST_TRY(put_norm(nw, c_ff, &ly.ln_pre_ff));
+        std::vector<double> act;
+        if (v->split)
+            ST_TRY(load.geglu(gu, v->I, v->H, nw, c_ff, &ly.w_gu, &ly.d_gu, act));
+        else
             ST_TRY(upload_owned(v->allocations, gu.data(), gu.size(), &ly.w_gu));
-        }
+        const ChannelScales c_act(act);
         ST_TRY(decode_named(by_name, p + "mlp.down_proj.linear.weight", a));
-        ST_TRY(put(a, v->I, ly.s_act, &ly.w_down, &ly.d_down));
-        ST_TRY(up(p + "input_layernorm.weight", &ly.ln_in));
+        ST_TRY(put(a, v->I, 1.f, &c_act, &ly.w_down, &ly.d_down));
         ST_TRY(up(p + "post_attention_layernorm.weight", &ly.ln_post_attn));
         ST_TRY(up(p + "post_feedforward_layernorm.weight", &ly.ln_post_ff));
-        ST_TRY(up(p + "self_attn.q_norm.weight", &ly.q_norm));
-        ST_TRY(up(p + "self_attn.k_norm.weight", &ly.k_norm));
     }
-    if (v->split) HIP_TRY(hipStreamSynchronize(nullptr));  // the weights' conversion
+    if (v->split) ST_TRY(load.finish(fits));
     HIP_TRY(hipStreamCreateWithFlags(&v->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&v->extra, hipStreamNonBlocking));
     HIP_TRY(hipEventCreateWithFlags(&v->ev_fork, hipEventDisableTiming));
@@ -874,6 +884,17 @@ svl_status svl_vision_model_set_pass_patches(svl_vision_model *model, int64_t pa
     std::lock_guard<std::mutex> lock(model->mu);
     model->pass_patches = patches;
     return SVL_OK;
+}
+
+svl_status svl_vision_model_create(svl_ctx *ctx, const svl_vision_config *cfg, int64_t text_hidden,
+                                   const svl_tensor_view *tensors, size_t n_tensors,
+                                   svl_vision_model **out) {
+    bool fits = true;
+    ST_TRY(create_vision(ctx, cfg, text_hidden, tensors, n_tensors, true, &fits, out));
+    if (fits) return SVL_OK;
+    delete *out;  // weights that the split operands would round: FP32 operands
+    *out = nullptr;
+    return create_vision(ctx, cfg, text_hidden, tensors, n_tensors, false, &fits, out);
 }
 
 svl_status svl_vision_model_destroy(svl_vision_model *model) {

@@ -80,3 +80,96 @@ def test_split_attention_matches_the_oracle_and_itself(heads, kv, hd):
         assert np.array_equal(alone.projected(), outs[i].projected())
         assert np.abs(alone.normalized() - oracle.forward(rows[i])["normalized"]).max() <= 1e-4
     model.close()
+
+
+def cancelling_gains(w, layers, heads_group, rng, k):
+    """The same function with some channels 2^k stronger where they are written and 2^-k weaker
+    where they are read: norm outputs, GeGLU and PLE activations, query and key pairs."""
+    w = dict(w)
+    up = np.float32(2.0 ** k)
+
+    def scaled(name, index, gain):
+        w[name] = w[name].copy()
+        w[name][index] *= gain
+
+    def channel(norm, readers):
+        c = int(rng.integers(len(w[norm])))
+        scaled(norm, c, up)
+        for r in readers:
+            scaled(r, (slice(None), c), 1 / up)
+
+    pre = "language_model."
+    channel(pre + "norm.weight", [pre + "embedding_projection.weight"])
+    ps = [f"{pre}layers.{l}." for l in range(layers)]
+    channel(pre + "ple.per_layer_projection_norm.weight",
+            [p + "ple_block.per_layer_projection.weight" for p in ps])
+    for p in ps:
+        channel(p + "input_layernorm.weight", [f"{p}self_attn.{x}_proj.weight" for x in "qkv"])
+        channel(p + "pre_feedforward_layernorm.weight",
+                [p + "mlp.gate_proj.weight", p + "mlp.up_proj.weight"])
+        j = int(rng.integers(len(w[p + "mlp.up_proj.weight"])))
+        scaled(p + "mlp.up_proj.weight", j, up)
+        scaled(p + "mlp.down_proj.weight", (slice(None), j), 1 / up)
+        i = int(rng.integers(heads_group // 2))
+        pair = [i, i + heads_group // 2]
+        scaled(p + "self_attn.q_norm.weight", pair, up)
+        scaled(p + "self_attn.k_norm.weight", pair, 1 / up)
+    return w
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(2, 1, 64), (3, 1, 256), (2, 1, 512), (2, 1, 128)])
+@pytest.mark.parametrize("k", [20, 7, -17])
+def test_channel_gains_that_cancel_leave_the_bits(heads, kv, hd, k):
+    """Every channel of a split operand has a scale of its own: one that stands out by any power of
+    two, undone by the weight that reads it, changes no bit (one scale per tensor held the other
+    channels in 2^k fewer)."""
+    cfg = small_config(128, 160, 64, heads, kv, hd, 96)
+    w = svl_synth.weights(cfg, seed=9)
+    tc = svl_amd.TextConfig.from_json_value(cfg)
+    rows = svl_synth.token_rows(97, [5, 40], seed=10)
+    outs = []
+    for v in (w, cancelling_gains(w, 2, hd, np.random.default_rng(k + 100), k)):
+        model = svl_amd.TextModel(tc, v)
+        outs.append([r.projected() for r in model.forward_batch(rows)])
+        model.close()
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
+def test_strong_gate_and_up_channels_match_the_oracle():
+    """A few gate and up rows 2^8 stronger (products of 2^16), not undone anywhere."""
+    cfg = small_config(128, 160, 64, 2, 1, 64, 96)
+    w = svl_synth.weights(cfg, seed=11)
+    for l in range(2):
+        for name in ("gate_proj", "up_proj"):
+            w[f"language_model.layers.{l}.mlp.{name}.weight"][[3, 77]] *= np.float32(256.0)
+    model = svl_amd.TextModel(svl_amd.TextConfig.from_json_value(cfg), w)
+    row = svl_synth.token_rows(97, [29], seed=12)[0]
+    ref = O.OracleTextModel(cfg, w).forward(row)["normalized"]
+    # two layers of float32 sums of at most 160 terms: a few 2^-23 of the vector's norm 1
+    assert np.abs(model.forward(row).normalized() - ref).max() <= 4e-6
+    model.close()
+
+
+@pytest.mark.parametrize("where", ["norm", "key pair"])
+def test_silent_outliers_keep_the_other_channels(where):
+    """An outlier that no later weight undoes and whose values happen to be zero: a norm weight of
+    2^30 over a column of zeros (its bound leaves the others' columns 2^30 below it, so the model
+    runs on FP32 operands), and query weights of 2^24 on a pair whose key weights are zero. In
+    FP32 neither changes anything."""
+    cfg = small_config(128, 160, 64, 2, 1, 64, 96)
+    w = svl_synth.weights(cfg, seed=13)
+    p = "language_model.layers.0."
+    if where == "norm":
+        w["language_model.embed_tokens.weight"][:, 17] = 0.0
+    else:
+        w[p + "self_attn.k_norm.weight"][[4, 36]] = 0.0
+    row = svl_synth.token_rows(97, [23], seed=14)[0]
+    ref = O.OracleTextModel(cfg, w).forward(row)["normalized"]
+    if where == "norm":
+        w[p + "input_layernorm.weight"][17] *= np.float32(2.0 ** 30)
+    else:
+        w[p + "self_attn.q_norm.weight"][[4, 36]] *= np.float32(2.0 ** 24)
+    model = svl_amd.TextModel(svl_amd.TextConfig.from_json_value(cfg), w)
+    assert np.abs(model.forward(row).normalized() - ref).max() <= 4e-6  # as above
+    model.close()

@@ -115,6 +115,32 @@ def test_batch_is_bit_identical_to_single_calls(tower_v2):
         assert np.array_equal(again[i].pooled(), batch[len(patches) - 1 - i].pooled())
 
 
+@pytest.mark.parametrize("k", [20, -9])
+def test_channel_gains_that_cancel_leave_the_bits(tower_v2, k):
+    """Channels 2^k stronger where they are written and 2^-k weaker where they are read (norm
+    outputs, GeGLU activations, rotated query and key pairs) are the same function, and every
+    channel of a split operand has a scale of its own: no bit changes."""
+    w, gpu, om = tower_v2
+    up = np.float32(2.0 ** k)
+    g = {n: v.copy() for n, v in w.items()}
+    for l in range(2):
+        p = f"vision_tower.encoder.layers.{l}."
+        for c, norm, readers in ((5 + l, "input_layernorm", [f"self_attn.{x}_proj" for x in "qkv"]),
+                                 (700, "pre_feedforward_layernorm", ["mlp.gate_proj", "mlp.up_proj"])):
+            g[f"{p}{norm}.weight"][c] *= up
+            for r in readers:
+                g[f"{p}{r}.linear.weight"][:, c] /= up
+        g[f"{p}mlp.up_proj.linear.weight"][1234] *= up
+        g[f"{p}mlp.down_proj.linear.weight"][:, 1234] /= up
+        for pair in ([3, 19], [40, 56]):      # each half of a head rotates by itself
+            g[f"{p}self_attn.q_norm.weight"][pair] *= up
+            g[f"{p}self_attn.k_norm.weight"][pair] /= up
+    gained = type(gpu)(gpu.config, g, 768)
+    patches = svl_synth.image_patches(1, 12, 9, seed=43)[0]
+    assert np.array_equal(gained.forward(patches).pooled(), gpu.forward(patches).pooled())
+    gained.close()
+
+
 def test_image_groups_are_bit_identical(tower_v2):
     # Batches of two or more images and 4096 or more patches run the encoder
     # layers as two image groups on two streams: here images 0-1 (2304 + 1296
