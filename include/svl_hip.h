@@ -220,7 +220,9 @@ svl_status svl_rope_with_inv_freq(float *d_values, int64_t seq_len, int64_t num_
                                   int64_t position_offset, void *stream);
 /* kernels.rs:991-1010 rope_inv_freq (host). */
 svl_status svl_rope_inv_freq(int64_t head_dim, float base, float *out);
-/* kernels.rs:1037-1135 bidirectional_attention; sliding_window < 0 = full. */
+/* kernels.rs:1037-1135 bidirectional_attention; sliding_window < 0 = full.
+ * Sizes that the entry point below takes run through it (and share its array
+ * and lock); larger ones allocate their work items for the call. */
 svl_status svl_bidirectional_attention(const float *d_q, const float *d_k, const float *d_v,
                                        int64_t seq_len, int64_t num_heads,
                                        int64_t num_kv_heads, int64_t head_dim,

@@ -888,16 +888,28 @@ svl_status seam_flag(hipStream_t s, SeamFlag **out) {
     return SVL_OK;
 }
 
-svl_status seam_read(hipStream_t s, const int *flag, int *h, const char *what) {
+// A call's stream, waited for on every way out: what calls share (the flag, the
+// allocation-free attention's scratch) is never left to work in flight, also
+// where a launch after the first fails.
+struct SeamCall {
+    hipStream_t s;
+    bool waited = false;
+    ~SeamCall() {
+        if (!waited) (void)hipStreamSynchronize(s);
+    }
+};
+
+svl_status seam_read(SeamCall &call, const int *flag, int *h, const char *what) {
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(h, flag, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(hipMemcpyAsync(h, flag, sizeof(int), hipMemcpyDeviceToHost, call.s));
+    HIP_TRY(hipStreamSynchronize(call.s));
+    call.waited = true;
     if (*h & FLAG_NONFINITE) return fail(SVL_INTERNAL, "%s produced a non-finite value", what);
     return SVL_OK;
 }
 
-svl_status seam_finish(hipStream_t s, SeamFlag *f, const char *what) {
-    ST_TRY(seam_read(s, f->dev, f->host, what));
+svl_status seam_finish(SeamCall &call, SeamFlag *f, const char *what) {
+    ST_TRY(seam_read(call, f->dev, f->host, what));
     f->dirty = *f->host != 0;
     return SVL_OK;
 }
@@ -1471,6 +1483,7 @@ svl_status svl_linear(const float *d_in, const float *d_w, int64_t rows, int64_t
     hipStream_t s = (hipStream_t)stream;
     SeamFlag *flag;
     ST_TRY(seam_flag(s, &flag));
+    SeamCall call{s};
     GemmArgs g{d_in, in_features, d_w, in_features, d_out, out_features, (int)rows,
                (int)out_features, (int)in_features, EPI_STORE, 1.f, nullptr, 0, 0};
     if (in_features == 0) {
@@ -1479,7 +1492,7 @@ svl_status svl_linear(const float *d_in, const float *d_w, int64_t rows, int64_t
         HIP_TRY(launch_gemm(g, s));
     }
     HIP_TRY(launch_finite_check(d_out, rows * out_features, flag->dev, s));
-    return seam_finish(s, flag, "linear projection");
+    return seam_finish(call, flag, "linear projection");
 }
 
 svl_status svl_rms_norm_rows(const float *d_in, const float *d_weight, int64_t rows,
@@ -1493,8 +1506,9 @@ svl_status svl_rms_norm_rows(const float *d_in, const float *d_weight, int64_t r
     hipStream_t s = (hipStream_t)stream;
     SeamFlag *flag;
     ST_TRY(seam_flag(s, &flag));
+    SeamCall call{s};
     HIP_TRY(launch_rms_rows(d_in, d_weight, d_out, rows, (int)width, eps, flag->dev, s));
-    return seam_finish(s, flag, "RMSNorm");
+    return seam_finish(call, flag, "RMSNorm");
 }
 
 svl_status svl_rope_inv_freq(int64_t head_dim, float base, float *out) {
@@ -1532,6 +1546,7 @@ svl_status svl_rope_with_inv_freq(float *d_values, int64_t seq_len, int64_t num_
     hipStream_t s = (hipStream_t)stream;
     SeamFlag *flag;
     ST_TRY(seam_flag(s, &flag));
+    SeamCall call{s};
     float *dc = nullptr, *ds = nullptr;
     HIP_TRY(hipMalloc((void **)&dc, c.size() * 4));
     HIP_TRY(hipMalloc((void **)&ds, sn.size() * 4));
@@ -1541,7 +1556,7 @@ svl_status svl_rope_with_inv_freq(float *d_values, int64_t seq_len, int64_t num_
         launch_rope(d_values, seq_len, (int)num_heads, (int)head_dim, dc, ds, flag->dev, s) !=
             hipSuccess)
         st = fail(SVL_DEVICE, "RoPE launch failed");
-    if (st == SVL_OK) st = seam_finish(s, flag, "RoPE");
+    if (st == SVL_OK) st = seam_finish(call, flag, "RoPE");
     (void)hipStreamSynchronize(s);
     (void)hipFree(dc);
     (void)hipFree(ds);
@@ -1614,6 +1629,7 @@ svl_status svl_bidirectional_attention(const float *d_q, const float *d_k, const
     hipStream_t s = (hipStream_t)stream;
     SeamFlag *flag;
     ST_TRY(seam_flag(s, &flag));
+    SeamCall call{s};
     AttnTile *dt = nullptr;
     int32_t *dp = nullptr, *dl = nullptr;
     HIP_TRY(hipMalloc((void **)&dt, std::max<size_t>(tiles.size(), 1) * sizeof(AttnTile)));
@@ -1633,7 +1649,7 @@ svl_status svl_bidirectional_attention(const float *d_q, const float *d_k, const
         hipMemcpyAsync(dl, rl.data(), rl.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess ||
         launch_attention(a, s) != hipSuccess)
         st = fail(SVL_DEVICE, "attention launch failed");
-    if (st == SVL_OK) st = seam_finish(s, flag, "attention");
+    if (st == SVL_OK) st = seam_finish(call, flag, "attention");
     (void)hipStreamSynchronize(s);
     (void)hipFree(dt);
     (void)hipFree(dp);
@@ -1673,10 +1689,11 @@ svl_status svl_bidirectional_attention_noalloc(const float *d_q, const float *d_
     hipStream_t s = (hipStream_t)stream;
     // one call at a time per process: every call on a GPU shares its scratch
     std::lock_guard<std::mutex> lock(g_noalloc_mu);
+    int raised = 0;
+    SeamCall call{s};  // ends before the lock does
     HIP_TRY(launch_noalloc_attn_setup(base, (int)seq_len, (int)(tiles / num_kv_heads), bv, a.n_tiles, s));
     if (launch_attention(a, s) != hipSuccess) return fail(SVL_DEVICE, "attention launch failed");
-    int raised = 0;
-    return seam_read(s, a.flag, &raised, "attention");
+    return seam_read(call, a.flag, &raised, "attention");
 }
 
 svl_status svl_set_attention_path(int path) {
@@ -1717,6 +1734,7 @@ svl_status svl_mean_pool(const float *d_values, int64_t rows, int64_t width, flo
     hipStream_t s = (hipStream_t)stream;
     SeamFlag *flag;
     ST_TRY(seam_flag(s, &flag));
+    SeamCall call{s};
     int64_t *doff = nullptr;
     const int64_t offs[2] = {0, rows};
     HIP_TRY(hipMalloc((void **)&doff, sizeof offs));
@@ -1726,7 +1744,7 @@ svl_status svl_mean_pool(const float *d_values, int64_t rows, int64_t width, flo
                     s) != hipSuccess ||
         launch_finite_check(d_out, width, flag->dev, s) != hipSuccess)
         st = fail(SVL_DEVICE, "mean pool launch failed");
-    if (st == SVL_OK) st = seam_finish(s, flag, "mean pooling");
+    if (st == SVL_OK) st = seam_finish(call, flag, "mean pooling");
     (void)hipStreamSynchronize(s);
     (void)hipFree(doff);
     return st;
@@ -1739,12 +1757,13 @@ svl_status svl_l2_normalize(const float *d_in, int64_t n, float *d_out, void *st
     hipStream_t s = (hipStream_t)stream;
     SeamFlag *flag;
     ST_TRY(seam_flag(s, &flag));
+    SeamCall call{s};
     // The pool-normalisation kernel on one already pooled row applies
     // l2_normalize_scalar's arithmetic.
     svl_status st = SVL_OK;
     if (launch_pool_norm(d_in, (int)n, 1, nullptr, 0, 0, d_out, nullptr, flag->dev, s) != hipSuccess)
         st = fail(SVL_DEVICE, "l2 launch failed");
-    if (st == SVL_OK) st = seam_finish(s, flag, "L2 normalization");
+    if (st == SVL_OK) st = seam_finish(call, flag, "L2 normalization");
     (void)hipStreamSynchronize(s);
     if (st == SVL_INTERNAL) g_err = "cannot normalize a zero or non-finite vector";
     return st;

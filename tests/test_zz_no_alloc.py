@@ -1,16 +1,18 @@
-"""The allocation-free attention entry point
-(svl_bidirectional_attention_noalloc, through the C ABI) against the
-allocating one it varies (svl_bidirectional_attention, kernels.rs:1037-1135):
-the same kernels, so the same bits, on two calls in a row with the second
-smaller than the first (the per-GPU scratch keeps the first call's work items
-and flag, which the second must not see). Also: a non-finite result raises
-Internal and the next call starts from a clear flag, and sizes beyond the
-scratch are rejected with LimitExceeded before anything runs."""
+"""The attention entry points' scratch (svl_bidirectional_attention_noalloc, and
+svl_bidirectional_attention, which takes the same way for sizes the scratch
+holds; kernels.rs:1037-1135) against the CPU oracle, on two calls in a row with
+the second smaller than the first (the per-GPU scratch keeps the first call's
+work items and flag, which the second must not see). Also: a size beyond the
+scratch through the entry point that allocates, a non-finite result raises
+Internal and the next call starts from a clear flag, and the allocation-free
+entry point rejects sizes beyond the scratch with LimitExceeded before anything
+runs."""
 import numpy as np
 import pytest
 import torch
 
 import svl_amd as S
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -41,17 +43,33 @@ def call(fn, shape, tensors):
     return out.cpu().numpy()
 
 
+def check_oracle(got, shape, tensors):
+    seq, nh, nkv, hd, window = shape
+    want = O.bidirectional_attention(*(t.cpu().numpy() for t in tensors), seq, nh, nkv, hd, window, 1.0)
+    assert np.isfinite(got).all(), shape
+    assert np.abs(got - want).max() <= 1e-4, shape  # the attention bound of the kernel tests
+
+
 @pytest.mark.parametrize("big,small", SHAPES)
-def test_noalloc_attention_equals_the_allocating_entry_point(big, small):
+def test_attention_scratch_holds_nothing_of_the_call_before(big, small):
     tb = inputs(*big[:4], seed=1)
     ts = inputs(*small[:4], seed=2)
-    got_big = call(S.bidirectional_attention_noalloc, big, tb)
-    got_small = call(S.bidirectional_attention_noalloc, small, ts)
-    want_big = call(S.bidirectional_attention, big, tb)
-    want_small = call(S.bidirectional_attention, small, ts)
-    for got, want, label in ((got_big, want_big, big), (got_small, want_small, small)):
-        assert np.isfinite(got).all(), label
-        assert got.tobytes() == want.tobytes(), label
+    for fn in (S.bidirectional_attention_noalloc, S.bidirectional_attention):
+        got_big = call(fn, big, tb)
+        got_small = call(fn, small, ts)
+        check_oracle(got_big, big, tb)
+        check_oracle(got_small, small, ts)
+
+
+def test_attention_beyond_the_scratch_allocates():
+    """8193 keys, one more than the scratch holds."""
+    shape = (8193, 1, 1, 64, 16)
+    t = inputs(*shape[:4], seed=5)
+    check_oracle(call(S.bidirectional_attention, shape, t), shape, t)
+    # and the scratch's next call is as before
+    small = (64, 3, 1, 256, None)
+    ts = inputs(*small[:4], seed=6)
+    check_oracle(call(S.bidirectional_attention, small, ts), small, ts)
 
 
 def test_noalloc_attention_flag_is_cleared_between_calls():
@@ -62,8 +80,7 @@ def test_noalloc_attention_flag_is_cleared_between_calls():
     with pytest.raises(S.SvlError) as e:
         call(S.bidirectional_attention_noalloc, shape, (bad, k, v))
     assert e.value.kind == "Internal"
-    got = call(S.bidirectional_attention_noalloc, shape, (q, k, v))
-    assert got.tobytes() == call(S.bidirectional_attention, shape, (q, k, v)).tobytes()
+    check_oracle(call(S.bidirectional_attention_noalloc, shape, (q, k, v)), shape, (q, k, v))
 
 
 def test_noalloc_attention_rejects_sizes_beyond_its_scratch():
@@ -86,5 +103,4 @@ def test_noalloc_attention_rejects_sizes_beyond_its_scratch():
     del q, out
     shape = (64, 3, 1, 256, None)
     t = inputs(*shape[:4], seed=4)
-    assert call(S.bidirectional_attention_noalloc, shape, t).tobytes() == \
-        call(S.bidirectional_attention, shape, t).tobytes()
+    check_oracle(call(S.bidirectional_attention_noalloc, shape, t), shape, t)
