@@ -217,46 +217,57 @@ def test_packed_batch_equals_independent_calls_bit_for_bit():
         assert a.normalized().tobytes() == b.normalized().tobytes()
 
 
-def test_two_stream_row_groups_are_bit_identical():
-    # Batches above 4096 tokens run as row groups on concurrent streams (a
-    # batch whose rows are all longer than the 512 window runs as one group).
-    cfg = svl_synth.config_a(layers=2, vocab=4096)
-    w = svl_synth.weights(cfg)
-    m = model(cfg, w)
+def groups_equal_one(m, rows, groups):
+    """The batch in `groups` row groups, equal to one group byte for byte."""
+    m.set_stream_split(1)
+    single = m.forward_batch(rows, capture_hidden=True)
+    for g in groups:
+        m.set_stream_split(g)
+        split = m.forward_batch(rows, capture_hidden=True)
+        for a, b in zip(split, single):
+            assert a.normalized().tobytes() == b.normalized().tobytes(), g
+            assert a.projected().tobytes() == b.projected().tobytes(), g
+            assert a.hidden_states().tobytes() == b.hidden_states().tobytes(), g
+    return single
+
+
+# Shape A, shape B (head dims 256 and 512), and an FFN width that keeps the
+# projections on FP32 operands (three groups by default).
+@pytest.mark.parametrize("shape", ["a", "b", "fp32"])
+def test_row_groups_are_bit_identical(shape):
+    # Batches of 4096 tokens or more run as the row groups asked for, each on
+    # a stream of its own (a batch whose rows are all longer than the 512
+    # window runs as one group).
+    cfg = (svl_synth.config_b if shape == "b" else svl_synth.config_a)(layers=2, vocab=4096)
+    if shape == "fp32":
+        cfg["intermediate_size"] = 1136
+    m = model(cfg, svl_synth.weights(cfg))
     rows = svl_synth.token_rows(4096, [512, 300, 500, 400, 100, 480, 500, 513, 64, 512, 300, 400,
                                        700])
     assert sum(len(r) for r in rows) >= 4096
-    split = m.forward_batch(rows, capture_hidden=True)
-    m.set_stream_split(False)
-    single = m.forward_batch(rows, capture_hidden=True)
-    m.set_stream_split(True)
-    for a, b in zip(split, single):
-        assert a.normalized().tobytes() == b.normalized().tobytes()
-        assert a.hidden_states().tobytes() == b.hidden_states().tobytes()
-    for r, a in zip(rows[:3], split[:3]):
+    default = m.forward_batch(rows)
+    single = groups_equal_one(m, rows, (2, 3, 4))
+    for r, a in zip(rows[:3], single[:3]):
         assert m.forward(r).normalized().tobytes() == a.normalized().tobytes()
+    for a, b in zip(default, single):
+        assert a.normalized().tobytes() == b.normalized().tobytes()
 
 
-def test_row_groups_in_grouped_tile_order_are_bit_identical():
-    # About 16,000 tokens: each of the three row groups' GEMMs has 80 or more
-    # 64-row M blocks, so the shared launches take the grouped tile order
-    # (odd groups of 8 M blocks run their N blocks in reverse, the last group
-    # is partial); the single-stream launches of the whole batch take it too,
-    # and one row alone runs small tiles in the plain order.
+@pytest.mark.parametrize("inter", [1152, 1136])
+def test_row_groups_in_grouped_tile_order_are_bit_identical(inter):
+    # About 16,000 tokens. On split operands (FFN 1152) the projections of 1280
+    # columns or more take the grouped tile order (groups of 8 M blocks, odd
+    # groups with their N blocks in reverse, a partial last group) in every
+    # launch; on FP32 operands (1136) the large ones do, and from 32 M blocks
+    # where launches of other row groups run beside them.
     cfg = svl_synth.config_a(layers=2, vocab=4096)
-    w = svl_synth.weights(cfg)
-    m = model(cfg, w)
+    cfg["intermediate_size"] = inter
+    m = model(cfg, svl_synth.weights(cfg))
     lengths = [300 + (97 * i) % 213 for i in range(40)]
     rows = svl_synth.token_rows(4096, lengths, seed=5)
-    split = m.forward_batch(rows, capture_hidden=True)
-    m.set_stream_split(False)
-    single = m.forward_batch(rows, capture_hidden=True)
-    m.set_stream_split(True)
-    for a, b in zip(split, single):
-        assert a.normalized().tobytes() == b.normalized().tobytes()
-        assert a.hidden_states().tobytes() == b.hidden_states().tobytes()
+    single = groups_equal_one(m, rows, (3,))
     for i in (0, 13, 39):
-        assert m.forward(rows[i]).normalized().tobytes() == split[i].normalized().tobytes()
+        assert m.forward(rows[i]).normalized().tobytes() == single[i].normalized().tobytes()
 
 
 def test_batches_run_in_passes_bit_for_bit():
