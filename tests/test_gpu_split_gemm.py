@@ -1,7 +1,9 @@
 """Projections on split operands (F16 matrix cores, three products) at the
 shapes where the kernel's tiles can go wrong: single 32-k blocks, slices of one
-to eight blocks, rows and columns that end inside a tile, narrow widths, and
-every epilogue of the text path, against the scalar oracle."""
+to eight blocks, rows and columns that end inside a small or a large tile,
+narrow widths, both tile orders, and every epilogue of the text path, against
+the scalar oracle; operands whose channels spread far apart; and attention on
+split head rows."""
 import numpy as np
 import pytest
 
@@ -43,6 +45,29 @@ def test_split_projections_match_the_oracle(shape):
             1.0, float(np.abs(ref["projected"]).max()))
         alone = model.forward(row)
         assert np.array_equal(alone.normalized(), out.normalized())
+    model.close()
+
+
+# tokens and embedding width: outputs that end inside a large tile and inside a run of four
+# columns, in the plain order (100 and 803 columns) and the grouped one (1301 and 2307); 64x64
+# tiles, then 64x128 and 128x128 ones by turns
+@pytest.mark.parametrize("tokens,out", [(24000, 100), (27000, 100), (24000, 803), (12000, 803),
+                                        (15700, 1301), (12000, 1301), (9000, 2307)])
+def test_large_tiles_end_inside_the_output(tokens, out):
+    cfg = small_config(64, 64, 32, 1, 1, 32, out)
+    w = svl_synth.weights(cfg, seed=15)
+    model = svl_amd.TextModel(svl_amd.TextConfig.from_json_value(cfg), w)
+    n = 61
+    lengths = [n] * (tokens // n) + [tokens % n or 1]
+    rows = svl_synth.token_rows(97, lengths, seed=16)
+    outs = model.forward_batch(rows)
+    oracle = O.OracleTextModel(cfg, w)
+    for i in (0, len(rows) // 2, len(rows) - 2, len(rows) - 1):
+        alone = model.forward(rows[i])  # small tiles
+        assert np.array_equal(alone.projected(), outs[i].projected())
+        ref = oracle.forward(rows[i])["projected"]
+        # as in test_split_projections_match_the_oracle
+        assert np.abs(outs[i].projected() - ref).max() <= 1e-4 * max(1.0, float(np.abs(ref).max()))
     model.close()
 
 
