@@ -34,6 +34,10 @@ constexpr int64_t MAX_EMBEDDING_DIMENSION = 8192;  // storage/model.rs:35
 // in place of copies: per query a flag word, a candidate count and the page
 // length, and the page where it is small.
 constexpr size_t HOST_PAGE_BYTES = (size_t)1 << 20;  // larger pages are copied instead
+// Allocated with the index (64 queries of 63 hits; larger ones grow it): in an
+// index's first call it took 30 to 100 us, which a small index does not win back
+// there.
+constexpr size_t HOST_PAGE_START = (size_t)64 << 10;
 struct HostPage {
     unsigned char *p = nullptr;
     size_t bytes = 0;
@@ -42,18 +46,18 @@ struct HostPage {
     int64_t *take = nullptr, *index = nullptr;  // index, score: null for large pages
     double *score = nullptr;
 
+    hipError_t reserve(size_t need) {
+        if (need <= bytes) return hipSuccess;
+        release();
+        const hipError_t e = hipHostMalloc((void **)&p, need, hipHostMallocDefault);
+        if (e != hipSuccess) p = nullptr;
+        else bytes = need;
+        return e;
+    }
     hipError_t ensure(int64_t nq, int64_t limit) {
         const bool page = limit <= (int64_t)(HOST_PAGE_BYTES / 16) / nq;
-        const size_t need = (size_t)nq * 16 + (page ? (size_t)(nq * limit) * 16 : 0);
-        if (need > bytes) {
-            release();
-            const hipError_t e = hipHostMalloc((void **)&p, need, hipHostMallocDefault);
-            if (e != hipSuccess) {
-                p = nullptr;
-                return e;
-            }
-            bytes = need;
-        }
+        const hipError_t e = reserve((size_t)nq * 16 + (page ? (size_t)(nq * limit) * 16 : 0));
+        if (e != hipSuccess) return e;
         take = reinterpret_cast<int64_t *>(p);
         flags = reinterpret_cast<int *>(take + nq);
         found = reinterpret_cast<unsigned int *>(flags + nq);
@@ -403,6 +407,7 @@ svl_status svl_vector_index_create(svl_ctx *ctx, const float *embeddings,
     ix->D = n > 0 ? dimension : 0;
     HIP_TRY(hipSetDevice(ix->device));
     HIP_TRY(hipStreamCreateWithFlags(&ix->stream, hipStreamNonBlocking));
+    HIP_TRY(ix->page.reserve(HOST_PAGE_START));
     ix->ids.assign(chunk_ids, chunk_ids + n);
     std::vector<int64_t> perm((size_t)n);
     std::iota(perm.begin(), perm.end(), 0);
