@@ -671,7 +671,9 @@ def main():
                                "vocab 262144): batch 64 rows, lengths U[64,512], padding masked, "
                                "Matryoshka outputs 768/512/256/128",
                    "batch": BATCH, "tokens": T, "max_seq_len": LEN_HI, "parallelism": "single GPU",
-                   "row_groups": args.row_groups},
+                   "row_groups": args.row_groups,
+                   "operands": "f32 values held as two f16 halves (22 bits), products as three "
+                               "f16 MFMAs, f32 accumulation"},
         "p50_ms": round(p50, 3),
         "t1_p50_ms": round(float(np.median(lat)), 3) if lat else None,
         "gemm_tflops": round(gemm_tflops, 3),

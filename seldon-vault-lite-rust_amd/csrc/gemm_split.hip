@@ -3,8 +3,8 @@
 //
 // Every product of two operands x = xh + xl, y = yh + yl is taken as xh.yh in
 // one FP32 accumulator and xl.yh + xh.yl in a second: three F16 MFMAs. xh and
-// yh carry the leading 11 bits of the scaled values and xl, yl the next 11,
-// so the dropped xl.yl is below 2^-22 of the product, and an MFMA of 32 k
+// yh carry the leading 11 bits of the scaled values and xl, yl the next 11 (of
+// values within 2^-16 of their scale's top, dev_common.hpp), so the dropped xl.yl is below 2^-22 of the product, and an MFMA of 32 k
 // rounds its accumulator 4 times (once per 8 products, probed) where the FP32
 // MFMA chain rounds 32 times. Against 64-bit sums of normal inputs the result
 // is off by 0.95e-7 / 1.9e-7 / 4.2e-7 (K = 64 / 768 / 4096, relative 2-norm)

@@ -361,12 +361,13 @@ void collect_timing(svl_text_model *m) {
 // the same number of tokens. Each group runs the whole encoder on its own
 // stream (all at the default priority), on its own token range of every
 // workspace buffer, so the streams' kernels fill each other's partial last
-// rounds of workgroups. Every row's arithmetic is unchanged. One group is the
-// default: with the projections and attention on split operands a launch over
-// the whole batch fills the GPU better than three smaller ones beside each
-// other (64 rows, 18432 tokens: 19.5 ms as one group, 21.1 as two, 20.7 as
-// three; 30 rows, 8640 tokens: 10.3, 10.3, 10.9; 40 rows, 14640 tokens: 16.8,
-// 16.0, 18.5), where three groups were 11 % faster on FP32 MFMAs.
+// rounds of workgroups. Every row's arithmetic is unchanged. With the
+// projections and attention on split operands the default is one group: up to
+// about 10000 tokens a launch over the whole batch fills the GPU better than
+// smaller ones beside each other (16 rows, 4800 tokens: 6.75 ms as one group,
+// 7.1 as two, 7.8 as three; 30 rows, 8640: 10.4, 10.6, 12.6), past it two are
+// 3-4 % ahead (40 rows, 14600: 16.8, 16.1, 16.6; 64 rows, 18432: 20.0, 19.4,
+// 20.1). Models on FP32 MFMAs default to three, which were 11 % faster there.
 
 constexpr int64_t SPLIT_MIN_TOKENS = 4096;
 

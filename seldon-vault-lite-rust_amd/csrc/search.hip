@@ -6,7 +6,9 @@
 // that order. A float * float product is exact in double, so the fused
 // multiply-add rounds exactly once per step like the reference's separate
 // multiply and add. score = dot / (query_norm * chunk_norm) with both norms
-// computed in the reference's order on the host.
+// summed in the reference's order: the chunks' on the host when the index is
+// made, the queries' on the host for host queries and in prepare_queries_kernel
+// for device queries.
 //
 // Layout: the chunk matrix V [n, D] (rows in ascending chunk-id order) is
 // streamed once per block of QB queries, a slice of 32 dimensions of the
