@@ -185,17 +185,22 @@ inline svl_status upload_owned(std::vector<float *> &owned, const float *host, s
 }
 
 // The power of two that brings a bound on a split operand's magnitude into
-// [2^13, 2^14) (halves reach 65504), within 2^-100 .. 2^100.
+// [2^13, 2^14) (halves reach 65504), within 2^-100 .. 2^100. From the bits: a
+// model takes some 10^5 of them.
 inline float split_scale(double bound) {
     if (!(bound > 0) || !std::isfinite(bound)) return 1.f;
-    int e;
-    (void)std::frexp(bound, &e);
-    return std::ldexp(1.f, std::max(-100, std::min(100, 14 - e)));
+    uint64_t b;
+    std::memcpy(&b, &bound, sizeof b);
+    const int e = (int)(b >> 52) - 1022;  // bound = f 2^e, f in [0.5, 1), but for denormals
+    const uint32_t s = (uint32_t)(127 + std::max(-100, std::min(100, 14 - e))) << 23;
+    float scale;
+    std::memcpy(&scale, &s, sizeof scale);
+    return scale;
 }
 
 // True where split_scale does bring it there (or there is nothing to bring).
 inline bool split_scalable(double bound) {
-    return bound == 0 || (bound >= std::ldexp(1.0, -80) && bound <= std::ldexp(1.0, 80));
+    return bound == 0 || (bound >= 0x1p-80 && bound <= 0x1p80);
 }
 
 // One scale per channel of a split operand, from a bound on each channel's
@@ -206,11 +211,13 @@ inline bool split_scalable(double bound) {
 struct ChannelScales {
     std::vector<float> scale, inverse;
     bool ok = true;
-    explicit ChannelScales(const std::vector<double> &bounds) {
-        for (double b : bounds) {
-            ok = ok && split_scalable(b);
-            scale.push_back(split_scale(b));
-            inverse.push_back(b > 0 ? 1.f / scale.back() : 0.f);
+    ChannelScales() = default;
+    explicit ChannelScales(const std::vector<double> &bounds)
+        : scale(bounds.size()), inverse(bounds.size()) {
+        for (size_t i = 0; i < bounds.size(); ++i) {
+            ok = ok && split_scalable(bounds[i]);
+            scale[i] = split_scale(bounds[i]);
+            inverse[i] = bounds[i] > 0 ? 1.f / scale[i] : 0.f;
         }
     }
 };
@@ -218,8 +225,9 @@ struct ChannelScales {
 // Largest magnitude of each channel of RMSNorm(x) * w: a normalised value is at
 // most sqrt(n).
 inline std::vector<double> norm_bounds(const std::vector<float> &w) {
-    std::vector<double> b;
-    for (float v : w) b.push_back(std::sqrt((double)w.size()) * std::fabs((double)v));
+    const double most = std::sqrt((double)w.size());
+    std::vector<double> b(w.size());
+    for (size_t i = 0; i < w.size(); ++i) b[i] = most * std::fabs((double)w[i]);
     return b;
 }
 
@@ -270,10 +278,19 @@ struct SplitLoader {
     DevBuf<float> cols, mul;
     DevBuf<int> flag;
     bool fits = true;
+    // The scale vectors' way to the device: pinned, so that a copy is only
+    // enqueued (from pageable memory each waits, some 40 us; a tower takes 80).
+    static constexpr size_t STAGE = (size_t)1 << 18;  // floats
+    float *stage = nullptr;
+    size_t staged = 0;
 
     explicit SplitLoader(std::vector<float *> &o) : owned(o) {}
     SplitLoader(const SplitLoader &) = delete;
     ~SplitLoader() {
+        if (stage) {
+            (void)hipStreamSynchronize(nullptr);
+            (void)hipHostFree(stage);
+        }
         cols.release();
         mul.release();
         flag.release();
@@ -281,7 +298,20 @@ struct SplitLoader {
 
     svl_status put(DevBuf<float> &to, const std::vector<float> &v) {
         HIP_TRY(to.ensure(v.size()));
-        HIP_TRY(hipMemcpy(to.p, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice));
+        if (v.size() > STAGE) {
+            HIP_TRY(hipMemcpy(to.p, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice));
+            return SVL_OK;
+        }
+        if (!stage)
+            HIP_TRY(hipHostMalloc((void **)&stage, STAGE * sizeof(float), hipHostMallocDefault));
+        if (staged + v.size() > STAGE) {
+            HIP_TRY(hipStreamSynchronize(nullptr));  // the copies before have left it
+            staged = 0;
+        }
+        std::copy(v.begin(), v.end(), stage + staged);
+        HIP_TRY(hipMemcpyAsync(to.p, stage + staged, v.size() * sizeof(float),
+                               hipMemcpyHostToDevice, nullptr));
+        staged += v.size();
         return SVL_OK;
     }
 
@@ -342,18 +372,20 @@ struct SplitLoader {
     // being at most |g| |u|, applied by the up rows' descale.
     svl_status geglu(const std::vector<float> &gu, int64_t I, int64_t K,
                      const std::vector<float> &norm, const ChannelScales &in, float **w, float **wd,
-                     std::vector<double> &act) {
+                     ChannelScales &act) {
         std::vector<float> b;
         ST_TRY(upload(gu.data(), 2 * I, K, w, wd));
         ST_TRY(bounds(*w, 2 * I, K, &norm, *wd, b));
-        act.clear();
-        std::vector<float> row_mul((size_t)(2 * I), 1.f);
+        auto at = [](int64_t j) { return (size_t)(32 * (j / 16) + j % 16); };
+        std::vector<double> most((size_t)I);
         for (int64_t j = 0; j < I; ++j) {
-            const size_t at = (size_t)(32 * (j / 16) + j % 16);
-            act.push_back((double)b[at] * (double)b[at + 16]);
-            fits = fits && split_scalable(b[at]) && split_scalable(b[at + 16]);
-            row_mul[at + 16] = split_scale(act.back());
+            const double g = b[at(j)], u = b[at(j) + 16];
+            fits = fits && split_scalable(g) && split_scalable(u);
+            most[(size_t)j] = g * u;
         }
+        act = ChannelScales(most);
+        std::vector<float> row_mul((size_t)(2 * I), 1.f);
+        for (int64_t j = 0; j < I; ++j) row_mul[at(j) + 16] = act.scale[(size_t)j];
         return convert(*w, 2 * I, K, 1.f, &in, *wd, 1.f, &row_mul);
     }
 

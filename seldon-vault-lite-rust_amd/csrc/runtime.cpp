@@ -1146,12 +1146,11 @@ static svl_status create_text(svl_ctx *ctx, const svl_text_config *cfg,
         ST_TRY(get(p + "pre_feedforward_layernorm.weight", nw));
         const ChannelScales c_ff(norm_bounds(nw));
         ST_TRY(put_norm(nw, c_ff, &ly.ln_pre_ff));
-        std::vector<double> act;
+        ChannelScales c_act;
         if (m->split)
-            ST_TRY(load.geglu(gu, m->I, H, nw, c_ff, &ly.w_gu, &ly.d_gu, act));
+            ST_TRY(load.geglu(gu, m->I, H, nw, c_ff, &ly.w_gu, &ly.d_gu, c_act));
         else
             ST_TRY(upload(m, gu.data(), gu.size(), &ly.w_gu));
-        const ChannelScales c_act(act);
         ST_TRY(get(p + "mlp.down_proj.weight", a));
         ST_TRY(put(a, m->I, 1.f, &c_act, &ly.w_down, &ly.d_down));
         ST_TRY(get(p + "ple_block.per_layer_input_gate.weight", a));

@@ -847,12 +847,11 @@ static svl_status create_vision(svl_ctx *ctx, const svl_vision_config *cfg, int6
         ST_TRY(decode_named(by_name, p + "pre_feedforward_layernorm.weight", nw));
         const ChannelScales c_ff(norm_bounds(nw));
         ST_TRY(put_norm(nw, c_ff, &ly.ln_pre_ff));
-        std::vector<double> act;
+        ChannelScales c_act;
         if (v->split)
-            ST_TRY(load.geglu(gu, v->I, v->H, nw, c_ff, &ly.w_gu, &ly.d_gu, act));
+            ST_TRY(load.geglu(gu, v->I, v->H, nw, c_ff, &ly.w_gu, &ly.d_gu, c_act));
         else
             ST_TRY(upload_owned(v->allocations, gu.data(), gu.size(), &ly.w_gu));
-        const ChannelScales c_act(act);
         ST_TRY(decode_named(by_name, p + "mlp.down_proj.linear.weight", a));
         ST_TRY(put(a, v->I, 1.f, &c_act, &ly.w_down, &ly.d_down));
         ST_TRY(up(p + "post_attention_layernorm.weight", &ly.ln_post_attn));
